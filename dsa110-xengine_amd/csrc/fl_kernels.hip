@@ -32,7 +32,6 @@
 #include "bf_common.h"
 
 namespace {
-constexpr int FL_SLAB = 256;   // channels per stats workgroup
 constexpr int FL_SW = 16;      // waves per stats workgroup
 constexpr int FL_NSEG = 32;    // the reference's threads per (beam, channel)
 constexpr int FL_TBIN = 128;   // ppspec bin
@@ -68,126 +67,199 @@ struct FlStats {
   float *spec, *var, *mx, *pp;
   int nb, nt, nc;
 };
-}  // namespace
 
-template <bool SCALE>
-__global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
-  __shared__ uint32_t lc[FL_NSEG][FL_SLAB];            // per segment: largest bin sum
-  __shared__ uint32_t ls[FL_SW][FL_SLAB], lq[FL_SW][FL_SLAB], lm[FL_SW][FL_SLAB];
-  // scaley as a table: the scaled byte of every input byte x for each channel
-  // of the slab, [x][channel] so that a wave's 64 lanes (consecutive channel
-  // quads) read 64 distinct banks whatever their bytes
-  __shared__ uint8_t lut[SCALE ? 256 * FL_SLAB : 4];
-  const int nslab = (a.nc + FL_SLAB - 1) / FL_SLAB;
-  const int bm = blockIdx.x / nslab, slab = blockIdx.x % nslab;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c0 = slab * FL_SLAB + lane * 4;
-  const bool live = c0 < a.nc;
-  const int per = a.nt / FL_NSEG;
-  const size_t nc = (size_t)a.nc;
-  if (SCALE) {
-    const int c = threadIdx.x & (FL_SLAB - 1), x0 = (threadIdx.x / FL_SLAB) * (256 / 4);
-    const int ch = slab * FL_SLAB + c;
-    if (ch < a.nc) {
-      const float s0 = a.spec0[(size_t)bm * nc + ch];
-      const double k = __ddiv_rn(FL_SIG, (double)__fsqrt_rn(a.var0[(size_t)bm * nc + ch]));
-      for (int x = x0; x < x0 + 256 / 4; x++) lut[x * FL_SLAB + c] = (uint8_t)fl_scale((uint32_t)x, s0, k);
-    }
-    __syncthreads();
-  }
-  uint32_t S[4] = {0, 0, 0, 0}, Q[4] = {0, 0, 0, 0}, M[4] = {0, 0, 0, 0};
-  // each wave walks its two segments' rows with PF loads in flight: row
-  // i + PF is loaded as row i is used (the last PF loads re-read the
-  // segment's last row).  Buffer loads over the beam's plane: 32-bit offsets,
-  // and non-live lanes read zeros past its end.
-  constexpr int PF = 16;
-  static_assert(FL_TBIN % PF == 0, "bins end on a prefetch block");
-  const size_t plane = (size_t)a.nt * nc;
-  // (the beam's base address through readfirstlane: the scaley path also uses
-  // bm in per-lane addresses, and a resource built from vector registers puts
-  // a waterfall loop around every load)
-  const uint64_t base = (uint64_t)(a.data + (size_t)bm * plane);
+// A beam's plane as a buffer resource.  The base goes through readfirstlane:
+// a resource built from vector registers puts a waterfall loop around every
+// load.
+__device__ inline __amdgpu_buffer_rsrc_t fl_plane(const uint8_t *data, int bm, size_t plane) {
+  const uint64_t base = (uint64_t)(data + (size_t)bm * plane);
   const uint64_t sbase = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base) |
                          (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32)) << 32;
-  const __amdgpu_buffer_rsrc_t rin = buffer_rsrc((const void *)sbase, (uint32_t)plane);
-  // the scaled block through a buffer store over the same plane of wdata:
-  // non-live lanes' stores (offset past the plane) are dropped, so the rows
-  // need no branch
-  __amdgpu_buffer_rsrc_t rout = rin;
-  if (SCALE) {
-    const uint64_t wbase = (uint64_t)(a.wdata + (size_t)bm * plane);
-    const uint64_t swbase = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)wbase) |
-                            (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(wbase >> 32)) << 32;
-    rout = buffer_rsrc((const void *)swbase, (uint32_t)plane);
+  return buffer_rsrc((const void *)sbase, (uint32_t)plane);
+}
+
+// Work item of this workgroup: consecutive items (the slabs of one beam, which
+// share its 128-byte lines below 128 channels) run on one XCD.
+__device__ inline int fl_item() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
+
+// scaley as a table: lut[x][channel], the scaled byte of every input byte x for
+// each of the slab's W channels, so that the lanes of a row (consecutive channel
+// quads) read distinct banks whatever their bytes.  s0 and k (LDS, W each) are
+// filled first; channels past the band get any finite values.
+template <int W>
+__device__ inline void fl_lut_build(uint8_t *lut, float *s0, double *k, const float *spec0, const float *var0, int slab,
+                                    int nc) {
+  const int tid = threadIdx.x;
+  if (tid < W) {
+    const int ch = slab * W + tid;
+    s0[tid] = ch < nc ? spec0[ch] : 0.f;
+    k[tid] = ch < nc ? __ddiv_rn(FL_SIG, (double)__fsqrt_rn(var0[ch])) : 0.;
   }
-  const uint32_t cl = live ? (uint32_t)c0 : 0x80000000u;
+  __syncthreads();
+  constexpr int QPR = W / 4;
+  const int q = tid % QPR;
+  const float4 s = *(const float4 *)(s0 + 4 * q);
+  const double k0 = k[4 * q], k1 = k[4 * q + 1], k2 = k[4 * q + 2], k3 = k[4 * q + 3];
+  for (int x = tid / QPR; x < 256; x += 1024 / QPR)
+    *(uint32_t *)(lut + x * W + 4 * q) = fl_scale((uint32_t)x, s.x, k0) | fl_scale((uint32_t)x, s.y, k1) << 8 |
+                                         fl_scale((uint32_t)x, s.z, k2) << 16 | fl_scale((uint32_t)x, s.w, k3) << 24;
+  __syncthreads();
+}
+
+// The four bytes of x (channels c .. c + 3 of the slab) through the table.
+template <int W>
+__device__ inline uint32_t fl_lut4(const uint8_t *lut, uint32_t x, uint32_t c) {
+  uint32_t a[4];
+  if constexpr (W == 256) {
+    // byte j of x over c's low byte, in one permute
+    a[0] = __builtin_amdgcn_perm(x, c, 0x0C0C0400u);
+    a[1] = __builtin_amdgcn_perm(x, c, 0x0C0C0500u);
+    a[2] = __builtin_amdgcn_perm(x, c, 0x0C0C0600u);
+    a[3] = __builtin_amdgcn_perm(x, c, 0x0C0C0700u);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; j++) a[j] = ((x >> (8 * j)) & 0xFFu) * W + c;
+  }
+  return (uint32_t)lut[a[0]] | (uint32_t)lut[a[1] + 1] << 8 | (uint32_t)lut[a[2] + 2] << 16 | (uint32_t)lut[a[3] + 3] << 24;
+}
+}  // namespace
+
+// Every statistic of a (beam, W-channel slab) in one pass, optionally through
+// scaley's table (SCALE) and writing the scaled block (WRITE).  Bound by the
+// stream over the block where the grid fills the chip: 64 x 16384 x 1024 takes
+// 0.197 ms (5.4 TB/s), 0.475 ms with scaley (4.5 TB/s read and written, a plain
+// copy 5.1).  12 x 8192 x 400 takes 16 and 31 us (51 and 102 us on 24 workgroups
+// of 256 channels).
+//
+// 16 waves; W/4 lanes read one row of the slab (a dword each), so a wave's load
+// covers RPI = 256/W consecutive rows.  W is 256 where that gives the chip
+// enough workgroups, else narrower (flk_stats says where).  Wave w walks
+// segments w and w + 16 with PF loads in flight.  Rows are taken four at a time
+// and their 4x4 bytes transposed, so that a channel's four samples are one
+// dword: its sum is one sad and its sum of squares one dot product, 16 + 8
+// instructions for 16 samples where byte-wise sums took 64.
+template <int W, bool SCALE, bool WRITE, bool WMAX>
+__global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
+  constexpr int LPR = W / 4, RPI = 64 / LPR, TB = FL_TBIN / RPI, PF = 16;
+  static_assert(TB % PF == 0, "bins end on a prefetch block");
+  // the table, and after the pass the waves' sums, in the same LDS
+  constexpr int RED = (FL_NSEG + 3 * FL_SW) * W * 4, LUT = SCALE ? 256 * W : 4;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[RED > LUT ? RED : LUT];
+  __shared__ __attribute__((aligned(16))) float ls0[SCALE ? W : 4];
+  __shared__ double lk[SCALE ? W : 1];
+  uint8_t *lut = lds;
+  const int nslab = (a.nc + W - 1) / W;
+  const int item = fl_item();
+  if (item >= a.nb * nslab) return;            // the whole workgroup
+  const int bm = item / nslab, slab = item % nslab;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int cl = (lane & (LPR - 1)) * 4, rg = lane / LPR;
+  const int c0 = slab * W + cl;
+  const bool live = c0 < a.nc;
+  const int per = a.nt / FL_NSEG, n1 = per / RPI, n2 = 2 * n1;   // loads per segment, per wave
+  const size_t plane = (size_t)a.nt * a.nc;
+  const __amdgpu_buffer_rsrc_t rin = fl_plane(a.data, bm, plane);
+  // (non-live lanes read zeros past the plane's end, and their stores there are
+  // dropped: the rows need no branch)
+  const __amdgpu_buffer_rsrc_t rout = WRITE ? fl_plane(a.wdata, bm, plane) : rin;
+  const uint32_t vo = live ? (uint32_t)rg * (uint32_t)a.nc + (uint32_t)c0 : 0x80000000u;
+  // byte offset of the rows of load i (the last ones are re-read past the end)
+  auto row = [&](int i) {
+    i = min(i, n2 - 1);
+    const int seg = i < n1 ? w : w + FL_SW, r = seg * per + (i < n1 ? i : i - n1) * RPI;
+    return (uint32_t)r * (uint32_t)a.nc;
+  };
+  uint32_t buf[PF];
+#pragma unroll
+  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(d), 0);
+  if (SCALE) fl_lut_build<W>(lut, ls0, lk, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, slab, a.nc);
+  uint32_t S[4] = {0, 0, 0, 0}, Q[4] = {0, 0, 0, 0}, bs[4] = {0, 0, 0, 0};
+  uint32_t cm[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, Me = 0, Mo = 0;
+#pragma unroll
   for (int h = 0; h < 2; h++) {
-    const int seg = w + FL_SW * h;
-    const uint32_t s0off = (uint32_t)(seg * per) * (uint32_t)a.nc;
-    uint32_t cm[4] = {0, 0, 0, 0}, bs[4] = {0, 0, 0, 0};
-    uint32_t buf[PF];
+    for (int i0 = h * n1; i0 < (h + 1) * n1; i0 += PF) {
 #pragma unroll
-    for (int d = 0; d < PF; d++)
-      buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, cl + s0off + (uint32_t)d * (uint32_t)a.nc, 0, 0);
-    for (int i0 = 0; i0 < per; i0 += PF) {
+      for (int d = 0; d < PF; d += 4) {
+        uint32_t x[4];
 #pragma unroll
-      for (int d = 0; d < PF; d++) {
-        uint32_t x = buf[d];
-        if (SCALE) {
-          // (every lane: lane * 4 + 3 < FL_SLAB keeps a non-live lane's
-          // lookups in the table, and its statistics are never written)
-          const uint8_t *t = lut + lane * 4;
-          x = (uint32_t)t[(x & 0xFF) * FL_SLAB] | (uint32_t)t[((x >> 8) & 0xFF) * FL_SLAB + 1] << 8 |
-              (uint32_t)t[((x >> 16) & 0xFF) * FL_SLAB + 2] << 16 | (uint32_t)t[(x >> 24) * FL_SLAB + 3] << 24;
-          __builtin_amdgcn_raw_buffer_store_b32(x, rout, cl + s0off + (uint32_t)(i0 + d) * (uint32_t)a.nc, 0, 0);
+        for (int r = 0; r < 4; r++) {
+          x[r] = buf[d + r];
+          // (every lane: cl + 3 < W keeps a non-live lane's lookups in the
+          // table, and its statistics are never written)
+          if (SCALE) x[r] = fl_lut4<W>(lut, x[r], (uint32_t)cl);
+          if (WRITE) __builtin_amdgcn_raw_buffer_store_b32(x[r], rout, vo, row(i0 + d + r), 0);
+          if (WMAX) {
+            typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+            const uint32_t e = x[r] & 0x00FF00FFu, o = (x[r] >> 8) & 0x00FF00FFu;
+            Me = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2, Me), __builtin_bit_cast(us2, e)));
+            Mo = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2, Mo), __builtin_bit_cast(us2, o)));
+          }
         }
+        const uint32_t l01 = __builtin_amdgcn_perm(x[1], x[0], 0x05010400u), h01 = __builtin_amdgcn_perm(x[1], x[0], 0x07030602u);
+        const uint32_t l23 = __builtin_amdgcn_perm(x[3], x[2], 0x05010400u), h23 = __builtin_amdgcn_perm(x[3], x[2], 0x07030602u);
+        const uint32_t t[4] = {__builtin_amdgcn_perm(l23, l01, 0x05040100u), __builtin_amdgcn_perm(l23, l01, 0x07060302u),
+                               __builtin_amdgcn_perm(h23, h01, 0x05040100u), __builtin_amdgcn_perm(h23, h01, 0x07060302u)};
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          const uint32_t v = (x >> (8 * j)) & 0xFF;
-          bs[j] += v;
-          Q[j] += v * v;
-          M[j] = max(M[j], v);
+          bs[j] = __builtin_amdgcn_sad_u8(t[j], 0u, bs[j]);
+          Q[j] = __builtin_amdgcn_udot4(t[j], t[j], Q[j], false);
         }
-        // the next load into buf[d] once x is dead, so that it can take x's
-        // register: a load issued while x is live needs another one, and the
-        // loop then rotates registers whose loads are still in flight
-        const uint32_t nx = (uint32_t)min(i0 + PF + d, per - 1);
-        buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, cl + s0off + nx * (uint32_t)a.nc, 0, 0);
+        // the next loads into these registers once their values are dead: a
+        // load issued earlier needs other registers, and the loop then rotates
+        // registers whose loads are still in flight
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          buf[d + r] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(i0 + PF + d + r), 0);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (((i0 + PF) & (FL_TBIN - 1)) == 0) {          // end of a 128-sample bin
+      if (((i0 - h * n1 + PF) & (TB - 1)) == 0) {          // end of a 128-sample bin
 #pragma unroll
         for (int j = 0; j < 4; j++) {
+#pragma unroll
+          for (int o = LPR; o < 64; o <<= 1) bs[j] += __shfl_xor(bs[j], o, 64);
           S[j] += bs[j];
-          cm[j] = max(cm[j], bs[j]);
+          cm[h][j] = max(cm[h][j], bs[j]);
           bs[j] = 0;
         }
       }
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) lc[seg][lane * 4 + j] = cm[j];
   }
+  uint32_t M[4] = {Me & 0xFFFFu, Mo & 0xFFFFu, Me >> 16, Mo >> 16};
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    ls[w][lane * 4 + j] = S[j];
-    lq[w][lane * 4 + j] = Q[j];
-    lm[w][lane * 4 + j] = M[j];
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (int o = LPR; o < 64; o <<= 1) {
+      Q[j] += __shfl_xor(Q[j], o, 64);
+      if (WMAX) M[j] = max(M[j], (uint32_t)__shfl_xor(M[j], o, 64));
+    }
+  uint32_t *lc = (uint32_t *)lds;                                          // [segment][W]: largest bin sum
+  uint32_t *ls = lc + FL_NSEG * W, *lq = ls + FL_SW * W, *lm = lq + FL_SW * W;   // [wave][W]
+  if (SCALE) __syncthreads();                                              // every wave is done with the table
+  if (rg == 0) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      lc[w * W + cl + j] = cm[0][j];
+      lc[(w + FL_SW) * W + cl + j] = cm[1][j];
+      ls[w * W + cl + j] = S[j];
+      lq[w * W + cl + j] = Q[j];
+      if (WMAX) lm[w * W + cl + j] = M[j];
+    }
   }
   __syncthreads();
-  const int c = threadIdx.x, ch = slab * FL_SLAB + c;
-  if (c >= FL_SLAB || ch >= a.nc) return;
+  const int c = threadIdx.x, ch = slab * W + c;
+  if (c >= W || ch >= a.nc) return;
   uint64_t St = 0, Qt = 0;
   uint32_t Mt = 0, cmax = 0, cmin = 0xFFFFFFFFu;
   for (int v = 0; v < FL_SW; v++) {
-    St += ls[v][c];
-    Qt += lq[v][c];
-    Mt = max(Mt, lm[v][c]);
+    St += ls[v * W + c];
+    Qt += lq[v * W + c];
+    if (WMAX) Mt = max(Mt, lm[v * W + c]);
   }
   for (int s = 0; s < FL_NSEG; s++) {
-    cmax = max(cmax, lc[s][c]);
-    if (s >= FL_NSEG / 2) cmin = min(cmin, lc[s][c]);
+    cmax = max(cmax, lc[s * W + c]);
+    if (s >= FL_NSEG / 2) cmin = min(cmin, lc[s * W + c]);
   }
-  const size_t i = (size_t)bm * nc + ch;
+  const size_t i = (size_t)bm * a.nc + ch;
   const double n = (double)a.nt;
   const float sp = (float)__ddiv_rn((double)St, n);
   if (a.spec) a.spec[i] = sp;
@@ -200,7 +272,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
     const double num = __dadd_rn((double)q, __dmul_rn(dl, dl));
     a.var[i] = (float)__ddiv_rn(__ddiv_rn(num, n), n);
   }
-  if (a.mx) a.mx[i] = (float)Mt;
+  if (WMAX) a.mx[i] = (float)Mt;
   if (a.pp) a.pp[i] = (float)cmax / (float)FL_TBIN - (float)cmin / (float)FL_TBIN;
 }
 
@@ -381,6 +453,29 @@ static bool fl_shape_ok(int nb, int nt, int nc, const char *who) {
   return true;
 }
 
+// Channels per slab of the block-wide passes: the widest that still gives more
+// than half the CUs a workgroup.  Wide slabs read whole cache lines (64 x 16384
+// x 1024 scaley: 256, 128, 64 and 32 channels take 475, 498, 540 and 693 us),
+// but few workgroups cannot draw the bandwidth (12 x 8192 x 400: 105, 62, 37
+// and 31 us; 8 x 8192 x 1024: 118, 80, 64 and 54; 30 x 16384 x 640: 249, 160,
+// 214 and 271).
+static int fl_slab_width(int nb, int nc) {
+  int w = 256;
+  while (w > 32 && (long)nb * ((nc + w - 1) / w) < 144) w >>= 1;
+  return w;
+}
+
+template <int W>
+static void fl_stats_launch(const FlStats &a, dim3 grid, dim3 block, hipStream_t s) {
+  if (a.wdata) {
+    if (a.mx) hipLaunchKernelGGL((fl_stats_kernel<W, true, true, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((fl_stats_kernel<W, true, true, false>), grid, block, 0, s, a);
+  } else {
+    if (a.mx) hipLaunchKernelGGL((fl_stats_kernel<W, false, false, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((fl_stats_kernel<W, false, false, false>), grid, block, 0, s, a);
+  }
+}
+
 extern "C" int flk_stats(const uint8_t *d_data, uint8_t *d_scaled, const float *d_spec0, const float *d_var0,
                          const float *d_spec_in, float *d_spec, float *d_var, float *d_max, float *d_pp,
                          int nb, int nt, int nc, void *stream) {
@@ -390,11 +485,14 @@ extern "C" int flk_stats(const uint8_t *d_data, uint8_t *d_scaled, const float *
     return -1;
   }
   FlStats a{d_data, d_scaled, d_spec0, d_var0, d_spec_in, d_spec, d_var, d_max, d_pp, nb, nt, nc};
-  const dim3 grid(nb * ((nc + FL_SLAB - 1) / FL_SLAB)), block(64 * FL_SW);
-  if (d_scaled)
-    hipLaunchKernelGGL(fl_stats_kernel<true>, grid, block, 0, (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(fl_stats_kernel<false>, grid, block, 0, (hipStream_t)stream, a);
+  const int w = fl_slab_width(nb, nc);
+  const int items = nb * ((nc + w - 1) / w);
+  const dim3 grid((items + 7) / 8 * 8), block(64 * FL_SW);
+  hipStream_t s = (hipStream_t)stream;
+  if (w == 256) fl_stats_launch<256>(a, grid, block, s);
+  else if (w == 128) fl_stats_launch<128>(a, grid, block, s);
+  else if (w == 64) fl_stats_launch<64>(a, grid, block, s);
+  else fl_stats_launch<32>(a, grid, block, s);
   return bfk_check(hipGetLastError(), "fl_stats_kernel");
 }
 

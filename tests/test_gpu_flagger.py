@@ -284,3 +284,38 @@ def test_full_reference_block_subset(orc):
     assert np.array_equal(scaled0, orc.fl_scaley(full[:1], g["spec"][:1], np.maximum(g["var"], 1.0)[:1]))
     for b in list(outs.values()) + [d, d_s0, d_v0, d_ts]:
         b.free()
+
+
+@pytest.mark.parametrize("nb,nc", [(36, 1008), (18, 1008), (9, 1008), (2, 304)])
+def test_every_slab_width_matches_oracle(orc, nb, nc):
+    """Beam and channel counts on each side of the slab widths' limits (256,
+    128, 64 and 32 channels a workgroup, the last slab part-filled): every
+    statistic of the block as it is and scaled, and the scaled bytes.  Whole
+    numbers: equal."""
+    nt = 4096
+    print(f"flagger slab widths {nb}x{nt}x{nc}", flush=True)
+    rng = np.random.default_rng(nb)
+    x = rng.integers(0, 256, (nb, nt, nc), dtype=np.uint8)
+    spec0 = rng.uniform(60, 190, (nb, nc)).astype(np.float32)
+    var0 = rng.uniform(500, 9000, (nb, nc)).astype(np.float32)
+    d = _dev(x)
+    outs = {k: DeviceBuffer(nb * nc * 4) for k in ("spec", "var", "max", "pp")}
+
+    def check(got, data, beams):
+        for b in beams:
+            y = np.ascontiguousarray(data[b:b + 1])
+            spec = orc.fl_stat("spectrum", y)
+            want = {"spec": spec, "var": orc.fl_stat("varspec_exact", y, spec), "max": orc.fl_stat("maxspec", y),
+                    "pp": orc.fl_stat("ppspec", y)}
+            for k, v in want.items():
+                assert np.array_equal(got[k][b:b + 1], v), (k, b)
+
+    beams = sorted({0, 1, nb // 2, nb - 1})
+    fl.stats(d, nb, nt, nc, d_spec=outs["spec"], d_var=outs["var"], d_max=outs["max"], d_pp=outs["pp"])
+    check({k: _get(v, (nb, nc), np.float32) for k, v in outs.items()}, x, beams)
+    fl.scaley(d, nb, nt, nc, _dev(spec0), _dev(var0), d_spec=outs["spec"], d_var=outs["var"], d_max=outs["max"],
+              d_pp=outs["pp"])
+    y = _get(d, x.shape, np.uint8)
+    for b in beams:
+        assert np.array_equal(y[b:b + 1], orc.fl_scaley(x[b:b + 1], spec0[b:b + 1], var0[b:b + 1])), b
+    check({k: _get(v, (nb, nc), np.float32) for k, v in outs.items()}, y, beams)
