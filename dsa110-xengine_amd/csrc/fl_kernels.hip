@@ -84,25 +84,42 @@ __device__ inline int fl_item() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (
 
 // scaley as a table: lut[x][channel], the scaled byte of every input byte x for
 // each of the slab's W channels, so that the lanes of a row (consecutive channel
-// quads) read distinct banks whatever their bytes.  s0 and k (LDS, W each) are
-// filled first; channels past the band get any finite values.
+// quads) read distinct banks whatever their bytes.  A channel with a nonzero
+// mask byte holds the beam's replacement byte for every x instead, which makes
+// flagging part of the lookup; channels past the band hold zeros.
+template <int W> struct FlLutScratch {
+  double k[W];
+  float s0[W];
+  int fix[W];                    // -1, or the byte of every x
+};
 template <int W>
-__device__ inline void fl_lut_build(uint8_t *lut, float *s0, double *k, const float *spec0, const float *var0, int slab,
-                                    int nc) {
+__device__ inline void fl_lut_build(uint8_t *lut, FlLutScratch<W> &t, const float *spec0, const float *var0,
+                                    const uint8_t *mask, uint32_t rep, int slab, int nc) {
   const int tid = threadIdx.x;
   if (tid < W) {
     const int ch = slab * W + tid;
-    s0[tid] = ch < nc ? spec0[ch] : 0.f;
-    k[tid] = ch < nc ? __ddiv_rn(FL_SIG, (double)__fsqrt_rn(var0[ch])) : 0.;
+    t.s0[tid] = ch < nc ? spec0[ch] : 0.f;
+    t.k[tid] = ch < nc ? __ddiv_rn(FL_SIG, (double)__fsqrt_rn(var0[ch])) : 0.;
+    t.fix[tid] = ch >= nc ? 0 : mask && mask[ch] ? (int)rep : -1;
   }
   __syncthreads();
   constexpr int QPR = W / 4;
   const int q = tid % QPR;
-  const float4 s = *(const float4 *)(s0 + 4 * q);
-  const double k0 = k[4 * q], k1 = k[4 * q + 1], k2 = k[4 * q + 2], k3 = k[4 * q + 3];
-  for (int x = tid / QPR; x < 256; x += 1024 / QPR)
-    *(uint32_t *)(lut + x * W + 4 * q) = fl_scale((uint32_t)x, s.x, k0) | fl_scale((uint32_t)x, s.y, k1) << 8 |
-                                         fl_scale((uint32_t)x, s.z, k2) << 16 | fl_scale((uint32_t)x, s.w, k3) << 24;
+  float s[4];
+  double k[4];
+  int fix[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    s[j] = t.s0[4 * q + j];
+    k[j] = t.k[4 * q + j];
+    fix[j] = t.fix[4 * q + j];
+  }
+  for (int x = tid / QPR; x < 256; x += 1024 / QPR) {
+    uint32_t o = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) o |= (fix[j] < 0 ? fl_scale((uint32_t)x, s[j], k[j]) : (uint32_t)fix[j]) << (8 * j);
+    *(uint32_t *)(lut + x * W + 4 * q) = o;
+  }
   __syncthreads();
 }
 
@@ -145,8 +162,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
   // the table, and after the pass the waves' sums, in the same LDS
   constexpr int RED = (FL_NSEG + 3 * FL_SW) * W * 4, LUT = SCALE ? 256 * W : 4;
   __shared__ __attribute__((aligned(16))) uint8_t lds[RED > LUT ? RED : LUT];
-  __shared__ __attribute__((aligned(16))) float ls0[SCALE ? W : 4];
-  __shared__ double lk[SCALE ? W : 1];
+  __shared__ FlLutScratch<SCALE ? W : 1> lt;
   uint8_t *lut = lds;
   const int nslab = (a.nc + W - 1) / W;
   const int item = fl_item();
@@ -172,7 +188,8 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
   uint32_t buf[PF];
 #pragma unroll
   for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(d), 0);
-  if (SCALE) fl_lut_build<W>(lut, ls0, lk, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, slab, a.nc);
+  if constexpr (SCALE)
+    fl_lut_build<W>(lut, lt, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, nullptr, 0, slab, a.nc);
   uint32_t S[4] = {0, 0, 0, 0}, Q[4] = {0, 0, 0, 0}, bs[4] = {0, 0, 0, 0};
   uint32_t cm[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, Me = 0, Mo = 0;
 #pragma unroll
@@ -276,6 +293,377 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
   if (a.pp) a.pp[i] = (float)cmax / (float)FL_TBIN - (float)cmin / (float)FL_TBIN;
 }
 
+// ---- the block step's second pass ---------------------------------------------
+namespace {
+// Value of the lane whose number differs in bit O.
+template <int O> __device__ inline uint32_t fl_xor_lane(uint32_t v) {
+  if constexpr (O == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);        // quad_perm 1,0,3,2
+  else if constexpr (O == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2,3,0,1
+  else if constexpr (O == 4) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x101F);
+  else return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, true);                        // O == 8: row_ror 8
+}
+// a summed over the lane pairs of bit O in the lanes with the bit clear, b in
+// those with it set.
+template <int O> __device__ inline uint32_t fl_fold(uint32_t a, uint32_t b, int lane) {
+  if constexpr (O == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    return r[0] + r[1];
+  } else if constexpr (O == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    return r[0] + r[1];
+  } else {
+    const bool up = lane & O;
+    return (up ? b : a) + fl_xor_lane<O>(up ? a : b);
+  }
+}
+// Sums of 16 rows over the LPR lanes of a row: rs[i] is this lane's share of
+// row i (any 8 lanes' shares below 2^16), the result two rows' sums packed,
+// rows 2k and 2k + 1 for k = (lane % LPR) / (LPR / 8).  Each fold halves both
+// the rows a lane carries and the lanes that share them: 26 instructions for 16
+// rows of 64 lanes, where a cross-lane sum per row takes 96.
+template <int LPR> __device__ inline uint32_t fl_row_sums(const uint32_t (&rs)[16], int lane) {
+  uint32_t p[8], q[4], r[2], v;
+#pragma unroll
+  for (int k = 0; k < 8; k++) p[k] = rs[2 * k] | rs[2 * k + 1] << 16;
+#pragma unroll
+  for (int k = 0; k < 4; k++) q[k] = fl_fold<LPR / 2>(p[k], p[k + 4], lane);
+#pragma unroll
+  for (int k = 0; k < 2; k++) r[k] = fl_fold<LPR / 4>(q[k], q[k + 2], lane);
+  v = fl_fold<LPR / 8>(r[0], r[1], lane);
+  if constexpr (LPR == 64) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);   // row_half_mirror
+  if constexpr (LPR >= 32) v += fl_xor_lane<2>(v);
+  if constexpr (LPR >= 16) v += fl_xor_lane<1>(v);
+  return v;
+}
+
+struct FlApply {
+  uint8_t *data;
+  const float *spec0, *var0;
+  const uint8_t *mask;
+  const float *bpwr;
+  uint16_t *part;              // [beam][slab][time] row sums of the slab, or NULL
+  const double *bsum;          // per-beam sums of the spectrum
+  int *ran, *h_ran;            // set to 1 by a pass that ran, else 0 (device and host)
+  float prev;                  // total power of the last block, and the jump that
+  float jump;                  // has the block replaced instead
+  int force;
+  int nb, nt, nc;
+};
+}  // namespace
+
+// scaley, flag and the row sums of make_ts in one pass in place, after the
+// masks: the statistics come from a pass that only read the raw block, so the
+// scaled block is written once and never read back.  64 x 16384 x 1024: the
+// read-only pass and this one move 3 GiB where scaley + flag moved 4.
+// Bound by the stream over the block (read and written).
+//
+// A workgroup takes a (beam, W-channel slab), its 16 waves a sixteenth of the
+// times each; rows and prefetch as in fl_stats_kernel.  The masked channels are
+// part of the table.  The slab's row sums (at most 256 * 255) go out as 16 bits.
+// The pass leaves the block alone when the total power has jumped: the block is
+// then replaced by noise, and the host, which sums the spectrum in the
+// reference's order meanwhile, has the last word (force, or the noise).
+template <int W>
+__global__ __launch_bounds__(1024) void fl_apply_kernel(FlApply a) {
+  constexpr int LPR = W / 4, RPI = 64 / LPR, PF = 16;
+  __shared__ __attribute__((aligned(16))) uint8_t lut[256 * W];
+  __shared__ FlLutScratch<W> lt;
+  const int nslab = (a.nc + W - 1) / W;
+  const int item = fl_item();
+  const int lane = threadIdx.x & 63;
+  bool go = true;
+  if (!a.force) {
+    double e = 0.;
+    for (int b = lane; b < a.nb; b += 64) e += a.bsum[b];
+    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+    go = !(fabs(e - (double)a.prev) / (double)a.prev >= (double)a.jump);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.ran = *a.h_ran = go;
+  if (!go || item >= a.nb * nslab) return;       // the whole workgroup
+  const int bm = item / nslab, slab = item % nslab;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int cl = (lane & (LPR - 1)) * 4, rg = lane / LPR;
+  const int c0 = slab * W + cl;
+  const int n = a.nt / 16 / RPI;                 // loads of this wave
+  const uint32_t r0 = (uint32_t)w * (uint32_t)(a.nt / 16);
+  const size_t plane = (size_t)a.nt * a.nc;
+  const __amdgpu_buffer_rsrc_t rsrc = fl_plane(a.data, bm, plane);
+  // (lanes past the band: zeros in, zeros from the table, stores dropped)
+  const uint32_t vo = c0 < a.nc ? (uint32_t)rg * (uint32_t)a.nc + (uint32_t)c0 : 0x80000000u;
+  auto row = [&](int i) { return (r0 + (uint32_t)(min(i, n - 1) * RPI)) * (uint32_t)a.nc; };
+  uint32_t buf[PF];
+#pragma unroll
+  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(d), 0);
+  fl_lut_build<W>(lut, lt, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, a.mask + (size_t)bm * a.nc,
+                  fl_rep(a.bpwr[bm]), slab, a.nc);
+  uint16_t *part = a.part ? a.part + (size_t)item * a.nt : nullptr;
+  for (int i0 = 0; i0 < n; i0 += PF) {
+    uint32_t rs[PF];
+#pragma unroll
+    for (int d = 0; d < PF; d++) {
+      const uint32_t x = fl_lut4<W>(lut, buf[d], (uint32_t)cl);
+      __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, vo, row(i0 + d), 0);
+      rs[d] = __builtin_amdgcn_sad_u8(x, 0u, 0u);
+      // (past the end this wave's last row again, into registers that are not used)
+      buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(i0 + PF + d), 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (part) {
+      const uint32_t v = fl_row_sums<LPR>(rs, lane);
+      const int l = lane & (LPR - 1), k = l / (LPR / 8);
+      if (l % (LPR / 8) == 0) {
+        const uint32_t t = r0 + (uint32_t)((i0 + 2 * k) * RPI + rg);
+        if constexpr (RPI == 1) {
+          *(uint32_t *)(part + t) = v;           // t is even
+        } else {
+          part[t] = (uint16_t)v;
+          part[t + RPI] = (uint16_t)(v >> 16);
+        }
+      }
+    }
+  }
+}
+
+// ---- the masks ------------------------------------------------------------------
+namespace {
+constexpr int FL_ZERO = 128, FL_FILT = 21, FL_FBIN = 8;   // band edge, median window, simple_channflag bin
+constexpr int FL_LDSN = 4096;                             // values of one selection kept in LDS
+
+// Floats in order as unsigned numbers (finite values).
+__device__ inline uint32_t fl_key(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  return u ^ ((uint32_t)((int)u >> 31) | 0x80000000u);
+}
+__device__ inline float fl_unkey(uint32_t k) {
+  return __builtin_bit_cast(float, k & 0x80000000u ? k ^ 0x80000000u : ~k);
+}
+
+// The k-th smallest (from 0) of the n keys get(i), found two bits a round from
+// the top by a team of four waves: every thread of the workgroup calls it (it
+// has barriers), teams with data of their own, cnt[2][12] theirs.
+template <class G>
+__device__ inline uint32_t fl_kth(G get, int n, int k, int tid, uint32_t (*cnt)[12]) {
+  uint32_t prefix = 0;
+  int buf = 0;
+  for (int b = 30; b >= 0; b -= 2, buf ^= 1) {
+    const uint32_t t1 = prefix | 1u << b, t2 = prefix | 2u << b, t3 = prefix | 3u << b;
+    uint32_t c1 = 0, c2 = 0, c3 = 0;
+    for (int i0 = 0; i0 < n; i0 += 256) {
+      const uint32_t key = i0 + tid < n ? get(i0 + tid) : 0xFFFFFFFFu;   // (no finite value's key)
+      c1 += __popcll(__ballot(key < t1));
+      c2 += __popcll(__ballot(key < t2));
+      c3 += __popcll(__ballot(key < t3));
+    }
+    if ((tid & 63) == 0) {
+      uint32_t *c = &cnt[buf][(tid >> 6) * 3];
+      c[0] = c1;
+      c[1] = c2;
+      c[2] = c3;
+    }
+    // (a wave that writes this buffer again has passed the next barrier, which
+    // the others reach after reading it)
+    __syncthreads();
+    const uint32_t *c = cnt[buf];
+    const uint32_t uk = (uint32_t)k;
+    const uint32_t digit = (uint32_t)(c[0] + c[3] + c[6] + c[9] <= uk) + (uint32_t)(c[1] + c[4] + c[7] + c[10] <= uk) +
+                           (uint32_t)(c[2] + c[5] + c[8] + c[11] <= uk);
+    prefix |= digit << b;
+  }
+  return prefix;
+}
+
+// Median of 21 values: of 12 the smallest and the largest are dropped and the
+// next value joins, until three are left (92 exchanges; no value can be the
+// median once it is the extreme of more than half of them).
+__device__ inline float fl_median21(const float *w) {
+  float a[12];
+#pragma unroll
+  for (int i = 0; i < 12; i++) a[i] = w[i];
+#pragma unroll
+  for (int n = 12; n > 3; n--) {
+    auto order = [&](int i, int j) {
+      const float lo = fminf(a[i], a[j]), hi = fmaxf(a[i], a[j]);
+      a[i] = lo;
+      a[j] = hi;
+    };
+#pragma unroll
+    for (int i = 0; i < n / 2; i++) order(i, n - 1 - i);
+#pragma unroll
+    for (int i = 1; i < (n + 1) / 2; i++) order(0, i);          // the smallest to the front
+#pragma unroll
+    for (int i = n / 2; i < n - 1; i++) order(i, n - 1);        // the largest to the back
+    a[0] = w[24 - n];                                           // n = 12: w[12], ..., n = 4: w[20]
+  }
+  return __builtin_amdgcn_fmed3f(a[0], a[1], a[2]);
+}
+
+struct FlMasks {
+  const float *spec, *var, *pp;
+  float *big;                   // [3][beam][nchan - 256] where that is above FL_LDSN, else NULL
+  uint8_t *mask;                // [beam][channel], 0 or 1
+  int *h_nmask;                 // per beam (host)
+  float *h_spec;                // the spectrum for the host
+  double *bsum;
+  float *bpwr;                  // calc_bpwr's levels, or NULL to leave them
+  float thr[3];                 // channflag of spec and of var, simple_channflag of pp (over sqrt(FBIN))
+  int nb, nc, nperm;
+  int perm[64];
+};
+}  // namespace
+
+// channflag on spec and var, simple_channflag on pp (gpu_flagger.cu:557-660),
+// and the count of the flagged channels: workgroup (beam, 0), a team of four
+// waves per statistic.  Every float and double operation of the reference's CPU
+// code, in its order; medians are selections, so which equal element is taken
+// does not matter.  Workgroup (beam, 1): the spectrum to the host, its sum, and
+// calc_bpwr.  64 beams x 1024 channels: 11 us for what took the host, with the
+// copies both ways, about 0.6 ms.
+__global__ __launch_bounds__(768) void fl_masks_kernel(FlMasks a) {
+  __shared__ float val[3][FL_LDSN];
+  __shared__ uint32_t cnt[3][2][12];
+  __shared__ double red[12];
+  const int bm = blockIdx.x, tid = threadIdx.x;
+  const size_t at = (size_t)bm * a.nc;
+  if (blockIdx.y == 1) {
+    double s = 0.;
+    for (int c = tid; c < a.nc; c += 768) {
+      const float v = a.spec[at + c];
+      a.h_spec[at + c] = v;
+      s += (double)v;
+    }
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((tid & 63) == 0) red[tid >> 6] = s;
+    __syncthreads();
+    if (tid == 0) {
+      for (int k = 1; k < 12; k++) s += red[k];
+      a.bsum[bm] = s;
+    }
+    if (!a.bpwr) return;
+    // calc_bpwr's float sum in channel order, a stretch of the row at a time
+    float f = 0.f;
+    for (int c0 = 0; c0 < a.nc; c0 += FL_LDSN) {
+      const int m = min(FL_LDSN, a.nc - c0);
+      __syncthreads();
+      for (int c = tid; c < m; c += 768) val[0][c] = a.spec[at + c0 + c];
+      __syncthreads();
+      if (tid == 0) {
+#pragma unroll 16
+        for (int c = 0; c < m; c++) f = __fadd_rn(f, val[0][c]);
+      }
+    }
+    if (tid == 0) a.bpwr[bm] = (float)__ddiv_rn(__ddiv_rn((double)f, (double)(a.nc - 2 * FL_ZERO)), FL_MN);
+    return;
+  }
+  const int team = tid >> 8, tt = tid & 255;
+  const int nin = a.nc - 2 * FL_ZERO;
+  uint8_t *mask = a.mask + at;
+  for (int c = tid; c < a.nc; c += 768) mask[c] = 0;
+  const float *row = (team == 0 ? a.spec : team == 1 ? a.var : a.pp) + at + FL_ZERO;
+  float *v = nin <= FL_LDSN ? val[team] : a.big + ((size_t)team * a.nb + bm) * nin;
+  for (int j = tt; j < nin; j += 256) {
+    float x = row[j];
+    if (team < 2) {
+      float w[FL_FILT];
+      const float *src = row + min(j, nin - FL_FILT);
+#pragma unroll
+      for (int i = 0; i < FL_FILT; i++) w[i] = src[i];
+      x = __fsub_rn(x, fl_median21(w));
+    }
+    v[j] = x;
+  }
+  __syncthreads();
+  const int k = (nin + 1) / 2 - 1;
+  const float med = fl_unkey(fl_kth([&](int i) { return fl_key(v[i]); }, nin, k, tt, cnt[team]));
+  const float mad = fl_unkey(fl_kth([&](int i) { return fl_key(fabsf(__fsub_rn(v[i], med))); }, nin, k, tt, cnt[team]));
+  const float lim = __fmul_rn(a.thr[team], mad);
+  // (teams that set the same byte store the same value)
+  if (team < 2) {
+    for (int j = tt; j < nin; j += 256)
+      if (v[j] > lim || v[j] < -lim) mask[FL_ZERO + j] = 1;
+    if (tid < a.nperm && a.perm[tid] >= FL_ZERO && a.perm[tid] < a.nc - FL_ZERO) mask[a.perm[tid]] = 1;
+  } else {
+    for (int j = tt; j < nin - FL_FBIN; j += 256) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < FL_FBIN; i++) s = __fadd_rn(s, v[j]);       // the same element FBIN times
+      if ((float)__dsub_rn((double)s * (1. / FL_FBIN), (double)med) > lim) mask[FL_ZERO + j] = 1;
+    }
+  }
+  __syncthreads();
+  uint32_t m = 0;
+  for (int c = tid; c < a.nc; c += 768) m += mask[c];
+  for (int o = 32; o > 0; o >>= 1) m += __shfl_xor(m, o, 64);
+  if ((tid & 63) == 0) cnt[0][0][tid >> 6] = m;
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 1; i < 12; i++) m += cnt[0][0][i];
+    a.h_nmask[bm] = (int)m;
+  }
+}
+
+namespace {
+struct FlTsMask {
+  const uint16_t *part;         // fl_apply_kernel's row sums, or NULL: ts holds the series
+  float *ts;
+  int *idx, *n_ts, *h_nts;      // per beam: flagged rows (beam * ntime + time), their count (device and host)
+  const int *ran;               // fl_apply_kernel's flag, or NULL
+  float thr;
+  int nb, nt, nc, nslab;
+};
+}  // namespace
+
+// make_ts's division and simple_tsflag (gpu_flagger.cu:413-452,662-700): a
+// workgroup per beam, the series' median and MAD over its first ntime/16
+// samples, and the list of its flagged rows.  (The four teams of four waves
+// each select the same values; the order of the list does not matter.)
+__global__ __launch_bounds__(1024) void fl_tsmask_kernel(FlTsMask a) {
+  __shared__ float val[FL_LDSN];
+  __shared__ uint32_t cnt[4][2][12];
+  __shared__ uint32_t nf;
+  const int bm = blockIdx.x, tid = threadIdx.x, tt = tid & 255, team = tid >> 8;
+  const int nm = a.nt / 16;
+  float *ts = a.ts + (size_t)bm * a.nt;
+  const bool live = !a.ran || *a.ran;
+  if (tid == 0) nf = 0;
+  if (!live) {                                   // the whole grid
+    if (tid == 0) a.n_ts[bm] = a.h_nts[bm] = 0;
+    return;
+  }
+  if (a.part) {
+    const uint16_t *p = a.part + (size_t)bm * a.nslab * a.nt;
+    for (int t = tid * 4; t < a.nt; t += 4096) {
+      uint32_t s[4] = {0, 0, 0, 0};
+      for (int k = 0; k < a.nslab; k++) {
+        const uint2 v = *(const uint2 *)(p + (size_t)k * a.nt + t);
+        s[0] += v.x & 0xFFFFu;
+        s[1] += v.x >> 16;
+        s[2] += v.y & 0xFFFFu;
+        s[3] += v.y >> 16;
+      }
+      float f[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) f[j] = (float)__ddiv_rn((double)s[j], (double)a.nc);
+      *(float4 *)(ts + t) = make_float4(f[0], f[1], f[2], f[3]);
+    }
+    __syncthreads();
+  }
+  const float *v = ts;
+  if (nm <= FL_LDSN) {
+    for (int t = tid; t < nm; t += 1024) val[t] = ts[t];
+    v = val;
+  }
+  __syncthreads();
+  const int k = (nm + 1) / 2 - 1;
+  const float med = fl_unkey(fl_kth([&](int i) { return fl_key(v[i]); }, nm, k, tt, cnt[team]));
+  const float mad = fl_unkey(fl_kth([&](int i) { return fl_key(fabsf(__fsub_rn(v[i], med))); }, nm, k, tt, cnt[team]));
+  const float lim = __fmul_rn(a.thr, mad);
+  int *idx = a.idx + (size_t)bm * a.nt;
+  for (int t = tid; t < a.nt; t += 1024)
+    if (__fsub_rn(ts[t], med) > lim) idx[atomicAdd(&nf, 1u)] = bm * a.nt + t;
+  __syncthreads();
+  if (tid == 0) a.n_ts[bm] = a.h_nts[bm] = (int)nf;
+}
+
 __device__ inline uint32_t fl_wave_sum(uint32_t v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -363,6 +751,19 @@ __global__ __launch_bounds__(256) void fl_flagts_kernel(uint8_t *data, const int
   const uint32_t rep = fl_rep(bpwr[bm]) * 0x01010101u;
   uint8_t *row = data + (size_t)m * nc;
   for (int q = 8 + lane; q < nc / 16 - 8; q += 64) *(uint4 *)(row + 16 * q) = make_uint4(rep, rep, rep, rep);
+}
+
+// flagts on fl_tsmask_kernel's lists: blockIdx.x the beam, the waves of the
+// beam's gridDim.y workgroups a row each in turn.
+__global__ __launch_bounds__(256) void fl_flagts_list_kernel(uint8_t *data, const int *idx, const int *n_ts,
+                                                             const float *bpwr, int nt, int nc) {
+  const int bm = blockIdx.x, lane = threadIdx.x & 63;
+  const int n = n_ts[bm];
+  const uint32_t rep = fl_rep(bpwr[bm]) * 0x01010101u;
+  for (int i = blockIdx.y * 4 + (threadIdx.x >> 6); i < n; i += gridDim.y * 4) {
+    uint8_t *row = data + (size_t)idx[(size_t)bm * nt + i] * nc;
+    for (int q = 8 + lane; q < nc / 16 - 8; q += 64) *(uint4 *)(row + 16 * q) = make_uint4(rep, rep, rep, rep);
+  }
 }
 
 // flag (gpu_flagger.cu:458-474): column midx[i] = bm * nchan + ch, every time.
@@ -467,7 +868,9 @@ static int fl_slab_width(int nb, int nc) {
 
 template <int W>
 static void fl_stats_launch(const FlStats &a, dim3 grid, dim3 block, hipStream_t s) {
-  if (a.wdata) {
+  if (a.spec0 && !a.wdata) {
+    hipLaunchKernelGGL((fl_stats_kernel<W, true, false, false>), grid, block, 0, s, a);
+  } else if (a.wdata) {
     if (a.mx) hipLaunchKernelGGL((fl_stats_kernel<W, true, true, true>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((fl_stats_kernel<W, true, true, false>), grid, block, 0, s, a);
   } else {
@@ -476,17 +879,10 @@ static void fl_stats_launch(const FlStats &a, dim3 grid, dim3 block, hipStream_t
   }
 }
 
-extern "C" int flk_stats(const uint8_t *d_data, uint8_t *d_scaled, const float *d_spec0, const float *d_var0,
-                         const float *d_spec_in, float *d_spec, float *d_var, float *d_max, float *d_pp,
-                         int nb, int nt, int nc, void *stream) {
-  if (!fl_shape_ok(nb, nt, nc, "flk_stats")) return -1;
-  if (d_scaled && (!d_spec0 || !d_var0)) {
-    bfk_set_error("flk_stats: scaling needs spec0 and var0");
-    return -1;
-  }
-  FlStats a{d_data, d_scaled, d_spec0, d_var0, d_spec_in, d_spec, d_var, d_max, d_pp, nb, nt, nc};
-  const int w = fl_slab_width(nb, nc);
-  const int items = nb * ((nc + w - 1) / w);
+static int fl_stats_any(const FlStats &a, const char *who, void *stream) {
+  if (!fl_shape_ok(a.nb, a.nt, a.nc, who)) return -1;
+  const int w = fl_slab_width(a.nb, a.nc);
+  const int items = a.nb * ((a.nc + w - 1) / w);
   const dim3 grid((items + 7) / 8 * 8), block(64 * FL_SW);
   hipStream_t s = (hipStream_t)stream;
   if (w == 256) fl_stats_launch<256>(a, grid, block, s);
@@ -494,6 +890,92 @@ extern "C" int flk_stats(const uint8_t *d_data, uint8_t *d_scaled, const float *
   else if (w == 64) fl_stats_launch<64>(a, grid, block, s);
   else fl_stats_launch<32>(a, grid, block, s);
   return bfk_check(hipGetLastError(), "fl_stats_kernel");
+}
+
+extern "C" int flk_stats(const uint8_t *d_data, uint8_t *d_scaled, const float *d_spec0, const float *d_var0,
+                         const float *d_spec_in, float *d_spec, float *d_var, float *d_max, float *d_pp,
+                         int nb, int nt, int nc, void *stream) {
+  if (d_scaled && (!d_spec0 || !d_var0)) {
+    bfk_set_error("flk_stats: scaling needs spec0 and var0");
+    return -1;
+  }
+  const FlStats a{d_data, d_scaled, d_scaled ? d_spec0 : NULL, d_scaled ? d_var0 : NULL, d_spec_in, d_spec, d_var,
+                  d_max,  d_pp,     nb, nt, nc};
+  return fl_stats_any(a, "flk_stats", stream);
+}
+
+// The statistics that the scaled block will have; the block is only read.
+extern "C" int flk_stats_scaled(const uint8_t *d_data, const float *d_spec0, const float *d_var0, float *d_spec,
+                                float *d_var, float *d_pp, int nb, int nt, int nc, void *stream) {
+  const FlStats a{d_data, NULL, d_spec0, d_var0, NULL, d_spec, d_var, NULL, d_pp, nb, nt, nc};
+  return fl_stats_any(a, "flk_stats_scaled", stream);
+}
+
+extern "C" size_t flk_masks_big_bytes(int nb, int nc) {
+  const int nin = nc - 2 * FL_ZERO;
+  return nin > FL_LDSN ? (size_t)3 * nb * nin * sizeof(float) : 0;
+}
+
+extern "C" int flk_masks(const float *d_spec, const float *d_var, const float *d_pp, float *d_big, uint8_t *d_mask,
+                         int *h_nmask, float *h_spec, double *d_bsum, float *d_bpwr, float thresh, const int *perm,
+                         int nperm, int nb, int nc, void *stream) {
+  if (nb < 1 || nc < 2 * FL_ZERO + FL_FILT || nperm < 0 || nperm > 64 || (flk_masks_big_bytes(nb, nc) && !d_big)) {
+    bfk_set_error("flk_masks: %d beams x %d channels, %d permanent", nb, nc, nperm);
+    return -1;
+  }
+  FlMasks a;
+  a.spec = d_spec;
+  a.var = d_var;
+  a.pp = d_pp;
+  a.big = d_big;
+  a.mask = d_mask;
+  a.h_nmask = h_nmask;
+  a.h_spec = h_spec;
+  a.bsum = d_bsum;
+  a.bpwr = d_bpwr;
+  a.thr[0] = thresh;
+  a.thr[1] = (float)((double)thresh + 0.5);
+  a.thr[2] = (float)(thresh / sqrt(1. * FL_FBIN));
+  a.nb = nb;
+  a.nc = nc;
+  a.nperm = nperm;
+  for (int i = 0; i < 64; i++) a.perm[i] = i < nperm ? perm[i] : 0;
+  hipLaunchKernelGGL(fl_masks_kernel, dim3(nb, 2), dim3(768), 0, (hipStream_t)stream, a);
+  return bfk_check(hipGetLastError(), "fl_masks_kernel");
+}
+
+extern "C" size_t flk_part_bytes(int nb, int nt, int nc) {
+  const int w = fl_slab_width(nb, nc);
+  return (size_t)nb * ((nc + w - 1) / w) * nt * sizeof(uint16_t);
+}
+
+extern "C" int flk_apply(uint8_t *d_data, const float *d_spec0, const float *d_var0, const uint8_t *d_mask,
+                         const float *d_bpwr, uint16_t *d_part, const double *d_bsum, int *d_ran, int *h_ran, float prev,
+                         float jump, int force, int nb, int nt, int nc, void *stream) {
+  if (!fl_shape_ok(nb, nt, nc, "flk_apply")) return -1;
+  const FlApply a{d_data, d_spec0, d_var0, d_mask, d_bpwr, d_part, d_bsum, d_ran, h_ran, prev, jump, force, nb, nt, nc};
+  const int w = fl_slab_width(nb, nc);
+  const int items = nb * ((nc + w - 1) / w);
+  const dim3 grid((items + 7) / 8 * 8), block(1024);
+  hipStream_t s = (hipStream_t)stream;
+  if (w == 256) hipLaunchKernelGGL(fl_apply_kernel<256>, grid, block, 0, s, a);
+  else if (w == 128) hipLaunchKernelGGL(fl_apply_kernel<128>, grid, block, 0, s, a);
+  else if (w == 64) hipLaunchKernelGGL(fl_apply_kernel<64>, grid, block, 0, s, a);
+  else hipLaunchKernelGGL(fl_apply_kernel<32>, grid, block, 0, s, a);
+  return bfk_check(hipGetLastError(), "fl_apply_kernel");
+}
+
+// simple_tsflag of the series (from fl_apply's row sums, or d_ts itself with
+// d_part NULL) and flagts of the rows it finds.
+extern "C" int flk_tsmask_flagts(uint8_t *d_data, const uint16_t *d_part, float *d_ts, int *d_idx, int *d_nts, int *h_nts,
+                                 const int *d_ran, const float *d_bpwr, float thr, int nb, int nt, int nc, void *stream) {
+  if (!fl_shape_ok(nb, nt, nc, "flk_tsmask_flagts")) return -1;
+  const int w = fl_slab_width(nb, nc);
+  const FlTsMask a{d_part, d_ts, d_idx, d_nts, h_nts, d_ran, thr, nb, nt, nc, (nc + w - 1) / w};
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(fl_tsmask_kernel, dim3(nb), dim3(1024), 0, s, a);
+  hipLaunchKernelGGL(fl_flagts_list_kernel, dim3(nb, 16), dim3(256), 0, s, d_data, d_idx, d_nts, d_bpwr, nt, nc);
+  return bfk_check(hipGetLastError(), "fl_tsmask_kernel");
 }
 
 extern "C" int flk_flag_ts(uint8_t *d_data, const uint8_t *d_mask, const float *d_bpwr, float *d_ts, int nb,

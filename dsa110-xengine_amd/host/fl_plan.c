@@ -6,9 +6,11 @@
  * scaley, calc_spectrum, calc_varspec, calc_spectrum (its "maxspec"),
  * calc_ppspec, flag, make_ts and flagts -- five full reads of the 1 GiB block
  * and two writes -- with blocking copies of every statistic between them.
- * The plan runs two passes over the block (scaley fused with every
- * statistic; flag fused with make_ts) plus flagts on the masked rows, and
- * copies only the spectra, the masks and the time series.
+ * The plan runs two passes over the block -- one that only reads it, for the
+ * statistics of the scaled block, and one that scales, flags and sums its rows
+ * in place -- plus flagts on the masked rows.  The masks are made on the device
+ * between them; the host only sums the spectrum (the total power, in the
+ * reference's order) while the second pass runs.
  */
 #include <hip/hip_runtime_api.h>
 #include <math.h>
@@ -22,6 +24,18 @@
 int flk_stats(const uint8_t *d_data, uint8_t *d_scaled, const float *d_spec0, const float *d_var0,
               const float *d_spec_in, float *d_spec, float *d_var, float *d_max, float *d_pp, int nb, int nt,
               int nc, void *stream);
+int flk_stats_scaled(const uint8_t *d_data, const float *d_spec0, const float *d_var0, float *d_spec, float *d_var,
+                     float *d_pp, int nb, int nt, int nc, void *stream);
+size_t flk_masks_big_bytes(int nb, int nc);
+int flk_masks(const float *d_spec, const float *d_var, const float *d_pp, float *d_big, uint8_t *d_mask, int *h_nmask,
+              float *h_spec, double *d_bsum, float *d_bpwr, float thresh, const int *perm, int nperm, int nb, int nc,
+              void *stream);
+size_t flk_part_bytes(int nb, int nt, int nc);
+int flk_apply(uint8_t *d_data, const float *d_spec0, const float *d_var0, const uint8_t *d_mask, const float *d_bpwr,
+              uint16_t *d_part, const double *d_bsum, int *d_ran, int *h_ran, float prev, float jump, int force, int nb,
+              int nt, int nc, void *stream);
+int flk_tsmask_flagts(uint8_t *d_data, const uint16_t *d_part, float *d_ts, int *d_idx, int *d_nts, int *h_nts,
+                      const int *d_ran, const float *d_bpwr, float thr, int nb, int nt, int nc, void *stream);
 int flk_flag_ts(uint8_t *d_data, const uint8_t *d_mask, const float *d_bpwr, float *d_ts, int nb, int nt, int nc,
                 void *stream);
 int flk_flagts(uint8_t *d_data, const int *d_midx, int n, const float *d_bpwr, int nb, int nt, int nc,
@@ -119,12 +133,14 @@ int dsaxfl_fix_zspec(float *d_s0, float *d_v0, int nbc, int naver, void *stream)
 struct dsaxfl_plan {
   dsaxfl_config cfg;
   hipStream_t stream;
-  float *d_spec0, *d_var0, *d_spec, *d_var, *d_pp, *d_ts, *d_bpwr;
+  hipEvent_t masked;               /* the masks and the host's spectrum are there */
+  float *d_spec0, *d_var0, *d_spec, *d_var, *d_pp, *d_ts, *d_bpwr, *d_big;
   uint8_t *d_mask, *d_repval;
-  int *d_tsidx;
-  float *h_spec, *h_var, *h_pp, *h_ts, *h_bpwr;
-  uint8_t *h_cmask;
-  int *h_mask, *h_tsmask, *h_tsidx;
+  uint16_t *d_part;                /* row sums of each slab of channels */
+  double *d_bsum;                  /* per-beam sums of the spectrum */
+  int *d_tsidx, *d_nts, *d_ran;
+  float *h_spec, *h_var;           /* pinned */
+  int *h_nmask, *h_nts, *h_ran;    /* pinned, written by the kernels */
   float prev_tpwr;
   int have_ref;
 };
@@ -157,15 +173,17 @@ void dsaxfl_destroy(dsaxfl_plan *p) {
   hipFree(p->d_mask);
   hipFree(p->d_repval);
   hipFree(p->d_tsidx);
+  hipFree(p->d_big);
+  hipFree(p->d_part);
+  hipFree(p->d_bsum);
+  hipFree(p->d_nts);
+  hipFree(p->d_ran);
   hipHostFree(p->h_spec);
   hipHostFree(p->h_var);
-  hipHostFree(p->h_pp);
-  hipHostFree(p->h_ts);
-  hipHostFree(p->h_bpwr);
-  hipHostFree(p->h_cmask);
-  hipHostFree(p->h_tsidx);
-  free(p->h_mask);
-  free(p->h_tsmask);
+  hipHostFree(p->h_nmask);
+  hipHostFree(p->h_nts);
+  hipHostFree(p->h_ran);
+  if (p->masked) hipEventDestroy(p->masked);
   if (p->stream) hipStreamDestroy(p->stream);
   free(p);
 }
@@ -204,19 +222,21 @@ int dsaxfl_create(dsaxfl_plan **out, const dsaxfl_config *cfg) {
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_tsidx, nbt * 4);
   if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_spec, nbc * 4, 0);
   if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_var, nbc * 4, 0);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_pp, nbc * 4, 0);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_ts, nbt * 4, 0);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_bpwr, (size_t)nb * 4, 0);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_cmask, nbc, 0);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_tsidx, nbt * 4, 0);
-  p->h_mask = malloc(nbc * sizeof(int));
-  p->h_tsmask = malloc(nbt * sizeof(int));
-  if (e != hipSuccess || !p->h_mask || !p->h_tsmask) {
+  if (e == hipSuccess && flk_masks_big_bytes(nb, nc)) e = hipMalloc((void **)&p->d_big, flk_masks_big_bytes(nb, nc));
+  if (e == hipSuccess) e = hipMalloc((void **)&p->d_part, flk_part_bytes(nb, nt, nc));
+  if (e == hipSuccess) e = hipMalloc((void **)&p->d_bsum, (size_t)nb * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc((void **)&p->d_nts, (size_t)nb * sizeof(int));
+  if (e == hipSuccess) e = hipMalloc((void **)&p->d_ran, sizeof(int));
+  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_nmask, (size_t)nb * sizeof(int), 0);
+  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_nts, (size_t)nb * sizeof(int), 0);
+  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_ran, sizeof(int), 0);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&p->masked, hipEventDisableTiming);
+  if (e != hipSuccess) {
     dsaxfl_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "flagger allocation failed: %s", hipGetErrorString(e));
   }
-  for (int b = 0; b < nb; b++) p->h_bpwr[b] = 1.f;       /* gpu_flagger.cu:1234 */
-  e = hipMemcpyAsync(p->d_bpwr, p->h_bpwr, (size_t)nb * 4, hipMemcpyHostToDevice, p->stream);
+  for (int b = 0; b < nb; b++) p->h_spec[b] = 1.f;       /* bpwr, gpu_flagger.cu:1234 */
+  e = hipMemcpyAsync(p->d_bpwr, p->h_spec, (size_t)nb * 4, hipMemcpyHostToDevice, p->stream);
   int rc = e == hipSuccess ? flk_genrand(p->d_repval, (size_t)nt * nc, cfg->seed, p->stream) : -1;
   if (rc == 0) e = hipStreamSynchronize(p->stream);
   if (e != hipSuccess || rc) {
@@ -302,6 +322,20 @@ int dsaxfl_set_total_power(dsaxfl_plan *p, float prev_tpwr) {
     if (rc_) return dsaxbf_fail(rc_ == -3 ? DSAXBF_EHIP : DSAXBF_EINVAL, "%s", bfk_last_error()); \
   } while (0)
 
+/* The second pass and the time masks; force: whatever the device makes of the
+ * total power. */
+static int apply(dsaxfl_plan *p, uint8_t *d_data, int force) {
+  const dsaxfl_config *c = &p->cfg;
+  const int nb = c->nbeam, nt = c->ntime, nc = c->nchan;
+  uint16_t *d_part = c->tsflag ? p->d_part : NULL;
+  FCALL(flk_apply(d_data, p->d_spec0, p->d_var0, p->d_mask, p->d_bpwr, d_part, p->d_bsum, p->d_ran, p->h_ran,
+                  p->prev_tpwr, c->mod_thresh, force, nb, nt, nc, p->stream));
+  if (d_part)
+    FCALL(flk_tsmask_flagts(d_data, d_part, p->d_ts, p->d_tsidx, p->d_nts, p->h_nts, p->d_ran, p->d_bpwr, c->tsthresh,
+                            nb, nt, nc, p->stream));
+  return DSAXBF_OK;
+}
+
 int dsaxfl_step(dsaxfl_plan *p, uint8_t *d_data, dsaxfl_step_info *info) {
   dsaxbf_clear_error();
   if (!p || !d_data) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
@@ -309,59 +343,47 @@ int dsaxfl_step(dsaxfl_plan *p, uint8_t *d_data, dsaxfl_step_info *info) {
   HCALL(hipSetDevice(p->cfg.device), "hipSetDevice");
   const dsaxfl_config *c = &p->cfg;
   const int nb = c->nbeam, nt = c->ntime, nc = c->nchan;
-  const size_t nbc = (size_t)nb * nc, nbt = (size_t)nb * nt;
+  const size_t nbc = (size_t)nb * nc;
   hipStream_t s = p->stream;
-  /* scaley + spectrum, varspec, ppspec of the scaled block, one pass */
-  FCALL(flk_stats(d_data, d_data, p->d_spec0, p->d_var0, NULL, p->d_spec, p->d_var, NULL, p->d_pp, nb, nt, nc, s));
-  HCALL(hipMemcpyAsync(p->h_spec, p->d_spec, nbc * 4, hipMemcpyDeviceToHost, s), "D2H spectrum");
-  HCALL(hipMemcpyAsync(p->h_var, p->d_var, nbc * 4, hipMemcpyDeviceToHost, s), "D2H varspec");
-  HCALL(hipMemcpyAsync(p->h_pp, p->d_pp, nbc * 4, hipMemcpyDeviceToHost, s), "D2H ppspec");
-  HCALL(hipStreamSynchronize(s), "statistics");
+  int rc;
+  /* spectrum, varspec and ppspec of the scaled block, which is not written yet */
+  FCALL(flk_stats_scaled(d_data, p->d_spec0, p->d_var0, p->d_spec, p->d_var, p->d_pp, nb, nt, nc, s));
+  /* channflag on spectrum - oldspec (oldspec is never updated from zero in
+     the reference), on varspec at thresh + 0.5 and on its "maxspec" (a
+     second calc_spectrum: the same mask again); simple_channflag on ppspec */
+  FCALL(flk_masks(p->d_spec, p->d_var, p->d_pp, p->d_big, p->d_mask, p->h_nmask, p->h_spec, p->d_bsum,
+                  c->pwr ? p->d_bpwr : NULL, c->thresh, c->perm, c->nperm, nb, nc, s));
+  HCALL(hipEventRecord(p->masked, s), "masks");
+  /* the rest of the step before its total power is known here: the device has
+     a sum of its own to go by, and the block is replaced or the pass run after
+     all where the sum in the reference's order says otherwise */
+  if (c->mkrand) FCALL(flk_noise(d_data, p->d_repval, nb, nt, nc, s));
+  else if ((rc = apply(p, d_data, 0))) return rc;
+  HCALL(hipEventSynchronize(p->masked), "statistics");
   float tpwr = 0.f;
   for (size_t i = 0; i < nbc; i++) tpwr += p->h_spec[i];
   dsaxfl_step_info inf = {tpwr, 0, -1, -1};
   if (fabs(tpwr - p->prev_tpwr) / p->prev_tpwr >= c->mod_thresh) {
     inf.replaced = 1;
-    FCALL(flk_noise(d_data, p->d_repval, nb, nt, nc, s));
+    if (!c->mkrand) FCALL(flk_noise(d_data, p->d_repval, nb, nt, nc, s));
+    HCALL(hipStreamSynchronize(s), "flagger step");
   } else {
-    /* channflag on spectrum - oldspec (oldspec is never updated from zero in
-       the reference), on varspec at thresh + 0.5 and on its "maxspec" (a
-       second calc_spectrum: the same mask again); simple_channflag on ppspec */
-    memset(p->h_mask, 0, nbc * sizeof(int));
-    dsaxfl_channflag(p->h_spec, nb, nc, c->thresh, c->perm, c->nperm, p->h_mask);
-    dsaxfl_channflag(p->h_var, nb, nc, (float)((double)c->thresh + 0.5), c->perm, c->nperm, p->h_mask);
-    dsaxfl_simple_channflag(p->h_pp, nb, nc, c->thresh, p->h_mask);
-    if (c->pwr) dsaxfl_calc_bpwr(p->h_spec, nb, nc, p->h_bpwr);
-    int nm = 0;
-    for (size_t i = 0; i < nbc; i++) {
-      p->h_cmask[i] = p->h_mask[i] == 1;
-      nm += p->h_mask[i] == 1;
+    if (c->mkrand && c->tsflag) {
+      FCALL(flk_flag_ts(d_data, NULL, p->d_bpwr, p->d_ts, nb, nt, nc, s));
+      FCALL(flk_tsmask_flagts(d_data, NULL, p->d_ts, p->d_tsidx, p->d_nts, p->h_nts, NULL, p->d_bpwr, c->tsthresh, nb,
+                              nt, nc, s));
     }
-    inf.n_mask = nm;
-    HCALL(hipMemcpyAsync(p->d_bpwr, p->h_bpwr, (size_t)nb * 4, hipMemcpyHostToDevice, s), "H2D bpwr");
-    float *d_ts = c->tsflag ? p->d_ts : NULL;
-    if (c->mkrand) {
-      FCALL(flk_noise(d_data, p->d_repval, nb, nt, nc, s));
-      if (d_ts) FCALL(flk_flag_ts(d_data, NULL, p->d_bpwr, d_ts, nb, nt, nc, s));
-    } else {
-      HCALL(hipMemcpyAsync(p->d_mask, p->h_cmask, nbc, hipMemcpyHostToDevice, s), "H2D mask");
-      FCALL(flk_flag_ts(d_data, p->d_mask, p->d_bpwr, d_ts, nb, nt, nc, s));
+    HCALL(hipStreamSynchronize(s), "flagger step");
+    if (!c->mkrand && !*p->h_ran) {
+      if ((rc = apply(p, d_data, 1))) return rc;
+      HCALL(hipStreamSynchronize(s), "flagger step");
     }
-    inf.n_tsmask = 0;
-    if (d_ts) {
-      HCALL(hipMemcpyAsync(p->h_ts, d_ts, nbt * 4, hipMemcpyDeviceToHost, s), "D2H ts");
-      HCALL(hipStreamSynchronize(s), "make_ts");
-      memset(p->h_tsmask, 0, nbt * sizeof(int));
-      dsaxfl_simple_tsflag(p->h_ts, nb, nt, c->tsthresh, p->h_tsmask);
-      const int nts = dsaxfl_gather_mask(p->h_tsmask, (long)nbt, p->h_tsidx);
-      inf.n_tsmask = nts;
-      if (nts > 0) {
-        HCALL(hipMemcpyAsync(p->d_tsidx, p->h_tsidx, (size_t)nts * 4, hipMemcpyHostToDevice, s), "H2D ts mask");
-        FCALL(flk_flagts(d_data, p->d_tsidx, nts, p->d_bpwr, nb, nt, nc, s));
-      }
+    inf.n_mask = inf.n_tsmask = 0;
+    for (int b = 0; b < nb; b++) {
+      inf.n_mask += p->h_nmask[b];
+      if (c->tsflag) inf.n_tsmask += p->h_nts[b];
     }
   }
-  HCALL(hipStreamSynchronize(s), "flagger step");
   p->prev_tpwr = tpwr;
   if (info) *info = inf;
   return DSAXBF_OK;

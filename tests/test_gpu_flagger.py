@@ -319,3 +319,73 @@ def test_every_slab_width_matches_oracle(orc, nb, nc):
     for b in beams:
         assert np.array_equal(y[b:b + 1], orc.fl_scaley(x[b:b + 1], spec0[b:b + 1], var0[b:b + 1])), b
     check({k: _get(v, (nb, nc), np.float32) for k, v in outs.items()}, y, beams)
+
+
+@pytest.mark.parametrize("nb,nt,nc,pwr", [(36, 4096, 720, 0), (18, 4096, 1024, 1), (9, 8192, 1040, 0), (2, 4096, 288, 1),
+                                          (1, 4096, 4496, 1)])
+def test_step_over_slab_widths_matches_oracle(orc, nb, nt, nc, pwr):
+    """The block step where its passes take 256, 128, 64 and 32 channels a
+    workgroup (the last slab part-filled), and with more channels than a
+    selection keeps in LDS.  Masked columns and rows, bytes, counts and total
+    power: equal."""
+    print(f"flagger step {nb}x{nt}x{nc} pwr={pwr}", flush=True)
+    cfg = fl.config(nb, nt, nc, pwr=pwr, tsflag=1, tsthresh=6.0, mod_thresh=0.5, seed=3, perm=(10, 200, nc - 129, nc - 128))
+    plan = fl.Plan(cfg)
+    rng = np.random.default_rng(nc)
+    x = _block(nc, nb, nt, nc)
+    spec0 = (x.mean(axis=1) + rng.normal(0, 0.02, (nb, nc))).astype(np.float32)
+    var0 = x.var(axis=1).astype(np.float32)
+    x[0, :, 150 + nb] += 12
+    x[nb - 1, 2000:2040, 128:] = 200
+    plan.set_reference(spec0, var0)
+    prev = np.float32(48.0 * nb * nc)
+    plan.set_total_power(float(prev))
+    d = _dev(x)
+    info = plan.step(d)
+    want, tp, bpwr, nm, _ = orc.fl_step(x, spec0, var0, np.zeros(nt * nc, np.uint8), prev, cfg.mod_thresh, cfg.thresh,
+                                        cfg.tsthresh, pwr=pwr, mkrand=0, tsflag=0, perm=(10, 200, nc - 129, nc - 128),
+                                        bpwr=np.ones(nb, np.float32), exact_var=True)
+    # the series is the mean over every channel (_row_mean), also where nc % 32 != 0
+    rows = np.flatnonzero(orc.fl_mask("simple_tsflag", _row_mean(want), cfg.tsthresh)).astype(np.int32)
+    want, nts = orc.fl_flag(want, rows, bpwr, ts=True), len(rows)
+    assert (info.replaced, info.n_mask, info.n_tsmask, info.tpwr) == (0, nm, nts, np.float32(tp))
+    assert nm > 0 and nts > 0
+    assert np.array_equal(_get(d, x.shape, np.uint8), want)
+    plan.close()
+
+
+@pytest.mark.parametrize("jump", [False, True])
+def test_step_total_power_at_the_threshold(orc, jump):
+    """A power jump so near its threshold that the device's own sum of the
+    spectrum and the reference's float sum fall on different sides: the float
+    sum decides, as in the oracle."""
+    nb, nt, nc = 8, 4096, 1024
+    print(f"flagger step at the power threshold jump={jump}", flush=True)
+    x = _block(61, nb, nt, nc)
+    spec0, var0 = x.mean(axis=1).astype(np.float32), x.var(axis=1).astype(np.float32)
+    spec = orc.fl_stat("spectrum", orc.fl_scaley(x, spec0, var0))
+    total = np.float32(0)
+    for v in spec.ravel():
+        total = np.float32(total + v)
+    exact = spec.astype(np.float64).sum()
+    if jump:                  # the exact sum has not moved, the float sum has
+        prev, thr = np.float32(exact), 1e-7
+        assert abs(exact - float(prev)) / float(prev) < thr <= abs(float(total) - float(prev)) / float(prev)
+    else:                     # the float sum has not moved, the exact sum has
+        prev, thr = total, 1e-9
+        assert abs(exact - float(prev)) / float(prev) >= thr
+    plan = fl.Plan(fl.config(nb, nt, nc, tsflag=1, tsthresh=6.0, mod_thresh=thr, seed=8))
+    plan.set_reference(spec0, var0)
+    plan.set_total_power(float(prev))
+    d = _dev(x)
+    info = plan.step(d)
+    assert info.tpwr == total and info.replaced == int(jump)
+    got = _get(d, x.shape, np.uint8)
+    if jump:
+        rep = np.broadcast_to(orc.fl_genrand(nt * nc, 8).reshape(nt, nc), x.shape).astype(int)
+        assert (np.abs(got.astype(int) - rep) <= 1).all() and (info.n_mask, info.n_tsmask) == (-1, -1)
+    else:
+        want, _, _, nm, nts = orc.fl_step(x, spec0, var0, np.zeros(nt * nc, np.uint8), prev, thr, 5.0, 6.0, pwr=0, mkrand=0,
+                                          tsflag=1, perm=(10,), bpwr=np.ones(nb, np.float32), exact_var=True)
+        assert (info.n_mask, info.n_tsmask) == (nm, nts) and np.array_equal(got, want)
+    plan.close()
