@@ -117,7 +117,10 @@ __device__ inline void fl_lut_build(uint8_t *lut, FlLutScratch<W> &t, const floa
   for (int x = tid / QPR; x < 256; x += 1024 / QPR) {
     uint32_t o = 0;
 #pragma unroll
-    for (int j = 0; j < 4; j++) o |= (fix[j] < 0 ? fl_scale((uint32_t)x, s[j], k[j]) : (uint32_t)fix[j]) << (8 * j);
+    for (int j = 0; j < 4; j++) {
+      const uint32_t v = fl_scale((uint32_t)x, s[j], k[j]);
+      o |= (fix[j] < 0 ? v : (uint32_t)fix[j]) << (8 * j);
+    }
     *(uint32_t *)(lut + x * W + 4 * q) = o;
   }
   __syncthreads();
@@ -154,10 +157,12 @@ __device__ inline uint32_t fl_lut4(const uint8_t *lut, uint32_t x, uint32_t c) {
 // segments w and w + 16 with PF loads in flight.  Rows are taken four at a time
 // and their 4x4 bytes transposed, so that a channel's four samples are one
 // dword: its sum is one sad and its sum of squares one dot product, 16 + 8
-// instructions for 16 samples where byte-wise sums took 64.
+// instructions for 16 samples where byte-wise sums took 64.  PF = 8 is enough
+// where the chip is full (the scaled read-only pass: 8 loads a wave 0.209 ms, 16
+// 0.220); with less to do more loads a wave draw more.
 template <int W, bool SCALE, bool WRITE, bool WMAX>
 __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
-  constexpr int LPR = W / 4, RPI = 64 / LPR, TB = FL_TBIN / RPI, PF = 16;
+  constexpr int LPR = W / 4, RPI = 64 / LPR, TB = FL_TBIN / RPI, PF = W == 256 ? 8 : 16;
   static_assert(TB % PF == 0, "bins end on a prefetch block");
   // the table, and after the pass the waves' sums, in the same LDS
   constexpr int RED = (FL_NSEG + 3 * FL_SW) * W * 4, LUT = SCALE ? 256 * W : 4;
@@ -438,38 +443,75 @@ __device__ inline float fl_unkey(uint32_t k) {
   return __builtin_bit_cast(float, k & 0x80000000u ? k ^ 0x80000000u : ~k);
 }
 
-// The k-th smallest (from 0) of the n keys get(i), found two bits a round from
-// the top by a team of four waves: every thread of the workgroup calls it (it
-// has barriers), teams with data of their own, cnt[2][12] theirs.
-template <class G>
-__device__ inline uint32_t fl_kth(G get, int n, int k, int tid, uint32_t (*cnt)[12]) {
-  uint32_t prefix = 0;
-  int buf = 0;
-  for (int b = 30; b >= 0; b -= 2, buf ^= 1) {
-    const uint32_t t1 = prefix | 1u << b, t2 = prefix | 2u << b, t3 = prefix | 3u << b;
-    uint32_t c1 = 0, c2 = 0, c3 = 0;
-    for (int i0 = 0; i0 < n; i0 += 256) {
-      const uint32_t key = i0 + tid < n ? get(i0 + tid) : 0xFFFFFFFFu;   // (no finite value's key)
-      c1 += __popcll(__ballot(key < t1));
-      c2 += __popcll(__ballot(key < t2));
-      c3 += __popcll(__ballot(key < t3));
-    }
-    if ((tid & 63) == 0) {
-      uint32_t *c = &cnt[buf][(tid >> 6) * 3];
-      c[0] = c1;
-      c[1] = c2;
-      c[2] = c3;
-    }
-    // (a wave that writes this buffer again has passed the next barrier, which
-    // the others reach after reading it)
-    __syncthreads();
-    const uint32_t *c = cnt[buf];
-    const uint32_t uk = (uint32_t)k;
-    const uint32_t digit = (uint32_t)(c[0] + c[3] + c[6] + c[9] <= uk) + (uint32_t)(c[1] + c[4] + c[7] + c[10] <= uk) +
-                           (uint32_t)(c[2] + c[5] + c[8] + c[11] <= uk);
-    prefix |= digit << b;
+// The k-th smallest (from 0) of the n keys get(i), for every thread of a team
+// of four waves.  The keys' range is cut into at most 256 bins of a power of two
+// and the one that holds the k-th taken as the next range: four rounds at most.
+// (One bit a round, counted by one wave or by all of them, took 9 us for 768
+// keys: few waves issue an instruction only every eight cycles or so.)  Every
+// thread of the workgroup calls it (it has barriers), teams with data and FlSel
+// of their own.
+struct FlSel {
+  uint32_t hist[256];
+  uint32_t lo[4], hi[4];             // per wave, then the range in [0]
+  uint32_t k;
+};
+template <class G> __device__ inline uint32_t fl_kth(G get, int n, int k, int tid, FlSel &t) {
+  const int lane = tid & 63;
+  uint32_t lo = 0xFFFFFFFFu, hi = 0;
+  for (int i = tid; i < n; i += 256) {
+    const uint32_t x = get(i);
+    lo = min(lo, x);
+    hi = max(hi, x);
   }
-  return prefix;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+    hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+  }
+  __syncthreads();                   // the last call's reads
+  if (lane == 0) {
+    t.lo[tid >> 6] = lo;
+    t.hi[tid >> 6] = hi;
+  }
+  t.hist[tid] = 0;
+  __syncthreads();
+  lo = min(min(t.lo[0], t.lo[1]), min(t.lo[2], t.lo[3]));
+  hi = max(max(t.hi[0], t.hi[1]), max(t.hi[2], t.hi[3]));
+  uint32_t uk = (uint32_t)k;
+#pragma unroll 1
+  for (int r = 0; r < 4; r++) {
+    const int width = 32 - __builtin_clz((hi - lo) | 1u), s = width > 8 ? width - 8 : 0;
+    for (int i = tid; i < n; i += 256) {
+      const uint32_t x = get(i);
+      if (x >= lo && x <= hi) atomicAdd(&t.hist[(x - lo) >> s], 1u);
+    }
+    __syncthreads();
+    if (tid < 64) {
+      const uint4 c = *(const uint4 *)&t.hist[4 * lane];
+      uint32_t sum = c.x + c.y + c.z + c.w;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t v = (uint32_t)__shfl_up((int)sum, o, 64);
+        if (lane >= o) sum += v;
+      }
+      // the first lane whose running count passes k, and its bin
+      const int at = __ffsll((unsigned long long)__ballot(sum > uk)) - 1;
+      if (lane == at) {
+        uint32_t e = sum - (c.x + c.y + c.z + c.w), bin = 4 * lane;
+        if (uk >= e + c.x) { e += c.x; bin++; if (uk >= e + c.y) { e += c.y; bin++; if (uk >= e + c.z) { e += c.z; bin++; } } }
+        t.k = uk - e;
+        t.lo[0] = lo + (bin << s);
+        t.hi[0] = min(hi, lo + (bin << s) + ((1u << s) - 1));
+      }
+    }
+    __syncthreads();
+    lo = t.lo[0];
+    hi = t.hi[0];
+    uk = t.k;
+    t.hist[tid] = 0;
+    __syncthreads();
+  }
+  return lo;
 }
 
 // Median of 21 values: of 12 the smallest and the largest are dropped and the
@@ -516,11 +558,13 @@ struct FlMasks {
 // waves per statistic.  Every float and double operation of the reference's CPU
 // code, in its order; medians are selections, so which equal element is taken
 // does not matter.  Workgroup (beam, 1): the spectrum to the host, its sum, and
-// calc_bpwr.  64 beams x 1024 channels: 11 us for what took the host, with the
-// copies both ways, about 0.6 ms.
+// calc_bpwr.  64 beams x 1024 channels: 20-30 us (a spread of the writes to host
+// memory) for what took the host, with the copies both ways, about 0.6 ms.
+// Bound by its barriers and the latency of few waves.
 __global__ __launch_bounds__(768) void fl_masks_kernel(FlMasks a) {
   __shared__ float val[3][FL_LDSN];
-  __shared__ uint32_t cnt[3][2][12];
+  __shared__ FlSel sel[3];
+  __shared__ uint32_t cnt[12];
   __shared__ double red[12];
   const int bm = blockIdx.x, tid = threadIdx.x;
   const size_t at = (size_t)bm * a.nc;
@@ -573,8 +617,8 @@ __global__ __launch_bounds__(768) void fl_masks_kernel(FlMasks a) {
   }
   __syncthreads();
   const int k = (nin + 1) / 2 - 1;
-  const float med = fl_unkey(fl_kth([&](int i) { return fl_key(v[i]); }, nin, k, tt, cnt[team]));
-  const float mad = fl_unkey(fl_kth([&](int i) { return fl_key(fabsf(__fsub_rn(v[i], med))); }, nin, k, tt, cnt[team]));
+  const float med = fl_unkey(fl_kth([&](int i) { return fl_key(v[i]); }, nin, k, tt, sel[team]));
+  const float mad = fl_unkey(fl_kth([&](int i) { return fl_key(fabsf(__fsub_rn(v[i], med))); }, nin, k, tt, sel[team]));
   const float lim = __fmul_rn(a.thr[team], mad);
   // (teams that set the same byte store the same value)
   if (team < 2) {
@@ -593,10 +637,10 @@ __global__ __launch_bounds__(768) void fl_masks_kernel(FlMasks a) {
   uint32_t m = 0;
   for (int c = tid; c < a.nc; c += 768) m += mask[c];
   for (int o = 32; o > 0; o >>= 1) m += __shfl_xor(m, o, 64);
-  if ((tid & 63) == 0) cnt[0][0][tid >> 6] = m;
+  if ((tid & 63) == 0) cnt[tid >> 6] = m;
   __syncthreads();
   if (tid == 0) {
-    for (int i = 1; i < 12; i++) m += cnt[0][0][i];
+    for (int i = 1; i < 12; i++) m += cnt[i];
     a.h_nmask[bm] = (int)m;
   }
 }
@@ -615,10 +659,11 @@ struct FlTsMask {
 // make_ts's division and simple_tsflag (gpu_flagger.cu:413-452,662-700): a
 // workgroup per beam, the series' median and MAD over its first ntime/16
 // samples, and the list of its flagged rows.  (The four teams of four waves
-// each select the same values; the order of the list does not matter.)
+// each select the same values; the order of the list does not matter.)  64 x
+// 16384: 23 us, bound by the latency of 64 workgroups.
 __global__ __launch_bounds__(1024) void fl_tsmask_kernel(FlTsMask a) {
   __shared__ float val[FL_LDSN];
-  __shared__ uint32_t cnt[4][2][12];
+  __shared__ FlSel sel[4];
   __shared__ uint32_t nf;
   const int bm = blockIdx.x, tid = threadIdx.x, tt = tid & 255, team = tid >> 8;
   const int nm = a.nt / 16;
@@ -631,8 +676,11 @@ __global__ __launch_bounds__(1024) void fl_tsmask_kernel(FlTsMask a) {
   }
   if (a.part) {
     const uint16_t *p = a.part + (size_t)bm * a.nslab * a.nt;
+    const double rnc = __ddiv_rn(1., (double)a.nc);
+#pragma unroll 2
     for (int t = tid * 4; t < a.nt; t += 4096) {
       uint32_t s[4] = {0, 0, 0, 0};
+#pragma unroll 4
       for (int k = 0; k < a.nslab; k++) {
         const uint2 v = *(const uint2 *)(p + (size_t)k * a.nt + t);
         s[0] += v.x & 0xFFFFu;
@@ -640,9 +688,15 @@ __global__ __launch_bounds__(1024) void fl_tsmask_kernel(FlTsMask a) {
         s[2] += v.y & 0xFFFFu;
         s[3] += v.y >> 16;
       }
+      // s / nc by its reciprocal and one exact remainder: a quotient that a
+      // double holds comes out exact, another one within an ulp of a double,
+      // which is far nearer than a float's rounding boundary can be
       float f[4];
 #pragma unroll
-      for (int j = 0; j < 4; j++) f[j] = (float)__ddiv_rn((double)s[j], (double)a.nc);
+      for (int j = 0; j < 4; j++) {
+        const double d = (double)s[j], q = d * rnc;
+        f[j] = (float)__builtin_fma(__builtin_fma(-q, (double)a.nc, d), rnc, q);
+      }
       *(float4 *)(ts + t) = make_float4(f[0], f[1], f[2], f[3]);
     }
     __syncthreads();
@@ -654,12 +708,18 @@ __global__ __launch_bounds__(1024) void fl_tsmask_kernel(FlTsMask a) {
   }
   __syncthreads();
   const int k = (nm + 1) / 2 - 1;
-  const float med = fl_unkey(fl_kth([&](int i) { return fl_key(v[i]); }, nm, k, tt, cnt[team]));
-  const float mad = fl_unkey(fl_kth([&](int i) { return fl_key(fabsf(__fsub_rn(v[i], med))); }, nm, k, tt, cnt[team]));
+  const float med = fl_unkey(fl_kth([&](int i) { return fl_key(v[i]); }, nm, k, tt, sel[team]));
+  const float mad = fl_unkey(fl_kth([&](int i) { return fl_key(fabsf(__fsub_rn(v[i], med))); }, nm, k, tt, sel[team]));
   const float lim = __fmul_rn(a.thr, mad);
   int *idx = a.idx + (size_t)bm * a.nt;
-  for (int t = tid; t < a.nt; t += 1024)
-    if (__fsub_rn(ts[t], med) > lim) idx[atomicAdd(&nf, 1u)] = bm * a.nt + t;
+#pragma unroll 4
+  for (int t = tid * 4; t < a.nt; t += 4096) {
+    const float4 f = *(const float4 *)(ts + t);
+    const float x[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (__fsub_rn(x[j], med) > lim) idx[atomicAdd(&nf, 1u)] = bm * a.nt + t + j;
+  }
   __syncthreads();
   if (tid == 0) a.n_ts[bm] = a.h_nts[bm] = (int)nf;
 }
