@@ -23,7 +23,9 @@
 //                     its unsynchronised max-then-min tree leaves in slot 0).
 //   fl_flag_ts_kernel one pass that replaces the masked (beam, channel)
 //                     columns and sums each row of the flagged block (flag +
-//                     make_ts): a wave per row, 16 bytes per lane.
+//                     make_ts): 16 bytes per lane.
+//   fl_masks_kernel, fl_apply_kernel, fl_tsmask_kernel: the block step's masks
+//                     and its second pass (scale, flag, row sums).
 //   fl_flagts_kernel  the masked (beam, time) rows, channels 128..nchan-129.
 //   and elementwise kernels for sumpulse, genrand (own counter-based
 //   generator), the noise replacement copy and fix_zspec's median.
@@ -36,7 +38,13 @@ constexpr int FL_SW = 16;      // waves per stats workgroup
 constexpr int FL_NSEG = 32;    // the reference's threads per (beam, channel)
 constexpr int FL_TBIN = 128;   // ppspec bin
 constexpr double FL_MN = 48.0, FL_SIG = 6.0;
-constexpr int FL_RPW = 16;     // rows per wave in fl_flag_ts_kernel
+constexpr int FL_RPW = 16;     // loads per wave in fl_flag_ts_kernel
+// Cache policy of the slab passes' buffer loads and stores: non-temporal where a
+// slab's rows are whole 128-byte lines (the statistics of 64 x 16384 x 1024 at
+// 256 channels: 0.195 -> 0.174 ms, with scaley 0.479 -> 0.468; 30 x 16384 x 640 at
+// 128: 64 -> 61 us), not where neighbouring slabs share them (12 x 8192 x 400 at
+// 32 channels: 16 us, 29 non-temporal).
+template <int W> constexpr int fl_policy() { return W >= 128 ? 2 : 0; }
 
 // (unsigned char)(__float2uint_rn(2 * val) / 2): round half to even, the
 // saturating conversion (NaN and negatives to 0), halve, keep the low byte.
@@ -147,7 +155,7 @@ __device__ inline uint32_t fl_lut4(const uint8_t *lut, uint32_t x, uint32_t c) {
 // Every statistic of a (beam, W-channel slab) in one pass, optionally through
 // scaley's table (SCALE) and writing the scaled block (WRITE).  Bound by the
 // stream over the block where the grid fills the chip: 64 x 16384 x 1024 takes
-// 0.197 ms (5.4 TB/s), 0.475 ms with scaley (4.5 TB/s read and written, a plain
+// 0.174 ms (6.2 TB/s), 0.468 ms with scaley (4.6 TB/s read and written, a plain
 // copy 5.1).  12 x 8192 x 400 takes 16 and 31 us (51 and 102 us on 24 workgroups
 // of 256 channels).
 //
@@ -158,8 +166,9 @@ __device__ inline uint32_t fl_lut4(const uint8_t *lut, uint32_t x, uint32_t c) {
 // and their 4x4 bytes transposed, so that a channel's four samples are one
 // dword: its sum is one sad and its sum of squares one dot product, 16 + 8
 // instructions for 16 samples where byte-wise sums took 64.  PF = 8 is enough
-// where the chip is full (the scaled read-only pass: 8 loads a wave 0.209 ms, 16
-// 0.220); with less to do more loads a wave draw more.
+// where the chip is full (the scaled read-only pass took 0.209 ms with 8 loads a
+// wave and 0.220 with 16; 0.186 with non-temporal loads since); with less to do
+// more loads a wave draw more.
 template <int W, bool SCALE, bool WRITE, bool WMAX>
 __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
   constexpr int LPR = W / 4, RPI = 64 / LPR, TB = FL_TBIN / RPI, PF = W == 256 ? 8 : 16;
@@ -192,7 +201,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
   };
   uint32_t buf[PF];
 #pragma unroll
-  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(d), 0);
+  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(d), fl_policy<W>());
   if constexpr (SCALE)
     fl_lut_build<W>(lut, lt, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, nullptr, 0, slab, a.nc);
   uint32_t S[4] = {0, 0, 0, 0}, Q[4] = {0, 0, 0, 0}, bs[4] = {0, 0, 0, 0};
@@ -209,7 +218,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
           // (every lane: cl + 3 < W keeps a non-live lane's lookups in the
           // table, and its statistics are never written)
           if (SCALE) x[r] = fl_lut4<W>(lut, x[r], (uint32_t)cl);
-          if (WRITE) __builtin_amdgcn_raw_buffer_store_b32(x[r], rout, vo, row(i0 + d + r), 0);
+          if (WRITE) __builtin_amdgcn_raw_buffer_store_b32(x[r], rout, vo, row(i0 + d + r), fl_policy<W>());
           if (WMAX) {
             typedef unsigned short us2 __attribute__((ext_vector_type(2)));
             const uint32_t e = x[r] & 0x00FF00FFu, o = (x[r] >> 8) & 0x00FF00FFu;
@@ -231,7 +240,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
         // registers whose loads are still in flight
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          buf[d + r] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(i0 + PF + d + r), 0);
+          buf[d + r] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(i0 + PF + d + r), fl_policy<W>());
         __builtin_amdgcn_sched_barrier(0);
       }
       if (((i0 - h * n1 + PF) & (TB - 1)) == 0) {          // end of a 128-sample bin
@@ -398,7 +407,7 @@ __global__ __launch_bounds__(1024) void fl_apply_kernel(FlApply a) {
   auto row = [&](int i) { return (r0 + (uint32_t)(min(i, n - 1) * RPI)) * (uint32_t)a.nc; };
   uint32_t buf[PF];
 #pragma unroll
-  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(d), 0);
+  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(d), fl_policy<W>());
   fl_lut_build<W>(lut, lt, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, a.mask + (size_t)bm * a.nc,
                   fl_rep(a.bpwr[bm]), slab, a.nc);
   uint16_t *part = a.part ? a.part + (size_t)item * a.nt : nullptr;
@@ -407,10 +416,10 @@ __global__ __launch_bounds__(1024) void fl_apply_kernel(FlApply a) {
 #pragma unroll
     for (int d = 0; d < PF; d++) {
       const uint32_t x = fl_lut4<W>(lut, buf[d], (uint32_t)cl);
-      __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, vo, row(i0 + d), 0);
+      __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, vo, row(i0 + d), fl_policy<W>());
       rs[d] = __builtin_amdgcn_sad_u8(x, 0u, 0u);
       // (past the end this wave's last row again, into registers that are not used)
-      buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(i0 + PF + d), 0);
+      buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(i0 + PF + d), fl_policy<W>());
       __builtin_amdgcn_sched_barrier(0);
     }
     if (part) {
@@ -724,11 +733,6 @@ __global__ __launch_bounds__(1024) void fl_tsmask_kernel(FlTsMask a) {
   if (tid == 0) a.n_ts[bm] = a.h_nts[bm] = (int)nf;
 }
 
-__device__ inline uint32_t fl_wave_sum(uint32_t v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 // bytes != 0 -> 0xFF, == 0 -> 0x00
 __device__ inline uint32_t fl_bytemask(uint32_t x) {
   x |= (x >> 4) & 0x0F0F0F0Fu;
@@ -737,33 +741,54 @@ __device__ inline uint32_t fl_bytemask(uint32_t x) {
   return (x & 0x01010101u) * 0xFFu;
 }
 
+// Sums of 16 rows over the LPR lanes of a row, for the lane's row
+// (lane % LPR) / (LPR / 16): as fl_row_sums, in 32 bits.
+template <int LPR> __device__ inline uint32_t fl_row_sums32(const uint32_t (&rs)[FL_RPW], int lane) {
+  static_assert(FL_RPW == 16 && LPR >= 16, "four folds");
+  uint32_t p[8], q[4], r[2], v;
+#pragma unroll
+  for (int k = 0; k < 8; k++) p[k] = fl_fold<LPR / 2>(rs[k], rs[k + 8], lane);
+#pragma unroll
+  for (int k = 0; k < 4; k++) q[k] = fl_fold<LPR / 4>(p[k], p[k + 4], lane);
+#pragma unroll
+  for (int k = 0; k < 2; k++) r[k] = fl_fold<LPR / 8>(q[k], q[k + 2], lane);
+  v = fl_fold<LPR / 16>(r[0], r[1], lane);
+  if constexpr (LPR == 64) v += fl_xor_lane<2>(v);
+  if constexpr (LPR >= 32) v += fl_xor_lane<1>(v);
+  return v;
+}
+
 // Replace the masked columns (mask[bm][ch] != 0) with the beam's byte and,
 // when ts is given, write ts[bm][t] = (sum over channels of the flagged row)
-// / nchan.  A wave per FL_RPW consecutive rows of one beam, 16 bytes per lane.
+// / nchan.  LPR lanes read a row, 16 bytes each (64, or 32 and 16 for rows of
+// fewer 16-byte chunks, so that lanes are not idle: make_ts of 12 x 8192 x 400
+// takes 8 us where a wave per row took 16), a wave FL_RPW loads of 64/LPR rows each.
 // A lane stores its chunk when the chunk holds a masked column, or, when at
 // least a quarter of the wave's chunks do, every lane stores (unchanged chunks
 // are written back as read): on the 64 x 16384 x 1024 block, 5 % of columns
 // masked at random touch every line of a row, and whole rows then take
-// 0.436 ms against 0.459 ms as scattered chunks, while 0.5 % at random or a
-// 64-channel band run faster as chunks (0.357 and 0.343 ms, against 0.431
-// whole).
+// 0.382 ms against 0.430 ms as scattered chunks, while 0.5 % at random or a
+// 64-channel band run faster as chunks (0.305 and 0.271 ms, against 0.414
+// whole).  (Row sums by a cross-lane sum per row: 0.425 ms with 5 %.)
+template <int LPR, bool MASK>
 __global__ __launch_bounds__(256) void fl_flag_ts_kernel(uint8_t *data, const uint8_t *mask,
                                                          const float *bpwr, float *ts, int nb, int nt,
                                                          int nc) {
-  const int lane = threadIdx.x & 63;
+  constexpr int RPI = 64 / LPR;                // rows per load
+  const int lane = threadIdx.x & 63, l = lane & (LPR - 1), rg = lane / LPR;
   const long gw = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int wpb = nt / FL_RPW;                 // waves per beam
+  const int wpb = nt / (FL_RPW * RPI);         // waves per beam
   if (gw >= (long)nb * wpb) return;            // the whole wave leaves together
-  const int bm = (int)(gw / wpb), t0 = (int)(gw % wpb) * FL_RPW;
+  const int bm = (int)(gw / wpb), t0 = (int)(gw % wpb) * FL_RPW * RPI;
   const int nq = nc / 16;                      // 16-byte chunks per row
-  const uint32_t rep = mask ? fl_rep(bpwr[bm]) * 0x01010101u : 0u;
+  const uint32_t rep = MASK ? fl_rep(bpwr[bm]) * 0x01010101u : 0u;
   uint32_t rs[FL_RPW];
 #pragma unroll
   for (int r = 0; r < FL_RPW; r++) rs[r] = 0;
-  for (int q = lane; q - lane < nq; q += 64) {
+  for (int q = l; q - l < nq; q += LPR) {
     if (q >= nq) break;
     uint4 m = make_uint4(0, 0, 0, 0);
-    if (mask) {
+    if (MASK) {
       m = *(const uint4 *)(mask + (size_t)bm * nc + 16 * q);
       m = make_uint4(fl_bytemask(m.x), fl_bytemask(m.y), fl_bytemask(m.z), fl_bytemask(m.w));
     }
@@ -771,10 +796,10 @@ __global__ __launch_bounds__(256) void fl_flag_ts_kernel(uint8_t *data, const ui
     // (both ballots in every active lane: under `own ||` they would run only
     // in the lanes whose chunk is clean)
     const bool whole = 4 * __popcll(__ballot(own)) >= __popcll(__ballot(1));
-    const bool any = own || whole;
+    const bool any = MASK && (own || whole);
 #pragma unroll
     for (int r = 0; r < FL_RPW; r++) {
-      uint4 *pv = (uint4 *)(data + ((size_t)bm * nt + t0 + r) * nc + 16 * q);
+      uint4 *pv = (uint4 *)(data + ((size_t)bm * nt + t0 + r * RPI + rg) * nc + 16 * q);
       uint4 v = *pv;
       if (any) {
         v.x = (v.x & ~m.x) | (rep & m.x);
@@ -790,11 +815,9 @@ __global__ __launch_bounds__(256) void fl_flag_ts_kernel(uint8_t *data, const ui
     }
   }
   if (ts) {
-#pragma unroll
-    for (int r = 0; r < FL_RPW; r++) {
-      const uint32_t s = fl_wave_sum(rs[r]);
-      if (lane == 0) ts[(size_t)bm * nt + t0 + r] = (float)__ddiv_rn((double)s, (double)nc);
-    }
+    const uint32_t s = fl_row_sums32<LPR>(rs, lane);
+    if (l % (LPR / 16) == 0)
+      ts[(size_t)bm * nt + t0 + l / (LPR / 16) * RPI + rg] = (float)__ddiv_rn((double)s, (double)nc);
   }
 }
 
@@ -1041,9 +1064,22 @@ extern "C" int flk_tsmask_flagts(uint8_t *d_data, const uint16_t *d_part, float 
 extern "C" int flk_flag_ts(uint8_t *d_data, const uint8_t *d_mask, const float *d_bpwr, float *d_ts, int nb,
                            int nt, int nc, void *stream) {
   if (!fl_shape_ok(nb, nt, nc, "flk_flag_ts")) return -1;
-  const long waves = (long)nb * (nt / FL_RPW);
-  hipLaunchKernelGGL(fl_flag_ts_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
-                     d_data, d_mask, d_bpwr, d_ts, nb, nt, nc);
+  // lanes per row: no more than the row has 16-byte chunks, in powers of two
+  const int lpr = nc > 512 ? 64 : nc > 256 ? 32 : 16;
+  const long waves = (long)nb * (nt / (FL_RPW * (64 / lpr)));
+  const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
+  hipStream_t s = (hipStream_t)stream;
+#define FL_FLAG_TS(L)                                                                                       \
+  do {                                                                                                      \
+    if (d_mask) hipLaunchKernelGGL((fl_flag_ts_kernel<L, true>), grid, block, 0, s, d_data, d_mask, d_bpwr, \
+                                   d_ts, nb, nt, nc);                                                       \
+    else hipLaunchKernelGGL((fl_flag_ts_kernel<L, false>), grid, block, 0, s, d_data, d_mask, d_bpwr, d_ts, \
+                            nb, nt, nc);                                                                    \
+  } while (0)
+  if (lpr == 64) FL_FLAG_TS(64);
+  else if (lpr == 32) FL_FLAG_TS(32);
+  else FL_FLAG_TS(16);
+#undef FL_FLAG_TS
   return bfk_check(hipGetLastError(), "fl_flag_ts_kernel");
 }
 

@@ -389,3 +389,22 @@ def test_step_total_power_at_the_threshold(orc, jump):
                                           tsflag=1, perm=(10,), bpwr=np.ones(nb, np.float32), exact_var=True)
         assert (info.n_mask, info.n_tsmask) == (nm, nts) and np.array_equal(got, want)
     plan.close()
+
+
+@pytest.mark.parametrize("nc", [16, 256, 272, 512, 528])
+def test_row_lanes_at_every_width(orc, nc):
+    """flag_mask with make_ts and make_ts alone where 16, 32 and 64 lanes read a
+    row, at the widths on each side: bytes and row means equal."""
+    nb, nt = 3, 4096
+    print(f"flagger row lanes nc={nc}", flush=True)
+    rng = np.random.default_rng(nc)
+    x = rng.integers(0, 256, (nb, nt, nc), dtype=np.uint8)
+    m = (rng.random((nb, nc)) < np.array([0.0, 0.02, 0.4])[:, None]).astype(np.uint8)
+    bp = np.array([1.0, 1.3, 0.7], np.float32)
+    d, d_ts = _dev(x), DeviceBuffer(nb * nt * 4)
+    fl.make_ts(d, nb, nt, nc, d_ts)
+    assert np.array_equal(_get(d_ts, (nb, nt), np.float32), _row_mean(x))
+    fl.flag_mask(d, nb, nt, nc, _dev(m), _dev(bp), d_ts)
+    want = orc.fl_flag(x, np.flatnonzero(m.ravel()).astype(np.int32), bp)
+    assert np.array_equal(_get(d, x.shape, np.uint8), want)
+    assert np.array_equal(_get(d_ts, (nb, nt), np.float32), _row_mean(want))
