@@ -68,7 +68,81 @@ extern "C" int bfk_beamform_shared8(const bfk_dims *d, const uint8_t *d_in, cons
                                    const float *d_wscale, const float *d_scale, uint8_t *d_out,
                                    float *d_power, float *d_bpart, void *stream);
 
+extern "C" int bfk_beamform_spread(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag, const float *d_wscale,
+                                   const float *d_scale, uint8_t *d_out, float *d_power, float *d_bpart, int nbw,
+                                   int pol_outer, void *stream);
+
 extern "C" int bfk_classic_beams(int variant, int nkc);
+
+// Spread tiles or the plan's variant (bf_launch.h), by the times below in us,
+// measured on blocks of 8 to 384 channels, 64 to 4096 samples and 20 to 1024
+// beams.
+//   spread: one workgroup per CU, t0 + t1 per 32-beam tile (FP6 three-part 13 %
+//     more), in rounds of 256; the beam tiles are dealt evenly to the sets.
+//   the variants: the 256-, 128- or 64-beam tiles of up to 64 antennas run two
+//     workgroups a CU (t1 with one each at most, t2 once most have two, per512 in
+//     the steady state), the 8-wave tiles of more antennas one (per round of 256).
+// A block alone takes `alone`; where several streams have blocks in flight (three
+// were measured), a pass takes `among`: a third of that latency, or its share of
+// the chip.  Spread tiles run where neither is longer, with the set size that
+// makes their product least.  E.g. 56 channels x 512 samples -> 256 beams of 64
+// antennas FP16: alone 41 -> 18 us, among others 16 -> 12.5; 100 antennas FP8: 55
+// -> 26 alone but 19 -> 22 among others, left alone.  Past one round, fine weights
+// of more than 64 antennas no longer share their rows in an XCD's L2 (825 tiles,
+// 300 beams FP6 three-part: 538 -> 395 alone, 500 -> 690 among others).
+struct TileTimes {
+  float t1, t2, per512;
+};
+struct TileCost {
+  float alone, among;
+};
+static TileCost variant_cost(const bfk_dims *d) {
+  const int k = d->nkc == 1 ? 0 : d->nkc == 2 ? 1 : 2;
+  const bool group = d->wmode == 0;
+  int beams = bfk_classic_beams(d->variant, d->nkc);
+  if (d->variant == BFK_VAR_SHARED_256) beams = 256;
+  const long n = (long)(d->nsamp / TCU) * d->ngroup * ((d->nbeam + beams - 1) / beams);
+  if (beams == 256 && d->nkc > 1) {
+    static const float per[2][2][4] = {{{68, 57, 49.5f, 70}, {66, 57, 48.5f, 67}}, {{150, 133, 126, 0}, {143, 123, 110, 0}}};
+    const float p = per[k - 1][group][d->prec], alone = (float)((n + 255) / 256) * p;
+    return {alone, fmaxf(alone / 3, (float)n * p / 256)};
+  }
+  static const TileTimes shared[2][4] = {{{38, 53, 58}, {33, 49, 52}, {31, 38, 43}, {39, 52, 59}},
+                                         {{36, 50, 54}, {28, 43, 44}, {22, 34, 35}, {26, 42, 46}}};
+  static const TileTimes half[3] = {{22, 42, 37}, {48, 87, 70}, {133, 256, 185}};      // 128 beams
+  static const TileTimes quarter[3] = {{17, 33, 26}, {35, 67, 45}, {106, 222, 137}};   // 64 beams
+  const TileTimes &t = beams == 256 ? shared[group][d->prec] : beams == 128 ? half[k] : quarter[k];
+  const float steady = (float)n * t.per512 / 512;
+  const float alone = n <= 256   ? t.t1
+                      : n <= 512 ? beams == 256 ? t.t2 : fminf(t.t2, t.t1 + (t.t2 - t.t1) * (float)(n - 256) / 192)
+                                 : fmaxf(t.t2, steady);
+  return {alone, fmaxf(alone / 3, steady)};
+}
+extern "C" int bfk_spread_tiles(const bfk_dims *d) {
+  static const float t0[3][2] = {{4.5f, 4.6f}, {5.5f, 5.f}, {17.5f, 16.f}}, t1[3][2] = {{3.9f, 3.6f}, {7.6f, 7.4f}, {15.f, 14.f}};
+  const int k = d->nkc == 1 ? 0 : d->nkc == 2 ? 1 : 2;
+  const bool group = d->wmode == 0;
+  const long ntile = (long)(d->nsamp / TCU) * d->ngroup;
+  const int live = (d->nbeam + 31) / 32;
+  const TileCost v = variant_cost(d);
+  float best = 0.f;
+  int tiles = 0;
+  for (int nset = (live + 15) / 16; nset <= live; nset++) {
+    const int nbw = (live + nset - 1) / nset;
+    const long wgs = ntile * nset, rounds = (wgs + 255) / 256;
+    if (!group && rounds > (d->nkc == 1 ? 2 : 1)) break;
+    const float wg = t0[k][group] + nbw * t1[k][group] * (d->prec == 3 ? 1.13f : 1.f);
+    // (blocks in flight together contend for the weights' bytes)
+    const float share = group || d->nkc == 1 ? 1.05f : d->prec == 3 ? 1.5f : 1.25f;
+    const float alone = rounds * wg, among = fmaxf(alone / 3, (float)wgs * wg / 256 * share);
+    if (alone * 1.08f > v.alone || among > v.among) continue;
+    if (!tiles || alone * among < best) {
+      best = alone * among;
+      tiles = nbw;
+    }
+  }
+  return tiles;
+}
 
 extern "C" int bfk_variant_supported(const bfk_dims *d, int v) {
   if (d->nant_pad != 64 * d->nkc || (d->nkc != 1 && d->nkc != 2 && d->nkc != 4)) return 0;
@@ -89,6 +163,14 @@ extern "C" int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *
   if (!bfk_variant_supported(d, d->variant)) {
     bfk_set_error("bfk_beamform: variant %d cannot run this shape (nant_pad %d)", d->variant, d->nant_pad);
     return -1;
+  }
+  if (const int nbw = d->pinned ? 0 : bfk_spread_tiles(d)) {
+    // the order in which the variant adds the (channel, pol) powers: the shared
+    // tiles take group weights pol-outer, except the two-part splits from 32
+    // samples a bin on (bf_shared.hip)
+    const int pol_outer = d->variant == BFK_VAR_SHARED_256 && d->nkc == 1 && d->wmode == 0 &&
+                          !((d->prec == 1 || d->prec == 2) && d->tavg >= 32);
+    return bfk_beamform_spread(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, nbw, pol_outer, stream);
   }
   if (d->variant == BFK_VAR_SHARED_256)
     return d->nkc == 1 ? bfk_beamform_shared(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, stream)

@@ -33,6 +33,7 @@ typedef struct bfk_dims {
   int stuff;      /* 0 none, 1 antennas, 2 incoherent beam 0              */
   int variant;    /* fused-kernel variant, BFK_VAR_*                      */
   int layout;     /* output layout: 0 [t][beam][g], 1 [beam][t][g]        */
+  int pinned;     /* 1: run `variant` itself, never the spread tiles      */
 } bfk_dims;
 
 /* Variants of the fused beamformer (same bits, different speed):
@@ -75,6 +76,11 @@ int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
 
 /* 1 if variant v (BFK_VAR_*) can run dims d, else 0. */
 int bfk_variant_supported(const bfk_dims *d, int v);
+
+/* 32-beam tiles per workgroup of the spread tiles (bf_spread.hip: the bits of
+ * the variant, for blocks whose tiles would leave the chip part idle) that
+ * bfk_beamform runs in the variant's place unless it is pinned, or 0. */
+int bfk_spread_tiles(const bfk_dims *d);
 
 /* Batched classic launches: all blocks of a batch in one launch per kernel
  * instantiation (precision, tavg, antenna chunks, beam tiles per wave).

@@ -190,7 +190,7 @@ static int time_graph(dsaxbf_batch *b, int reps, float *out_ms) {
 /* Set the plans' variants to v[] and capture the graph again. */
 static int apply(dsaxbf_batch *b, const int *v) {
   for (int i = 0; i < b->n; i++) {
-    int rc = dsaxbf_set_variant(b->plans[i], v[i]);
+    int rc = dsaxbf_pick_variant(b->plans[i], v[i]);
     if (rc) return rc;
   }
   return build(b);
@@ -220,7 +220,7 @@ int dsaxbf_batch_autotune(dsaxbf_batch *b, int reps, float *ms) {
       }
     if (*best >= 0) continue;
     rc = dsaxbf_time_variants(b->plans[i], b->bufs[i].d_in, b->bufs[i].d_scale, b->bufs[i].d_out, reps,
-                              ms ? ms + (size_t)i * DSAXBF_NVARIANT : NULL, best);
+                              ms ? ms + (size_t)i * DSAXBF_NVARIANT : NULL, best, NULL);
   }
   /* the whole graph decides between the candidates */
   int pick = 0;

@@ -16,8 +16,13 @@ int dsaxbf_plan_internals(dsaxbf_plan *p, struct bfk_dims *dims, void **d_wfrag,
                           float **d_bpart);
 /* Time each variant the plan's shape supports on the given device buffers
  * (reps launches after one warm-up);
- * ms[v] = mean ms or -1, *best = fastest.  The plan's variant is unchanged. */
+ * ms[v] = mean ms or -1, *best = fastest.  With spread_wins, also time what
+ * the plan runs unpinned in its place: 1 if that is no slower (or the same).
+ * The plan's variant is unchanged. */
 int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
-                         int reps, float *ms, int *best);
+                         int reps, float *ms, int *best, int *spread_wins);
+/* dsaxbf_set_variant for the batch layer's own choice: the plan's executes may
+ * still run the spread tiles. */
+int dsaxbf_pick_variant(dsaxbf_plan *p, int v);
 
 #endif

@@ -380,7 +380,15 @@ int dsaxbf_set_variant(dsaxbf_plan *p, int v) {
   if (!bfk_variant_supported(&p->dims, v))
     return dsaxbf_fail(DSAXBF_EINVAL, "variant %d cannot run this shape (nant %d)", v, p->cfg.nant);
   p->dims.variant = v;
+  p->dims.pinned = 1;
   return DSAXBF_OK;
+}
+
+int dsaxbf_pick_variant(dsaxbf_plan *p, int v) {
+  const int pinned = p->dims.pinned;
+  int rc = dsaxbf_set_variant(p, v);
+  p->dims.pinned = pinned;
+  return rc;
 }
 
 int dsaxbf_get_variant(const dsaxbf_plan *p) { return p ? p->dims.variant : -1; }
@@ -397,7 +405,7 @@ int dsaxbf_plan_internals(dsaxbf_plan *p, bfk_dims *dims, void **d_wfrag, float 
 }
 
 int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
-                         int reps, float *ms, int *best_out) {
+                         int reps, float *ms, int *best_out, int *spread_wins) {
   if (!p || !d_in || !d_scale || !d_out) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
   if (reps < 1) return dsaxbf_fail(DSAXBF_EINVAL, "reps must be >= 1");
   if (!p->have_weights && p->dims.stuff != DSAXBF_STUFF_ANTS)
@@ -410,15 +418,19 @@ int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_sca
     hipEventDestroy(e0);
     return dsaxbf_fail(DSAXBF_EHIP, "hipEventCreate: %s", hipGetErrorString(he));
   }
-  const int keep = p->dims.variant;
+  const int keep = p->dims.variant, keep_pinned = p->dims.pinned;
   int best = keep, rc = DSAXBF_OK;
-  float best_ms = -1.f;
-  for (int v = 0; v < DSAXBF_NVARIANT && rc == DSAXBF_OK; v++) {
-    if (!bfk_variant_supported(&p->dims, v)) {
+  float best_ms = -1.f, spread_ms = -1.f;
+  for (int v = 0; v <= DSAXBF_NVARIANT && rc == DSAXBF_OK; v++) {
+    /* every variant itself, then what runs unpinned in the best one's place */
+    const int unpinned = v == DSAXBF_NVARIANT;
+    if (!unpinned && !bfk_variant_supported(&p->dims, v)) {
       if (ms) ms[v] = -1.f;   /* not a candidate for this shape */
       continue;
     }
-    p->dims.variant = v;
+    p->dims.variant = unpinned ? best : v;
+    p->dims.pinned = !unpinned;
+    if (unpinned && (!spread_wins || !bfk_spread_tiles(&p->dims))) break;
     float t = 0.f;
     he = hipSuccess;
     for (int r = -1; r < reps && rc == DSAXBF_OK && he == hipSuccess; r++) {
@@ -434,6 +446,10 @@ int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_sca
       break;
     }
     t /= (float)reps;
+    if (unpinned) {
+      spread_ms = t;
+      break;
+    }
     if (ms) ms[v] = t;
     if (best_ms < 0.f || t < best_ms) {
       best_ms = t;
@@ -443,7 +459,9 @@ int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_sca
   hipEventDestroy(e0);
   hipEventDestroy(e1);
   p->dims.variant = keep;
+  p->dims.pinned = keep_pinned;
   if (best_out) *best_out = best;
+  if (spread_wins) *spread_wins = spread_ms < 0.f || spread_ms <= best_ms;
   return rc;
 }
 
@@ -454,8 +472,11 @@ int dsaxbf_autotune(dsaxbf_plan *p, int reps, float *ms) {
   /* any voltages do: the work does not depend on the values */
   HIPCHK(hipMemsetAsync(p->d_in, 0x5a, dsaxbf_input_bytes(&p->cfg), p->stream), "hipMemsetAsync");
   HIPCHK(hipMemsetAsync(p->d_scale, 0, sizeof(float) * p->cfg.nbeam, p->stream), "hipMemsetAsync");
-  int best;
-  int rc = dsaxbf_time_variants(p, p->d_in, p->d_scale, p->d_out, reps, ms, &best);
-  if (rc == DSAXBF_OK) p->dims.variant = best;
+  int best, spread;
+  int rc = dsaxbf_time_variants(p, p->d_in, p->d_scale, p->d_out, reps, ms, &best, &spread);
+  if (rc == DSAXBF_OK) {
+    p->dims.variant = best;
+    p->dims.pinned = !spread;
+  }
   return rc;
 }

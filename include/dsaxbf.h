@@ -242,6 +242,9 @@ int dsaxbf_beam_power(dsaxbf_plan *plan, float *d_beam_power, void *stream);
  *                  8 waves of 32 beams (nant > 64) (default above 128 beams).
  * Value 1 is retired (a persistent schedule that never won): no shape
  * supports it, and dsaxbf_set_variant rejects it.
+ * A plan whose variant nobody set runs, where its tiles would leave the chip
+ * part idle, smaller work items in the variant's place (one 32-beam tile and one
+ * channel and pol per wave) with the variant's bits.
  * No counterpart in the reference (its five kernels per int have one fixed
  * launch shape, dsaX_beamformer.cu:955-1003). */
 enum {
@@ -253,14 +256,14 @@ enum {
   DSAXBF_NVARIANT = 6
 };
 
-/* Select the variant used by later executes on this plan; DSAXBF_EINVAL if
- * it cannot run the plan's shape. */
+/* Run this variant in later executes on this plan, whatever the block's size;
+ * DSAXBF_EINVAL if it cannot run the plan's shape. */
 int dsaxbf_set_variant(dsaxbf_plan *plan, int variant);
 int dsaxbf_get_variant(const dsaxbf_plan *plan);
 
 /* Autotuner: times every variant the shape supports (the plan's own device
  * buffers, current weights; reps launches each after one warm-up) and keeps
- * the fastest.  ms, if not NULL, receives DSAXBF_NVARIANT mean launch times in
+ * the fastest (or the smaller work items above, where they are no slower).  ms, if not NULL, receives DSAXBF_NVARIANT mean launch times in
  * milliseconds (-1 for a variant that cannot run this shape).  Synchronous;
  * requires dsaxbf_set_weights (or -s mode).  No counterpart in the reference. */
 int dsaxbf_autotune(dsaxbf_plan *plan, int reps, float *ms);

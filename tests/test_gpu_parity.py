@@ -666,3 +666,38 @@ def test_batch_graph_matches_per_block(bf):
     batch.close()
     for p in plans:
         p.close()
+
+
+@pytest.mark.parametrize("tavg", [8, 16, 32, 64])
+@pytest.mark.parametrize("prec", [0, 1, 2, 3])
+def test_spread_tiles_have_the_variants_bits(bf, prec, tavg):
+    """Blocks too small to fill the chip run spread tiles (one 32-beam tile and
+    one channel and pol per wave) unless a variant is set: output, power and beam
+    power equal the variant's bit for bit, with one and several beam tiles a
+    workgroup, part-filled beam tiles and antennas, group widths that are and
+    are not multiples of four, both input orders and output layouts, fine and
+    group weights (whose steps the shared tiles of up to 64 antennas take
+    pol-outer).  (antennas, channels, packets, beams) at each antenna chunk count:
+    one tile; a ragged set; the most beams; enough tiles for sets of several."""
+    shapes = [(1, 8, 32, 1), (64, 8, 32, 32), (30, 40, 96, 100), (64, 32, 64, 1024), (63, 56, 512, 256), (65, 16, 64, 33),
+              (128, 32, 96, 540), (100, 56, 256, 300)]
+    if prec < 3:
+        shapes += [(129, 8, 32, 31), (256, 24, 64, 300), (200, 40, 256, 256)]
+    for i, (nant, nchan, npkt, nbeam) in enumerate(shapes):
+        for fine in (False, True):
+            print(f"spread prec={prec} tavg={tavg} {nant}x{nchan}x{npkt}->{nbeam} fine={fine}", flush=True)
+            cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, precision=prec,
+                            weight_mode=int(fine), angle_mode=bf.ANGLE_SIN, input_order=i & 1, output_layout=(i >> 1) & 1)
+            antpos, cal, theta = bf.synth_geometry(nant, cfg.ncal, nbeam, 5 + i)
+            block = bf.synth_block(cfg, 90 + i)
+            scale = np.full(nbeam, 2e-3 / nant, np.float32)
+            got = []
+            for pin in (False, True):
+                plan = bf.Plan(cfg)
+                plan.set_weights(antpos, cal, bf.reference_freqs(1498.75, nchan), theta)
+                if pin:
+                    plan.variant = plan.variant
+                got.append(plan.process_block(block, scale, want_power=True, want_beam_power=True))
+                plan.close()
+            for a, b in zip(*got):
+                assert np.array_equal(a, b)
