@@ -178,6 +178,11 @@ struct BfArgs {
   int kind;                               // tile schedule of a mixed batch job (MIX_*)
   uint32_t pstride, astride, gstride;     // input bytes per packet, antenna, channel group
   uint32_t in_bytes, wfrag_bytes, wscale_bytes;
+  // spread tiles that sum the beam powers themselves (beam_power NULL: not): their
+  // copy of the per-unit sums [beam / 32][nsamp/32][ngroup][beam % 32], and the
+  // workgroups of each beam set that have finished
+  float *beam_power, *psum;
+  unsigned *count;
 };
 
 // Output (and power) index of bin o, beam b, group g: [o][beam][g], the
@@ -700,8 +705,9 @@ __device__ __forceinline__ void stage_store(uint8_t *stage, const uint32_t (&v)[
 // tt_first + k (k < ntt); lanes h = 0 and h = 1 hold the two row halves of each
 // bin.  TAVG 64 has one bin per tile, the sum of both units' halves, so it
 // needs ntt = 2.  Each unit's sum per beam (the AGC input) goes to bpart
-// [nbeam][nsamp/32][ngroup].
-template <int TAVG, int NB>
+// [nbeam][nsamp/32][ngroup], and with PSUM to psum too, past this XCD's L2 for a
+// reader on another XCD in the same launch.
+template <int TAVG, int NB, bool PSUM = false>
 __device__ __forceinline__ void tile_output(const BfArgs &a, const TileId &t, int btw, int n, int h,
                                             float (&part)[2][NB][TAVG <= 32 ? 32 / TAVG : 1],
                                             int tt_first, int ntt) {
@@ -721,7 +727,11 @@ __device__ __forceinline__ void tile_output(const BfArgs &a, const TileId &t, in
         unit_sum += x[k][j];
       }
       const int tt = tt_first + k;
-      if (own) a.bpart[((long)b * 2 * a.ntblk + 2 * t.tblk + tt) * a.ngroup + t.g] = unit_sum;
+      const int unit = (2 * t.tblk + tt) * a.ngroup + t.g;
+      if (PSUM && a.beam_power && h == 0)   // (beams past nbeam: sums of zero weights, not read)
+        __hip_atomic_store(a.psum + ((long)(btw + bt) * 2 * a.ntblk * a.ngroup + unit) * 32 + n, unit_sum,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (own) a.bpart[(long)b * 2 * a.ntblk * a.ngroup + unit] = unit_sum;
       if (TAVG < 64 && own)
 #pragma unroll
         for (int j = 0; j < NP; j++) {

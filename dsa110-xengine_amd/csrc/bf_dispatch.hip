@@ -55,6 +55,8 @@ BfArgs bf_make_args(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
   a.wfrag_bytes = (uint32_t)bfk_wfrag_bytes(d);
   a.wscale_bytes = (uint32_t)bfk_wscale_bytes(d);
   a.split = 0;
+  a.beam_power = a.psum = NULL;
+  a.count = NULL;
   return a;
 }
 
@@ -69,8 +71,8 @@ extern "C" int bfk_beamform_shared8(const bfk_dims *d, const uint8_t *d_in, cons
                                    float *d_power, float *d_bpart, void *stream);
 
 extern "C" int bfk_beamform_spread(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag, const float *d_wscale,
-                                   const float *d_scale, uint8_t *d_out, float *d_power, float *d_bpart, int nbw,
-                                   int pol_outer, void *stream);
+                                   const float *d_scale, uint8_t *d_out, float *d_power, float *d_bpart, float *d_beam_power, void *d_psum,
+                                   int nbw, int pol_outer, void *stream);
 
 extern "C" int bfk_classic_beams(int variant, int nkc);
 
@@ -154,7 +156,9 @@ extern "C" int bfk_variant_supported(const bfk_dims *d, int v) {
 
 extern "C" int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                             const float *d_wscale, const float *d_scale, uint8_t *d_out,
-                            float *d_power, float *d_bpart, void *stream) {
+                            float *d_power, float *d_bpart, float *d_beam_power, void *d_psum,
+                            int *summed, void *stream) {
+  *summed = 0;
   // buffer offsets are 32-bit
   if ((size_t)d->npkt * d->nant * d->nchan * 4 > 0x7fffffffu || bfk_wfrag_bytes(d) > 0x7fffffffu) {
     bfk_set_error("bfk_beamform: block or weights above 2 GiB");
@@ -170,7 +174,10 @@ extern "C" int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *
     // samples a bin on (bf_shared.hip)
     const int pol_outer = d->variant == BFK_VAR_SHARED_256 && d->nkc == 1 && d->wmode == 0 &&
                           !((d->prec == 1 || d->prec == 2) && d->tavg >= 32);
-    return bfk_beamform_spread(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, nbw, pol_outer, stream);
+    if (!d_psum || !bfk_psum_bytes(d)) d_beam_power = NULL;
+    *summed = d_beam_power != NULL;
+    return bfk_beamform_spread(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, d_beam_power, d_psum,
+                               nbw, pol_outer, stream);
   }
   if (d->variant == BFK_VAR_SHARED_256)
     return d->nkc == 1 ? bfk_beamform_shared(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, stream)

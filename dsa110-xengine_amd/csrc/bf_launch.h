@@ -69,10 +69,18 @@ int bfk_weights(const bfk_dims *d, const float *d_antpos, const float *d_cal,
 size_t bfk_bpart_bytes(const bfk_dims *d);
 
 /* Fused unpack -> MFMA beam GEMM -> |B|^2 -> average -> requantise.
- * d_power is optional; d_bpart receives the per-tile beam power sums. */
+ * d_power is optional; d_bpart receives the per-tile beam power sums.
+ * d_beam_power (optional) receives bfk_beam_power's sums where the launch makes
+ * them itself (*summed 1; else the caller asks bfk_beam_power).  It does so with
+ * d_psum (NULL: it does not): bfk_psum_bytes, 0 for shapes that never do, for one
+ * launch at a time; the first BFK_COUNTS words of it zero before the first launch
+ * and left zero by each. */
+enum { BFK_COUNTS = 32 };
+size_t bfk_psum_bytes(const bfk_dims *d);
 int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                  const float *d_wscale, const float *d_scale, uint8_t *d_out,
-                 float *d_power, float *d_bpart, void *stream);
+                 float *d_power, float *d_bpart, float *d_beam_power, void *d_psum,
+                 int *summed, void *stream);
 
 /* 1 if variant v (BFK_VAR_*) can run dims d, else 0. */
 int bfk_variant_supported(const bfk_dims *d, int v);

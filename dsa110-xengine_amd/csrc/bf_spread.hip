@@ -39,6 +39,7 @@ template <int NKC, int NP> struct Spread {
   static constexpr int SH = NCH == 4 ? 2 : NCH == 8 ? 1 : 0;
   static constexpr int STAGE = 16 * RS * ROW;
   static constexpr int XBUF = 16 * NU * NP * 64;  // floats: [cq][unit][bin][lane]
+  static_assert(XBUF >= SW * 64, "the beam power sums reuse it");
   static constexpr int SBUF = 16 * 32;            // floats: [cq][beam] weight scales
   // two exchange buffers where they fit: one barrier per beam tile, else two;
   // the scales beside them where those fit (not 128 or 256 antennas in 8-sample
@@ -95,6 +96,54 @@ __device__ __forceinline__ void spread_unit(f16v &cr, f16v &ci, WFrag<PREC, 1, 1
       ci = mfma64<PREC>(aim, W.lo[0][0][s2], ci, W.slo(0, 0, s2));
       if (pf) W.load_one_rb(src, wnext, 0, s2);
     }
+  }
+}
+
+// The beam power sums of the set's beam tiles bt0 .. bt0 + nbt - 1, as
+// bf_beam_power_kernel (bf_aux.hip) adds up to 1792 per-unit sums a beam.  There thread 64 q + l adds sums 64 q + l + 256 k (one
+// after another), each wave q its threads' by lane ^ 32, 16, ..., 1, and the four
+// waves (0 + 1) + (2 + 3).  Here wave 4 j + q of the workgroup is pass q of beam
+// tile j, a lane one beam: half h holds l = 32 h .. 32 h + 31, so the first step
+// adds across the halves and the others in registers.  (Which of two values
+// comes first does not matter.)  The sums [unit][32 beams] are read in whole lines
+// past this XCD's L2, 32 loads in flight; those past the end read as zeros, the
+// whole offset being the lane's (a scalar offset past the buffer's size would wrap
+// the check).
+__device__ __forceinline__ void spread_beam_power(const BfArgs &a, int bt0, int nbt, int wave, int lane, float *lds) {
+  constexpr int SC1 = 16;            // agent-scope loads
+  const int n = 2 * a.ntblk * a.ngroup, q = wave & 3, h = lane >> 5;
+  for (int j0 = 0; j0 < nbt; j0 += 4) {
+    const int bt = bt0 + j0 + (wave >> 2);
+    float v[32];
+#pragma unroll
+    for (int l = 0; l < 32; l++) v[l] = 0.f;
+    if (j0 + (wave >> 2) < nbt) {
+      const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(a.psum + (long)bt * n * 32, (uint32_t)n * 128u);
+      for (int k = 0; 64 * q + 256 * k < n; k++)
+#pragma unroll
+        for (int l = 0; l < 32; l++)
+          v[l] += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                rs, (uint32_t)(64 * q + 256 * k + 32 * h + l) * 128u + (lane & 31) * 4u,
+                                                0, SC1));
+    }
+#pragma unroll
+    for (int l = 0; l < 32; l++) {
+      const uint32_t x = __builtin_bit_cast(uint32_t, v[l]);
+      const auto s = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+      const uint32_t lo = s[0], hi = s[1];       // (bit_cast of s[1] itself takes s[0])
+      v[l] = __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+    }
+#pragma unroll
+    for (int m = 16; m > 0; m >>= 1)
+#pragma unroll
+      for (int l = 0; l < m; l++) v[l] += v[l + m];
+    __syncthreads();
+    lds[wave * 64 + lane] = v[0];
+    __syncthreads();
+    const float *r = lds + (wave & ~3) * 64 + lane;
+    const int b = bt * 32 + lane;
+    if (q == 0 && lane < 32 && j0 + (wave >> 2) < nbt && b < a.nbeam)
+      a.beam_power[b] = (r[0] + r[64]) + (r[128] + r[192]);
   }
 }
 
@@ -268,12 +317,12 @@ __global__ __launch_bounds__(ST) void bf_spread_kernel(BfArgs a, int nbw, int po
           const int ln = hide(lane);
           add(i, 0, 0, x, ln);
           add(i, 1, 1, x, ln);
-          tile_output<TAVG>(a, t, bt0 + i, ln & 31, ln >> 5, part, 0, 2);
+          tile_output<TAVG, 1, true>(a, t, bt0 + i, ln & 31, ln >> 5, part, 0, 2);
         }
       } else if (cq >> 1 == (i & 7)) {
         const int ln = hide(lane);
         add(i, cq & 1, 0, x, ln);
-        tile_output<TAVG>(a, t, bt0 + i, ln & 31, ln >> 5, part, cq & 1, 1);
+        tile_output<TAVG, 1, true>(a, t, bt0 + i, ln & 31, ln >> 5, part, cq & 1, 1);
       }
       if (S::NX == 1 && i + 1 < nbt) __syncthreads();   // before the buffer is written again
     }
@@ -293,13 +342,31 @@ __global__ __launch_bounds__(ST) void bf_spread_kernel(BfArgs a, int nbw, int po
         if (cq == i) {
           const int ln = hide(lane);
           add(i, u, u, xch[S::NX == 2 ? i & 1 : 0], ln);
-          if (u) tile_output<TAVG>(a, t, bt0 + i, ln & 31, ln >> 5, part, 0, 2);
+          if (u) tile_output<TAVG, 1, true>(a, t, bt0 + i, ln & 31, ln >> 5, part, 0, 2);
         }
         if (S::NX == 1) __syncthreads();                // before the buffer is written again
       }
       if (S::NX == 2) __syncthreads();
     }
   }
+  // (d) the last workgroup of the beam set to finish sums its beams' powers.  The
+  // partial sums are agent-scope stores and loads, past the XCDs' L2s; every
+  // wave waits for its own stores before the barrier, so they are all performed
+  // when the workgroup is counted.  (Fences instead write back and invalidate the
+  // XCD's L2 once a workgroup: 56 channels x 512 samples -> 128 beams 24 us
+  // alone and 18 among others, against 16 and 6.3.)
+  if (!a.beam_power) return;
+  unsigned *last = (unsigned *)xch[0];           // (free once every wave is past its sums)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const unsigned total = (unsigned)(a.ngroup * a.ntblk);
+    *last = atomicInc(a.count + L % nset, total - 1) == total - 1;
+  }
+  __syncthreads();
+  if (!*last) return;
+  __syncthreads();                               // (`last` is read)
+  spread_beam_power(a, bt0, nbt, cq, lane, xch[0]);
 }
 
 template <int PREC, int NKC>
@@ -312,15 +379,36 @@ static void spread_launch(int tavg, dim3 grid, hipStream_t s, const BfArgs &a, i
   }
 }
 
+// Where the launch sums the beam powers: up to one chain (64 antennas) per CU.
+// There a second launch is what bounds a run of blocks (us among others, two
+// launches and one; 64 antennas unless said: 8 channels x 64 samples -> 32 beams
+// 6.5 and 4.0, 8 x 4096 -> 64 8.3 and 5.0, 24 x 3520 -> 30 8.2 and 6.6, 56 x 512 ->
+// 128 6.8 and 6.3, 16 x 512 -> 300 8.1 and 6.2, 100 antennas 24 x 256 -> 64 8.1 and
+// 5.1), against up to 1.1 us more for a block alone (11.1 and 12.2 at the 300
+// beams).  Beyond it the last workgroup's sums cost what the launch did (56 x 512
+// -> 256 12.7 and 12.9, FP6x3 14.4 and 14.9; 100 antennas 88 x 448 -> 125 15.9 and
+// 16.5).
+extern "C" size_t bfk_psum_bytes(const bfk_dims *d) {
+  const long live_bt = (d->nbeam + 31) / 32, chains = live_bt * d->ngroup * (d->nsamp / TCU) * d->nkc;
+  return chains <= 256 && live_bt <= BFK_COUNTS ? (BFK_COUNTS + live_bt * 32 * (d->nsamp / 32) * d->ngroup) * sizeof(float) : 0;
+}
+
 extern "C" int bfk_beamform_spread(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag, const float *d_wscale,
-                                   const float *d_scale, uint8_t *d_out, float *d_power, float *d_bpart, int nbw,
-                                   int pol_outer, void *stream) {
+                                   const float *d_scale, uint8_t *d_out, float *d_power, float *d_bpart,
+                                   float *d_beam_power, void *d_psum, int nbw, int pol_outer, void *stream) {
+  if (d_beam_power && (!d_psum || !bfk_psum_bytes(d))) {
+    bfk_set_error("bfk_beamform_spread: no sums of %d beams x %d units here", d->nbeam, d->nsamp / 32 * d->ngroup);
+    return -1;
+  }
   if (d->nant_pad != 64 * d->nkc || (d->nkc != 1 && d->nkc != 2 && d->nkc != 4) || d->nsamp % TCU || nbw < 1 || nbw > SW ||
       (d->prec == 3 && d->nkc > 2)) {
     bfk_set_error("bfk_beamform_spread: nant_pad=%d nsamp=%d nbw=%d", d->nant_pad, d->nsamp, nbw);
     return -1;
   }
-  const BfArgs a = bf_make_args(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, 32);
+  BfArgs a = bf_make_args(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, 32);
+  a.beam_power = d_beam_power;
+  a.count = (unsigned *)d_psum;
+  a.psum = (float *)d_psum + BFK_COUNTS;
   const int nset = ((d->nbeam + 31) / 32 + nbw - 1) / nbw;
   const dim3 grid((unsigned)((nset * d->ngroup * a.ntblk + 7) / 8 * 8));
   hipStream_t s = (hipStream_t)stream;

@@ -28,6 +28,7 @@ struct dsaxbf_plan {
   float *d_beam_power;
   float *d_scale;
   float *d_bpart;       /* per-tile beam power sums of the last execute */
+  void *d_psum;         /* of launches that sum the beam powers themselves, or NULL */
   void *d_scratch;      /* the device's static scratch array (dsaxbf_execute_noalloc) */
   int have_weights;
 };
@@ -83,6 +84,7 @@ void dsaxbf_destroy(dsaxbf_plan *p) {
   hipFree(p->d_beam_power);
   hipFree(p->d_scale);
   hipFree(p->d_bpart);
+  hipFree(p->d_psum);
   if (p->stream) hipStreamDestroy(p->stream);
   free(p);
 }
@@ -117,6 +119,11 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_beam_power, (size_t)cfg->nbeam * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_scale, (size_t)cfg->nbeam * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_bpart, bfk_bpart_bytes(d));
+  if (bfk_psum_bytes(d)) {
+    if (e == hipSuccess) e = hipMalloc(&p->d_psum, bfk_psum_bytes(d));
+    if (e == hipSuccess) e = hipMemsetAsync(p->d_psum, 0, bfk_psum_bytes(d), p->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
+  }
   if (e != hipSuccess) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "device allocation failed: %s", hipGetErrorString(e));
@@ -276,23 +283,25 @@ int dsaxbf_get_weights(dsaxbf_plan *p, double *w) {
 
 /* One block on device buffers with the per-unit beam-power partial sums in
  * bpart (kernel launches only). */
-static int execute_with(dsaxbf_plan *p, float *bpart, const uint8_t *d_in, const float *d_scale,
+static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, const uint8_t *d_in, const float *d_scale,
                         uint8_t *d_out, float *d_power, float *d_beam_power, void *stream) {
   if (!p || !d_in || !d_scale || !d_out) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
   const bfk_dims *d = &p->dims;
   if (!p->have_weights && d->stuff != DSAXBF_STUFF_ANTS)
     return dsaxbf_fail(DSAXBF_ESTATE, "execute before dsaxbf_set_weights");
   void *s = stream ? stream : (void *)p->stream;
-  int rc;
+  int rc, summed = 0;
   if (d->stuff != DSAXBF_STUFF_ANTS) {
-    rc = bfk_beamform(d, d_in, p->d_wfrag, p->d_wscale, d_scale, d_out, d_power, bpart, s);
+    /* (-q replaces beam 0's partial sums afterwards) */
+    rc = bfk_beamform(d, d_in, p->d_wfrag, p->d_wscale, d_scale, d_out, d_power, bpart,
+                      d->stuff == DSAXBF_STUFF_NONE ? d_beam_power : NULL, psum, &summed, s);
     if (rc) return dsaxbf_fail(rc, "%s", bfk_last_error());
   }
   if (d->stuff != DSAXBF_STUFF_NONE) {
     rc = bfk_stuff(d, d_in, d_scale, d_out, d_power, bpart, s);
     if (rc) return dsaxbf_fail(rc, "%s", bfk_last_error());
   }
-  if (d_beam_power) {
+  if (d_beam_power && !summed) {
     rc = bfk_beam_power(d, bpart, d_beam_power, s);
     if (rc) return dsaxbf_fail(rc, "%s", bfk_last_error());
   }
@@ -302,7 +311,7 @@ static int execute_with(dsaxbf_plan *p, float *bpart, const uint8_t *d_in, const
 int dsaxbf_execute(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
                    float *d_power, float *d_beam_power, void *stream) {
   if (!p) return dsaxbf_fail(DSAXBF_EINVAL, "NULL plan");
-  return execute_with(p, p->d_bpart, d_in, d_scale, d_out, d_power, d_beam_power, stream);
+  return execute_with(p, p->d_bpart, p->d_psum, d_in, d_scale, d_out, d_power, d_beam_power, stream);
 }
 
 int dsaxbf_execute_noalloc(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
@@ -316,7 +325,7 @@ int dsaxbf_execute_noalloc(dsaxbf_plan *p, const uint8_t *d_in, const float *d_s
                        need, have);
   /* every partial sum is overwritten by this launch before it is read: the
      array needs no clearing between calls */
-  return execute_with(p, (float *)p->d_scratch, d_in, d_scale, d_out, d_power, d_beam_power, stream);
+  return execute_with(p, (float *)p->d_scratch, NULL, d_in, d_scale, d_out, d_power, d_beam_power, stream);
 }
 
 int dsaxbf_beam_power(dsaxbf_plan *p, float *d_beam_power, void *stream) {

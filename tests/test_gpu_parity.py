@@ -701,3 +701,31 @@ def test_spread_tiles_have_the_variants_bits(bf, prec, tavg):
                 plan.close()
             for a, b in zip(*got):
                 assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tavg", [8, 64])
+def test_spread_tiles_sum_the_beam_powers(bf, tavg):
+    """Spread launches of up to 256 chains (beam tiles x groups x 64-sample blocks x
+    antenna chunks) sum the beam powers themselves: equal to the pinned variant's
+    sums bit for bit, launch after launch on other blocks, on both sides of the
+    limit, with part-filled beam tiles, several tiles and sets a workgroup, and
+    more than one round of 256 sums a beam."""
+    for prec, nant, nchan, npkt, nbeam in [(0, 64, 8, 32, 1), (0, 30, 8, 8192, 20), (1, 64, 8, 8224, 32),
+                                           (2, 64, 32, 64, 1000), (3, 64, 32, 64, 1024), (0, 200, 16, 160, 97),
+                                           (1, 128, 24, 224, 180), (2, 250, 24, 128, 140)]:
+        print(f"beam powers prec={prec} {nant}x{nchan}x{npkt}->{nbeam}", flush=True)
+        cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, precision=prec,
+                        weight_mode=1, angle_mode=bf.ANGLE_SIN)
+        antpos, cal, theta = bf.synth_geometry(nant, cfg.ncal, nbeam, 7)
+        plans = [bf.Plan(cfg), bf.Plan(cfg)]
+        for plan in plans:
+            plan.set_weights(antpos, cal, bf.reference_freqs(1498.75, nchan), theta)
+        plans[1].variant = plans[1].variant
+        scale = np.full(nbeam, 2e-3 / nant, np.float32)
+        for i in range(3):
+            block = bf.synth_block(cfg, 40 + i)
+            a, b = (plan.process_block(block, scale, want_beam_power=True)[-1] for plan in plans)
+            assert np.array_equal(a, b)
+        for plan in plans:
+            plan.close()
