@@ -729,3 +729,52 @@ def test_spread_tiles_sum_the_beam_powers(bf, tavg):
             assert np.array_equal(a, b)
         for plan in plans:
             plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stuff", [1, 2])
+@pytest.mark.parametrize("tavg", [8, 16, 64])
+def test_stuffed_sums_are_exact(bf, stuff, tavg):
+    """-s and -q beams are whole numbers: equal to integer sums at antenna counts
+    around a wave's eight and a workgroup's 64, with one group, parts of four and
+    several fours, both input orders and output layouts.  The last case, 256
+    antennas at full scale, has sums above 2^24, which are FP32 sums antenna by
+    antenna."""
+    cases = [(1, 8, 32), (7, 24, 64), (8, 32, 32), (63, 40, 96), (64, 64, 64), (65, 16, 32), (200, 56, 32), (256, 32, 32)]
+    for i, (nant, nchan, npkt) in enumerate(cases):
+        for order in (0, 1):
+            nbeam = 70
+            cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, weight_mode=0,
+                            angle_mode=bf.ANGLE_SIN, stuffants=stuff, input_order=order, output_layout=i & 1)
+            rng = np.random.default_rng(i)
+            block = rng.integers(0, 256, npkt * nant * nchan * 4, dtype=np.uint8)
+            if nant == 256:
+                block[:] = 0x88
+                block[::7] = 0x87
+            print(f"stuff={stuff} tavg={tavg} {nant}x{nchan}x{npkt} order={order}", flush=True)
+            plan = bf.Plan(cfg)
+            if stuff == 2:
+                antpos, cal, theta = bf.synth_geometry(nant, cfg.ncal, nbeam, 5)
+                plan.set_weights(antpos, cal, bf.reference_freqs(1498.75, nchan), theta)
+            scale = np.full(nbeam, 3e-4, np.float32)
+            out, power, bp = plan.process_block(block, scale, want_power=True, want_beam_power=True)
+            plan.close()
+            ng = nchan // 8
+            v = block.reshape((npkt, nant, ng, 32) if order == 0 else (npkt, ng, nant, 32))
+            v = v if order == 0 else v.transpose(0, 2, 1, 3)
+            lo, hi = ((v & 15) ^ 8).astype(np.int64) - 8, ((v >> 4) ^ 8).astype(np.int64) - 8
+            s = (lo * lo + hi * hi).sum(-1).reshape(2 * npkt // tavg, tavg // 2, nant, ng).sum(1)
+            if stuff == 2:
+                x = np.zeros((s.shape[0], 1, ng), np.float32)
+                for a in range(nant):
+                    x[:, 0] += s[:, a].astype(np.float32)
+            else:
+                ant = (np.arange(nbeam) // 16 % 4) * 16 + np.arange(nbeam) % 16
+                x = np.where((ant < nant)[None, :, None], s[:, np.minimum(ant, nant - 1)], 0).astype(np.float32)
+            if cfg.output_layout:
+                x = x.transpose(1, 0, 2)
+            nb = 1 if stuff == 2 else nbeam
+            got = power[:nb] if cfg.output_layout else power[:, :nb]
+            got_u8 = out[:nb] if cfg.output_layout else out[:, :nb]
+            assert np.array_equal(got, x)
+            assert np.array_equal(got_u8, (np.rint(x * np.float32(3e-4)).astype(np.int64) // 2 % 256).astype(np.uint8))
