@@ -778,3 +778,31 @@ def test_stuffed_sums_are_exact(bf, stuff, tavg):
             got_u8 = out[:nb] if cfg.output_layout else out[:, :nb]
             assert np.array_equal(got, x)
             assert np.array_equal(got_u8, (np.rint(x * np.float32(3e-4)).astype(np.int64) // 2 % 256).astype(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", PRECS)
+def test_weights_at_the_edges_of_a_threads_antennas(bf, orc, prec):
+    """The weights kernel's threads hold 16 antennas of one beam and its workgroups
+    32 beams: antenna counts around 16, 64 and 128, part-filled beam tiles, both
+    weight modes, some antennas and one whole channel flagged."""
+    for nant, nchan, nbeam in [(1, 8, 1), (15, 8, 32), (17, 16, 33), (49, 8, 257), (64, 8, 31), (65, 8, 64), (128, 8, 40),
+                               (129, 8, 33), (255, 8, 32)]:
+        if prec == 3 and nant > 128:
+            continue
+        for wmode in (0, 1):
+            print(f"weights prec={prec} {nant}x{nchan}->{nbeam} wmode={wmode}", flush=True)
+            cfg = bf.config(nant=nant, nchan=nchan, npkt=32, nbeam=nbeam, tavg=32, precision=prec, weight_mode=wmode,
+                            angle_mode=bf.ANGLE_SIN)
+            antpos, cal, theta = bf.synth_geometry(nant, cfg.ncal, nbeam, nant)
+            cal = np.array(cal)
+            cal[1::5] = 0
+            cal[:, 0, 0] = 0
+            freqs = bf.reference_freqs(1498.75, nchan)
+            plan = bf.Plan(cfg)
+            plan.set_weights(antpos, cal, freqs, theta)
+            got = plan.get_weights()
+            plan.close()
+            W = orc.weights(orc.dims(nant, nchan, 32, nbeam, 32), wmode, 1, antpos, cal, freqs, theta)
+            assert not got[0, 0].any()
+            _check_weights(got, orc.quant_weights(orc.dims(nant, nchan, 32, nbeam, 32), wmode, prec, W))
