@@ -137,10 +137,10 @@ struct dsaxfl_plan {
   float *d_spec0, *d_var0, *d_spec, *d_var, *d_pp, *d_ts, *d_bpwr, *d_big;
   uint8_t *d_mask, *d_repval;
   uint16_t *d_part;                /* row sums of each slab of channels */
-  double *d_bsum;                  /* per-beam sums of the spectrum */
+  double *d_bsum;                  /* per-beam sums of the spectrum, then d_nts and d_ran */
   int *d_tsidx, *d_nts, *d_ran;
-  float *h_spec, *h_var;           /* pinned */
-  int *h_nmask, *h_nts, *h_ran;    /* pinned, written by the kernels */
+  float *h_spec, *h_var;           /* pinned; after h_spec's values */
+  int *h_nmask, *h_nts, *h_ran;    /* those that the kernels write */
   float prev_tpwr;
   int have_ref;
 };
@@ -176,13 +176,8 @@ void dsaxfl_destroy(dsaxfl_plan *p) {
   hipFree(p->d_big);
   hipFree(p->d_part);
   hipFree(p->d_bsum);
-  hipFree(p->d_nts);
-  hipFree(p->d_ran);
   hipHostFree(p->h_spec);
   hipHostFree(p->h_var);
-  hipHostFree(p->h_nmask);
-  hipHostFree(p->h_nts);
-  hipHostFree(p->h_ran);
   if (p->masked) hipEventDestroy(p->masked);
   if (p->stream) hipStreamDestroy(p->stream);
   free(p);
@@ -220,21 +215,21 @@ int dsaxfl_create(dsaxfl_plan **out, const dsaxfl_config *cfg) {
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_mask, nbc);
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_repval, (size_t)nt * nc);
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_tsidx, nbt * 4);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_spec, nbc * 4, 0);
+  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_spec, nbc * 4 + (2 * (size_t)nb + 1) * sizeof(int), 0);
   if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_var, nbc * 4, 0);
   if (e == hipSuccess && flk_masks_big_bytes(nb, nc)) e = hipMalloc((void **)&p->d_big, flk_masks_big_bytes(nb, nc));
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_part, flk_part_bytes(nb, nt, nc));
-  if (e == hipSuccess) e = hipMalloc((void **)&p->d_bsum, (size_t)nb * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void **)&p->d_nts, (size_t)nb * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc((void **)&p->d_ran, sizeof(int));
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_nmask, (size_t)nb * sizeof(int), 0);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_nts, (size_t)nb * sizeof(int), 0);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&p->h_ran, sizeof(int), 0);
+  if (e == hipSuccess) e = hipMalloc((void **)&p->d_bsum, nb * sizeof(double) + (nb + 1) * sizeof(int));
   if (e == hipSuccess) e = hipEventCreateWithFlags(&p->masked, hipEventDisableTiming);
   if (e != hipSuccess) {
     dsaxfl_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "flagger allocation failed: %s", hipGetErrorString(e));
   }
+  p->d_nts = (int *)(p->d_bsum + nb);
+  p->d_ran = p->d_nts + nb;
+  p->h_nmask = (int *)(p->h_spec + nbc);
+  p->h_nts = p->h_nmask + nb;
+  p->h_ran = p->h_nts + nb;
   for (int b = 0; b < nb; b++) p->h_spec[b] = 1.f;       /* bpwr, gpu_flagger.cu:1234 */
   e = hipMemcpyAsync(p->d_bpwr, p->h_spec, (size_t)nb * 4, hipMemcpyHostToDevice, p->stream);
   int rc = e == hipSuccess ? flk_genrand(p->d_repval, (size_t)nt * nc, cfg->seed, p->stream) : -1;
