@@ -74,6 +74,12 @@ extern "C" int bfk_beamform_spread(const bfk_dims *d, const uint8_t *d_in, const
                                    const float *d_scale, uint8_t *d_out, float *d_power, float *d_bpart, float *d_beam_power, void *d_psum,
                                    int nbw, int pol_outer, void *stream);
 
+extern "C" int bfk_beamform_packed(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag, const float *d_wscale,
+                                   const float *d_scale, uint8_t *d_out, float *d_power, float *d_bpart, void *d_packed,
+                                   void *stream);
+// beam sets of `live` beam tiles, and the waves that share a beam tile in one
+extern "C" int bfk_packed_sets(int live);
+extern "C" int bfk_packed_split(int live, int set);
 extern "C" int bfk_classic_beams(int variant, int nkc);
 
 // Spread tiles or the plan's variant (bf_launch.h), by the times below in us,
@@ -120,7 +126,7 @@ static TileCost variant_cost(const bfk_dims *d) {
                                  : fmaxf(t.t2, steady);
   return {alone, fmaxf(alone / 3, steady)};
 }
-extern "C" int bfk_spread_tiles(const bfk_dims *d) {
+static int spread_tiles(const bfk_dims *d, TileCost *cost) {
   static const float t0[3][2] = {{4.5f, 4.6f}, {5.5f, 5.f}, {17.5f, 16.f}}, t1[3][2] = {{3.9f, 3.6f}, {7.6f, 7.4f}, {15.f, 14.f}};
   const int k = d->nkc == 1 ? 0 : d->nkc == 2 ? 1 : 2;
   const bool group = d->wmode == 0;
@@ -141,9 +147,86 @@ extern "C" int bfk_spread_tiles(const bfk_dims *d) {
     if (!tiles || alone * among < best) {
       best = alone * among;
       tiles = nbw;
+      *cost = {alone, among};
     }
   }
   return tiles;
+}
+extern "C" int bfk_spread_tiles(const bfk_dims *d) {
+  TileCost c;
+  return spread_tiles(d, &c);
+}
+
+// Whether a block of more than 64 antennas is repacked (bf_packed.hip), by the us
+// of its workgroups of 8, 4 and 2 beam tiles (one per CU) and the repacking at 5.1
+// TB/s, against the spread tiles or the variant: where the product of the two
+// times (see above) is 5 % less and neither is more than 5 % longer.  256 antennas
+// gain at whole sets of eight beam tiles (256 channels x 4096 samples -> 256 beams,
+// fine weights, alone and among others: FP8 1096/1211 -> 947/920, FP6 1058/1253 ->
+// 830/793), 128 antennas only with fine weights (FP6 three-part 582/751 ->
+// 558/536; FP8 489/542 -> 492/452; group weights, which stay in the L2, 466/457 and
+// 481/439), two beam tiles hardly (256 antennas, group weights FP8: 98/101 and
+// 131/117).
+static TileCost packed_cost(const bfk_dims *d) {
+  static const float per[2][2][3][4] = {
+      {{{112, 92, 74, 110}, {64, 53, 47, 70}, {56, 32, 29, 43}}, {{110, 88, 70, 100}, {62, 48, 41, 60}, {55, 30, 27, 39}}},
+      {{{222, 182, 152, 0}, {135, 117, 104, 0}, {110, 70, 66, 0}}, {{214, 175, 138, 0}, {130, 104, 90, 0}, {115, 68, 62, 0}}}};
+  const float(&p)[3][4] = per[d->nkc == 4][d->wmode == 0];
+  const long tiles = (long)((d->nsamp + 2 * TCU - 1) / (2 * TCU)) * d->ngroup;
+  const int live = (d->nbeam + 31) / 32, nset = bfk_packed_sets(live);
+  // the sets one after another, each workgroup on the CU that is free first: up to
+  // 8 times at which CUs become free (more are taken as the last)
+  struct {
+    float at;
+    long n;
+  } cu[9] = {{0.f, 256}};
+  int ncu = 1;
+  float sum = 0.f, end = 0.f;
+  for (int i = 0; i < nset; i++) {
+    const int split = bfk_packed_split(live, i);
+    const float t = p[split == 1 ? 0 : split == 2 ? 1 : 2][d->prec];
+    sum += t;
+    for (long n = tiles; n > 0;) {
+      if (ncu == 1 && n >= 256) {
+        cu[0].at += t * (float)(n / 256);
+        end = fmaxf(end, cu[0].at);
+        n %= 256;
+        continue;
+      }
+      const long k = n < cu[0].n ? n : cu[0].n;
+      const float at = cu[0].at + t;
+      end = fmaxf(end, at);
+      n -= k;
+      cu[0].n -= k;
+      if (!cu[0].n) {
+        ncu--;
+        for (int j = 0; j < ncu; j++) cu[j] = cu[j + 1];
+      }
+      int j = ncu;
+      for (; j > 0 && cu[j - 1].at > at; j--) cu[j] = cu[j - 1];
+      if (j > 0 && (ncu == 8 || cu[j - 1].at == at)) {
+        cu[j - 1].n += k;
+        for (; j < ncu; j++) cu[j] = cu[j + 1];
+      } else {
+        cu[j].at = at;
+        cu[j].n = k;
+        ncu++;
+      }
+    }
+  }
+  const float pack = 2.f * d->nsamp * d->nchan * (d->nant + d->nant_pad) / 5.1e6f, share = sum * (float)tiles / 256;
+  const float alone = pack + 5 + end;
+  return {alone, fmaxf(alone / 3, share + pack)};
+}
+extern "C" int bfk_use_packed(const bfk_dims *d) {
+  if (d->pinned || !bfk_packed_bytes(d) || !bfk_variant_supported(d, d->variant)) return 0;
+  // (fine weights of 256-beam tiles contend for the L2 among others)
+  static const float contend[4] = {1.05f, 1.1f, 1.25f, 1.27f};
+  TileCost v = variant_cost(d);
+  if (d->variant == BFK_VAR_SHARED_256 && d->wmode != 0) v.among *= contend[d->prec];
+  spread_tiles(d, &v);
+  const TileCost k = packed_cost(d);
+  return k.alone < 1.05f * v.alone && k.among < 1.05f * v.among && k.alone * k.among < 0.95f * v.alone * v.among;
 }
 
 extern "C" int bfk_variant_supported(const bfk_dims *d, int v) {
@@ -157,7 +240,7 @@ extern "C" int bfk_variant_supported(const bfk_dims *d, int v) {
 extern "C" int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                             const float *d_wscale, const float *d_scale, uint8_t *d_out,
                             float *d_power, float *d_bpart, float *d_beam_power, void *d_psum,
-                            int *summed, void *stream) {
+                            int *summed, void *d_packed, void *stream) {
   *summed = 0;
   // buffer offsets are 32-bit
   if ((size_t)d->npkt * d->nant * d->nchan * 4 > 0x7fffffffu || bfk_wfrag_bytes(d) > 0x7fffffffu) {
@@ -168,6 +251,8 @@ extern "C" int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *
     bfk_set_error("bfk_beamform: variant %d cannot run this shape (nant_pad %d)", d->variant, d->nant_pad);
     return -1;
   }
+  if (d_packed)
+    return bfk_beamform_packed(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, d_packed, stream);
   if (const int nbw = d->pinned ? 0 : bfk_spread_tiles(d)) {
     // the order in which the variant adds the (channel, pol) powers: the shared
     // tiles take group weights pol-outer, except the two-part splits from 32

@@ -9,6 +9,7 @@
  */
 #include <hip/hip_runtime_api.h>
 #include <math.h>
+#include <pthread.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -29,6 +30,9 @@ struct dsaxbf_plan {
   float *d_scale;
   float *d_bpart;       /* per-tile beam power sums of the last execute */
   void *d_wargs, *h_wargs;  /* dsaxbf_set_weights' arguments, on the device and packed for it */
+  void *d_packed;       /* the repacked block (or NULL), and its last use */
+  hipEvent_t packed_done;
+  pthread_mutex_t packed_lock;
   void *d_psum;         /* of launches that sum the beam powers themselves, or NULL */
   void *d_scratch;      /* the device's static scratch array (dsaxbf_execute_noalloc) */
   int have_weights;
@@ -91,6 +95,9 @@ void dsaxbf_destroy(dsaxbf_plan *p) {
   hipFree(p->d_scale);
   hipFree(p->d_bpart);
   hipFree(p->d_psum);
+  hipFree(p->d_packed);
+  if (p->packed_done) hipEventDestroy(p->packed_done);
+  pthread_mutex_destroy(&p->packed_lock);
   hipFree(p->d_wargs);
   free(p->h_wargs);
   if (p->stream) hipStreamDestroy(p->stream);
@@ -115,6 +122,7 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   dsaxbf_plan *p = calloc(1, sizeof(*p));
   if (!p) return dsaxbf_fail(DSAXBF_ENOMEM, "plan allocation failed");
   p->cfg = *cfg;
+  pthread_mutex_init(&p->packed_lock, NULL);
   fill_dims(cfg, &p->dims);
   const bfk_dims *d = &p->dims;
   size_t nin = dsaxbf_input_bytes(cfg), nout = dsaxbf_output_bytes(cfg);
@@ -136,6 +144,14 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   if (e != hipSuccess) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "device allocation failed: %s", hipGetErrorString(e));
+  }
+  /* (without the memory for it the block runs the variant) */
+  if (bfk_use_packed(d)) {
+    if (hipEventCreateWithFlags(&p->packed_done, hipEventDisableTiming) != hipSuccess ||
+        hipMalloc(&p->d_packed, bfk_packed_bytes(d)) != hipSuccess) {
+      p->d_packed = NULL;
+      (void)hipGetLastError();
+    }
   }
   p->h_wargs = malloc(wargs_bytes(d));
   if (!p->h_wargs) {
@@ -289,7 +305,7 @@ int dsaxbf_get_weights(dsaxbf_plan *p, double *w) {
 
 /* One block on device buffers with the per-unit beam-power partial sums in
  * bpart (kernel launches only). */
-static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, const uint8_t *d_in, const float *d_scale,
+static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, void *packed, const uint8_t *d_in, const float *d_scale,
                         uint8_t *d_out, float *d_power, float *d_beam_power, void *stream) {
   if (!p || !d_in || !d_scale || !d_out) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
   const bfk_dims *d = &p->dims;
@@ -298,9 +314,28 @@ static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, const uint8_t 
   void *s = stream ? stream : (void *)p->stream;
   int rc, summed = 0;
   if (d->stuff != DSAXBF_STUFF_ANTS) {
+    /* The repacked block: executes of the plan that overlap, on several streams or
+       from several threads, take it in turn.  A graph's replays would not wait for
+       each other, so under capture the block runs without. */
+    if (packed) {
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      if (!bfk_use_packed(d) || hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+        packed = NULL;
+    }
+    if (packed) {
+      pthread_mutex_lock(&p->packed_lock);
+      if (hipStreamWaitEvent(s, p->packed_done, 0) != hipSuccess) {
+        pthread_mutex_unlock(&p->packed_lock);
+        return dsaxbf_fail(DSAXBF_EHIP, "waiting for the repacked block");
+      }
+    }
     /* (-q replaces beam 0's partial sums afterwards) */
     rc = bfk_beamform(d, d_in, p->d_wfrag, p->d_wscale, d_scale, d_out, d_power, bpart,
-                      d->stuff == DSAXBF_STUFF_NONE ? d_beam_power : NULL, psum, &summed, s);
+                      d->stuff == DSAXBF_STUFF_NONE ? d_beam_power : NULL, psum, &summed, packed, s);
+    if (packed) {
+      if (!rc && hipEventRecord(p->packed_done, s) != hipSuccess) hipStreamSynchronize(s);
+      pthread_mutex_unlock(&p->packed_lock);
+    }
     if (rc) return dsaxbf_fail(rc, "%s", bfk_last_error());
   }
   if (d->stuff != DSAXBF_STUFF_NONE) {
@@ -317,7 +352,7 @@ static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, const uint8_t 
 int dsaxbf_execute(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
                    float *d_power, float *d_beam_power, void *stream) {
   if (!p) return dsaxbf_fail(DSAXBF_EINVAL, "NULL plan");
-  return execute_with(p, p->d_bpart, p->d_psum, d_in, d_scale, d_out, d_power, d_beam_power, stream);
+  return execute_with(p, p->d_bpart, p->d_psum, p->d_packed, d_in, d_scale, d_out, d_power, d_beam_power, stream);
 }
 
 int dsaxbf_execute_noalloc(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
@@ -331,7 +366,7 @@ int dsaxbf_execute_noalloc(dsaxbf_plan *p, const uint8_t *d_in, const float *d_s
                        need, have);
   /* every partial sum is overwritten by this launch before it is read: the
      array needs no clearing between calls */
-  return execute_with(p, (float *)p->d_scratch, NULL, d_in, d_scale, d_out, d_power, d_beam_power, stream);
+  return execute_with(p, (float *)p->d_scratch, NULL, NULL, d_in, d_scale, d_out, d_power, d_beam_power, stream);
 }
 
 int dsaxbf_beam_power(dsaxbf_plan *p, float *d_beam_power, void *stream) {
@@ -445,7 +480,7 @@ int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_sca
     }
     p->dims.variant = unpinned ? best : v;
     p->dims.pinned = !unpinned;
-    if (unpinned && (!spread_wins || !bfk_spread_tiles(&p->dims))) break;
+    if (unpinned && (!spread_wins || !(bfk_spread_tiles(&p->dims) || (p->d_packed && bfk_use_packed(&p->dims))))) break;
     float t = 0.f;
     he = hipSuccess;
     for (int r = -1; r < reps && rc == DSAXBF_OK && he == hipSuccess; r++) {

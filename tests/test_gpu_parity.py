@@ -16,6 +16,7 @@ Every beamformed result is checked three ways:
 uint8 bytes are within +-1 LSB everywhere (distance modulo the uint8 wrap).
 Integer-valued outputs (-s, -q) are bit-exact.
 """
+import ctypes
 import os
 import struct
 import subprocess
@@ -806,3 +807,109 @@ def test_weights_at_the_edges_of_a_threads_antennas(bf, orc, prec):
             W = orc.weights(orc.dims(nant, nchan, 32, nbeam, 32), wmode, 1, antpos, cal, freqs, theta)
             assert not got[0, 0].any()
             _check_weights(got, orc.quant_weights(orc.dims(nant, nchan, 32, nbeam, 32), wmode, prec, W))
+
+
+def _use_packed(bf, cfg):
+    """Whether the library repacks blocks of this shape (bf_launch.h's bfk_dims)."""
+    pad = 64 if cfg.nant <= 64 else 128 if cfg.nant <= 128 else 256
+    bpad = (cfg.nbeam + 255) // 256 * 256
+    variant = 5 if cfg.nbeam > 128 or cfg.precision >= 2 else 3 if cfg.nbeam > 64 else 4
+    d = (ctypes.c_int * 21)(cfg.nant, pad, pad // 64, cfg.nchan, cfg.nchan // 8, cfg.npkt, 2 * cfg.npkt, cfg.nbeam, bpad,
+                            bpad // 32, cfg.tavg, 2 * cfg.npkt // cfg.tavg, cfg.ncal, cfg.weight_mode, cfg.angle_mode,
+                            cfg.precision, cfg.input_order, 0, variant, cfg.output_layout, 0)
+    return bool(bf.lib.bfk_use_packed(d))
+
+
+# antennas, channels, packets, beams, precision, fine weights: 128 and 256 padded
+# antennas; 1, 2, 3, 4, 5, 6, 7 and 8 beam tiles in the last set; odd and even
+# numbers of 64-sample blocks; a group count that is and is not a multiple of four
+PACKED = [(70, 104, 640, 150, 0, 1), (66, 112, 608, 290, 0, 1), (67, 120, 768, 100, 1, 0), (68, 104, 640, 190, 1, 1),
+          (65, 56, 640, 290, 2, 0), (65, 96, 704, 70, 2, 1), (67, 104, 640, 1, 3, 1), (127, 112, 672, 224, 3, 1),
+          (132, 112, 736, 70, 0, 1), (133, 112, 608, 256, 0, 0), (130, 64, 512, 100, 1, 1), (129, 72, 480, 400, 1, 0),
+          (131, 48, 448, 190, 2, 1), (256, 104, 640, 1, 2, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tavg", [8, 16, 32, 64])
+def test_packed_blocks_have_the_variants_bits(bf, tavg):
+    """Blocks of more than 64 antennas that are repacked first: output, power and
+    beam power equal the pinned variant's bit for bit, both input orders and
+    output layouts, also after a block with other voltages."""
+    for i, (nant, nchan, npkt, nbeam, prec, fine) in enumerate(PACKED):
+        if (i + tavg.bit_length()) % 2:      # (each shape at two of the four)
+            continue
+        print(f"packed {nant}x{nchan}x{npkt}->{nbeam} prec={prec} fine={fine} tavg={tavg}", flush=True)
+        cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, precision=prec, weight_mode=fine,
+                        angle_mode=bf.ANGLE_SIN, input_order=(i >> 1) & 1, output_layout=(i >> 2) & 1)
+        assert _use_packed(bf, cfg)
+        antpos, cal, theta = bf.synth_geometry(nant, cfg.ncal, nbeam, 5 + i)
+        scale = np.full(nbeam, 2e-3 / nant, np.float32)
+        plans = [bf.Plan(cfg), bf.Plan(cfg)]
+        for plan in plans:
+            plan.set_weights(antpos, cal, bf.reference_freqs(1498.75, nchan), theta)
+        plans[1].variant = plans[1].variant
+        rng = np.random.default_rng(i)
+        for _ in range(2):
+            block = rng.integers(0, 256, bf.input_bytes(cfg), dtype=np.uint8)
+            for a, b in zip(*(plan.process_block(block, scale, want_power=True, want_beam_power=True) for plan in plans)):
+                assert np.array_equal(a, b)
+        for plan in plans:
+            plan.close()
+
+
+@pytest.mark.gpu
+def test_packed_blocks_on_several_streams_and_in_a_graph(bf):
+    """One plan's repacked blocks queued on three streams without a wait between
+    them, and captured in a graph that is replayed between eager executes, each
+    give their own block's output."""
+    hip = bf.lib                     # (the HIP runtime is among its dependencies)
+
+    def ok(rc):
+        assert rc == 0
+
+    nant, nchan, npkt, nbeam, prec, fine = PACKED[3]
+    cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=16, precision=prec, weight_mode=fine)
+    assert _use_packed(bf, cfg)
+    antpos, cal, theta = bf.synth_geometry(nant, cfg.ncal, nbeam, 3)
+    plan = bf.Plan(cfg)
+    plan.set_weights(antpos, cal, bf.reference_freqs(1498.75, nchan), theta)
+    scale = np.full(nbeam, 2e-3 / nant, np.float32)
+    rng = np.random.default_rng(1)
+    blocks = [rng.integers(0, 256, bf.input_bytes(cfg), dtype=np.uint8) for _ in range(3)]
+    want = [plan.process_block(b, scale)[0].ravel() for b in blocks]
+    d_scale, ins, outs = bf.DeviceBuffer(scale.nbytes), [], []
+    d_scale.upload(scale)
+    for b in blocks:
+        ins.append(bf.DeviceBuffer(b.nbytes))
+        ins[-1].upload(b)
+        outs.append(bf.DeviceBuffer(want[0].nbytes))
+    streams = [ctypes.c_void_p() for _ in range(3)]
+    for s in streams:
+        ok(hip.hipStreamCreateWithFlags(ctypes.byref(s), 1))
+    run = lambda k: plan.execute(ins[k], d_scale, outs[k], stream=streams[k])  # noqa: E731
+
+    def check():
+        ok(hip.hipDeviceSynchronize())
+        for k in range(3):
+            assert np.array_equal(outs[k].download(np.empty_like(want[k])), want[k])
+            outs[k].upload(np.zeros_like(want[k]))
+
+    for _ in range(4):
+        for k in range(3):
+            run(k)
+    check()
+    graph, launch = ctypes.c_void_p(), ctypes.c_void_p()
+    ok(hip.hipStreamBeginCapture(streams[0], 0))
+    run(0)
+    ok(hip.hipStreamEndCapture(streams[0], ctypes.byref(graph)))
+    ok(hip.hipGraphInstantiate(ctypes.byref(launch), graph, None, None, ctypes.c_size_t(0)))
+    for _ in range(3):
+        run(1)
+        ok(hip.hipGraphLaunch(launch, streams[0]))
+        run(2)
+        check()
+    ok(hip.hipGraphExecDestroy(launch))
+    ok(hip.hipGraphDestroy(graph))
+    plan.close()
+    for s in streams:
+        ok(hip.hipStreamDestroy(s))
