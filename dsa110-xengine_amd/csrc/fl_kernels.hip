@@ -39,13 +39,6 @@ constexpr int FL_NSEG = 32;    // the reference's threads per (beam, channel)
 constexpr int FL_TBIN = 128;   // ppspec bin
 constexpr double FL_MN = 48.0, FL_SIG = 6.0;
 constexpr int FL_RPW = 16;     // loads per wave in fl_flag_ts_kernel
-// Cache policy of the slab passes' buffer loads and stores: non-temporal where a
-// slab's rows are whole 128-byte lines (the statistics of 64 x 16384 x 1024 at
-// 256 channels: 0.195 -> 0.174 ms, with scaley 0.479 -> 0.468; 30 x 16384 x 640 at
-// 128: 64 -> 61 us), not where neighbouring slabs share them (12 x 8192 x 400 at
-// 32 channels: 16 us, 29 non-temporal).
-template <int W> constexpr int fl_policy() { return W >= 128 ? 2 : 0; }
-
 // (unsigned char)(__float2uint_rn(2 * val) / 2): round half to even, the
 // saturating conversion (NaN and negatives to 0), halve, keep the low byte.
 __device__ inline uint32_t fl_u8(float val) {
@@ -169,7 +162,7 @@ __device__ inline uint32_t fl_lut4(const uint8_t *lut, uint32_t x, uint32_t c) {
 // where the chip is full (the scaled read-only pass took 0.209 ms with 8 loads a
 // wave and 0.220 with 16; 0.186 with non-temporal loads since); with less to do
 // more loads a wave draw more.
-template <int W, bool SCALE, bool WRITE, bool WMAX>
+template <int W, bool NT, bool SCALE, bool WRITE, bool WMAX>
 __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
   constexpr int LPR = W / 4, RPI = 64 / LPR, TB = FL_TBIN / RPI, PF = W == 256 ? 8 : 16;
   static_assert(TB % PF == 0, "bins end on a prefetch block");
@@ -201,7 +194,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
   };
   uint32_t buf[PF];
 #pragma unroll
-  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(d), fl_policy<W>());
+  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(d), (NT ? 2 : 0));
   if constexpr (SCALE)
     fl_lut_build<W>(lut, lt, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, nullptr, 0, slab, a.nc);
   uint32_t S[4] = {0, 0, 0, 0}, Q[4] = {0, 0, 0, 0}, bs[4] = {0, 0, 0, 0};
@@ -218,7 +211,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
           // (every lane: cl + 3 < W keeps a non-live lane's lookups in the
           // table, and its statistics are never written)
           if (SCALE) x[r] = fl_lut4<W>(lut, x[r], (uint32_t)cl);
-          if (WRITE) __builtin_amdgcn_raw_buffer_store_b32(x[r], rout, vo, row(i0 + d + r), fl_policy<W>());
+          if (WRITE) __builtin_amdgcn_raw_buffer_store_b32(x[r], rout, vo, row(i0 + d + r), (NT ? 2 : 0));
           if (WMAX) {
             typedef unsigned short us2 __attribute__((ext_vector_type(2)));
             const uint32_t e = x[r] & 0x00FF00FFu, o = (x[r] >> 8) & 0x00FF00FFu;
@@ -240,7 +233,7 @@ __global__ __launch_bounds__(1024) void fl_stats_kernel(FlStats a) {
         // registers whose loads are still in flight
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          buf[d + r] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(i0 + PF + d + r), fl_policy<W>());
+          buf[d + r] = __builtin_amdgcn_raw_buffer_load_b32(rin, vo, row(i0 + PF + d + r), (NT ? 2 : 0));
         __builtin_amdgcn_sched_barrier(0);
       }
       if (((i0 - h * n1 + PF) & (TB - 1)) == 0) {          // end of a 128-sample bin
@@ -377,7 +370,7 @@ struct FlApply {
 // The pass leaves the block alone when the total power has jumped: the block is
 // then replaced by noise, and the host, which sums the spectrum in the
 // reference's order meanwhile, has the last word (force, or the noise).
-template <int W>
+template <int W, bool NT>
 __global__ __launch_bounds__(1024) void fl_apply_kernel(FlApply a) {
   constexpr int LPR = W / 4, RPI = 64 / LPR, PF = 16;
   __shared__ __attribute__((aligned(16))) uint8_t lut[256 * W];
@@ -407,7 +400,7 @@ __global__ __launch_bounds__(1024) void fl_apply_kernel(FlApply a) {
   auto row = [&](int i) { return (r0 + (uint32_t)(min(i, n - 1) * RPI)) * (uint32_t)a.nc; };
   uint32_t buf[PF];
 #pragma unroll
-  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(d), fl_policy<W>());
+  for (int d = 0; d < PF; d++) buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(d), (NT ? 2 : 0));
   fl_lut_build<W>(lut, lt, a.spec0 + (size_t)bm * a.nc, a.var0 + (size_t)bm * a.nc, a.mask + (size_t)bm * a.nc,
                   fl_rep(a.bpwr[bm]), slab, a.nc);
   uint16_t *part = a.part ? a.part + (size_t)item * a.nt : nullptr;
@@ -416,10 +409,10 @@ __global__ __launch_bounds__(1024) void fl_apply_kernel(FlApply a) {
 #pragma unroll
     for (int d = 0; d < PF; d++) {
       const uint32_t x = fl_lut4<W>(lut, buf[d], (uint32_t)cl);
-      __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, vo, row(i0 + d), fl_policy<W>());
+      __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, vo, row(i0 + d), (NT ? 2 : 0));
       rs[d] = __builtin_amdgcn_sad_u8(x, 0u, 0u);
       // (past the end this wave's last row again, into registers that are not used)
-      buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(i0 + PF + d), fl_policy<W>());
+      buf[d] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, row(i0 + PF + d), (NT ? 2 : 0));
       __builtin_amdgcn_sched_barrier(0);
     }
     if (part) {
@@ -941,24 +934,37 @@ static bool fl_shape_ok(int nb, int nt, int nc, const char *who) {
 // than half the CUs a workgroup.  Wide slabs read whole cache lines (64 x 16384
 // x 1024 scaley: 256, 128, 64 and 32 channels take 475, 498, 540 and 693 us),
 // but few workgroups cannot draw the bandwidth (12 x 8192 x 400: 105, 62, 37
-// and 31 us; 8 x 8192 x 1024: 118, 80, 64 and 54; 30 x 16384 x 640: 249, 160,
-// 214 and 271).
+// and 31 us; 8 x 8192 x 1024, where 64 channels give just half: 118, 80, 64 and 54;
+// 30 x 16384 x 640: 249, 160, 214 and 271; a step of 20 x 16384 x 400: 64 and 32
+// channels, 140 and 260 workgroups, 170 and 214).
 static int fl_slab_width(int nb, int nc) {
   int w = 256;
-  while (w > 32 && (long)nb * ((nc + w - 1) / w) < 144) w >>= 1;
+  while (w > 32 && (long)nb * ((nc + w - 1) / w) <= 128) w >>= 1;
   return w;
 }
 
-template <int W>
+// Whether the slab passes read and write the block non-temporally: where the rows
+// of slabs of 128 channels or more are whole 128-byte lines (64 x 16384 x 1008, the
+// scaley loop 1170 us and 1425 non-temporal) and the block is larger than the
+// Infinity Cache, from which the next pass reads a smaller one; a block that scaley
+// has written it reads in part from there up to about twice its size.  us of three
+// blocks in turn, without and with: steps 64 x 16384 x 1024 787 and 707, 24 x 12288 x
+// 896 (264 MB) 269 and 251, 49 x 4096 x 768 (154 MB) 182 and 175 but 154 and 176 one
+// at a time; loops 1209 and 1127, 206 and 271, 138 and 165.
+static bool fl_nontemporal(int nb, int nt, int nc, bool scaley) {
+  return nc % 128 == 0 && (long)nb * nt * nc > (scaley ? 500000000L : 250000000L);
+}
+
+template <int W, bool NT>
 static void fl_stats_launch(const FlStats &a, dim3 grid, dim3 block, hipStream_t s) {
   if (a.spec0 && !a.wdata) {
-    hipLaunchKernelGGL((fl_stats_kernel<W, true, false, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((fl_stats_kernel<W, NT, true, false, false>), grid, block, 0, s, a);
   } else if (a.wdata) {
-    if (a.mx) hipLaunchKernelGGL((fl_stats_kernel<W, true, true, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((fl_stats_kernel<W, true, true, false>), grid, block, 0, s, a);
+    if (a.mx) hipLaunchKernelGGL((fl_stats_kernel<W, NT, true, true, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((fl_stats_kernel<W, NT, true, true, false>), grid, block, 0, s, a);
   } else {
-    if (a.mx) hipLaunchKernelGGL((fl_stats_kernel<W, false, false, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((fl_stats_kernel<W, false, false, false>), grid, block, 0, s, a);
+    if (a.mx) hipLaunchKernelGGL((fl_stats_kernel<W, NT, false, false, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((fl_stats_kernel<W, NT, false, false, false>), grid, block, 0, s, a);
   }
 }
 
@@ -968,10 +974,13 @@ static int fl_stats_any(const FlStats &a, const char *who, void *stream) {
   const int items = a.nb * ((a.nc + w - 1) / w);
   const dim3 grid((items + 7) / 8 * 8), block(64 * FL_SW);
   hipStream_t s = (hipStream_t)stream;
-  if (w == 256) fl_stats_launch<256>(a, grid, block, s);
-  else if (w == 128) fl_stats_launch<128>(a, grid, block, s);
-  else if (w == 64) fl_stats_launch<64>(a, grid, block, s);
-  else fl_stats_launch<32>(a, grid, block, s);
+  const bool nt = fl_nontemporal(a.nb, a.nt, a.nc, a.wdata != NULL);
+  if (w == 256 && nt) fl_stats_launch<256, true>(a, grid, block, s);
+  else if (w == 256) fl_stats_launch<256, false>(a, grid, block, s);
+  else if (w == 128 && nt) fl_stats_launch<128, true>(a, grid, block, s);
+  else if (w == 128) fl_stats_launch<128, false>(a, grid, block, s);
+  else if (w == 64) fl_stats_launch<64, false>(a, grid, block, s);
+  else fl_stats_launch<32, false>(a, grid, block, s);
   return bfk_check(hipGetLastError(), "fl_stats_kernel");
 }
 
@@ -1041,10 +1050,15 @@ extern "C" int flk_apply(uint8_t *d_data, const float *d_spec0, const float *d_v
   const int items = nb * ((nc + w - 1) / w);
   const dim3 grid((items + 7) / 8 * 8), block(1024);
   hipStream_t s = (hipStream_t)stream;
-  if (w == 256) hipLaunchKernelGGL(fl_apply_kernel<256>, grid, block, 0, s, a);
-  else if (w == 128) hipLaunchKernelGGL(fl_apply_kernel<128>, grid, block, 0, s, a);
-  else if (w == 64) hipLaunchKernelGGL(fl_apply_kernel<64>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(fl_apply_kernel<32>, grid, block, 0, s, a);
+#define FL_APPLY(W, NT) hipLaunchKernelGGL((fl_apply_kernel<W, NT>), grid, block, 0, s, a)
+  const bool nontemporal = fl_nontemporal(nb, nt, nc, false);
+  if (w == 256 && nontemporal) FL_APPLY(256, true);
+  else if (w == 256) FL_APPLY(256, false);
+  else if (w == 128 && nontemporal) FL_APPLY(128, true);
+  else if (w == 128) FL_APPLY(128, false);
+  else if (w == 64) FL_APPLY(64, false);
+  else FL_APPLY(32, false);
+#undef FL_APPLY
   return bfk_check(hipGetLastError(), "fl_apply_kernel");
 }
 
