@@ -10,6 +10,8 @@
 // upper triangle into [baseline][channel][pol][re, im] (:366-457).
 //
 // Here:
+//   - Up to 64 antennas, where that is faster, one kernel reads the block itself
+//     (xc_fused_kernel below); else:
 //   - xc_turn_kernel turns the packed block, still one byte (4-bit re, 4-bit
 //     im) per sample, into (channel, pol) planes [channel*2 + pol][antenna]
 //     [sample]: each lane reads one channel's 4-byte words of 64 packets
@@ -314,6 +316,165 @@ __global__ __launch_bounds__(256) void xc_kernel(XcArgs a) {
   xc_share_of<NB, NS, 0, PD>(part, a, pq, ub, nunit, out, lane);
 }
 
+// Up to 64 antennas the correlation reads the block itself.  The samples of a
+// (channel, pol) may enter the sums in any order, so the words of four packets
+// become the operands' eight samples by byte permutes, with no turned copy of the
+// block: one workgroup takes CH channels (16 or 32 bytes of each packet and
+// antenna), a thread four packets of one antenna and four channels, and stages
+// [channel][four packets][antenna][pol][8 samples] in LDS, double-buffered per 32
+// packets with two more units in flight; a wave takes one (channel, pol) of 33 to 64
+// antennas or one channel of up to 32.  Workgroups that share 128-byte lines are
+// neighbours on one XCD.  64 antennas x 384 channels x 4096 samples with groups
+// outermost: 127 -> 51 us (201 MB, 3.9 TB/s), with antennas outermost 129 -> 91.  (Three
+// units in flight: the same, and scratch up to 32 antennas.)
+namespace {
+constexpr int XF = 512;                   // threads
+}  // namespace
+
+template <int NB, int CH>
+__global__ __launch_bounds__(XF, NB == 1 ? 4 : 2) void xc_fused_kernel(XcArgs a, int order) {
+  constexpr int NA = 32 * NB, NT = NB * (NB + 1) / 2, NPOL = CH / 4;   // pols of a wave
+  static_assert(NA * 8 * (CH / 4) == XF, "one staging task per thread and unit");
+  __shared__ uint4 lds[2][CH * 8 * NA];
+  const int P = blockIdx.x, nq = a.nchan / CH;
+  const int L = (P & 7) * (gridDim.x >> 3) + (P >> 3);
+  if (L >= nq * a.nslice) return;
+  const int c0 = L % nq * CH, slice = L / nq;
+  const int ntot = a.npkt / XUP;
+  const int ub = (int)((long)ntot * slice / a.nslice), nunit = (int)((long)ntot * (slice + 1) / a.nslice) - ub;
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // staging task: antenna ant, packets 4 wave .. + 3 of the unit, channels c0 + 4 half .. + 3
+  const int ant = CH == 4 ? lane : n, half = CH == 4 ? 0 : h;
+  const __amdgpu_buffer_rsrc_t rin = buffer_rsrc(a.in, a.in_bytes);
+  uint32_t off[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    off[k] = ant < a.nant ? (uint32_t)(chunk_offset(order, 4 * wave + k, ant, c0 >> 3, a.nant, a.nchan, a.nchan / 8) +
+                                       ((c0 & 7) + 4 * half) * 4)
+                          : 0x80000000u;
+  // (units past the slice read at offset in_bytes and up, which the buffer's range
+  // check answers with zeros)
+  auto load = [&](int u, u4v (&r)[4]) __attribute__((always_inline)) {
+    const uint32_t so = (uint32_t)__builtin_amdgcn_readfirstlane(
+        u < nunit ? (int)((long)(ub + u) * XUP * a.nant * a.nchan * 4) : (int)a.in_bytes);
+#pragma unroll
+    for (int k = 0; k < 4; k++) r[k] = __builtin_amdgcn_raw_buffer_load_b128(rin, off[k], so, 0);
+  };
+  auto store = [&](uint4 *st, const u4v (&r)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      st[((4 * half + c) * 8 + wave) * NA + ant] =
+          make_uint4(__builtin_amdgcn_perm(r[1][c], r[0][c], 0x06040200u), __builtin_amdgcn_perm(r[3][c], r[2][c], 0x06040200u),
+                     __builtin_amdgcn_perm(r[1][c], r[0][c], 0x07050301u), __builtin_amdgcn_perm(r[3][c], r[2][c], 0x07050301u));
+  };
+
+  const int cw = NPOL == 1 ? wave >> 1 : wave, q0 = NPOL == 1 ? wave & 1 : 0;   // this wave's channel and first pol
+  i16v accr[NPOL][NT], acci[NPOL][NT];
+  uint32_t sr[NPOL][NB], si[NPOL][NB];
+#pragma unroll
+  for (int q = 0; q < NPOL; q++) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) { accr[q][t] = (i16v){}; acci[q][t] = (i16v){}; }
+#pragma unroll
+    for (int b = 0; b < NB; b++) sr[q][b] = si[q][b] = 0;
+  }
+  auto compute = [&](const uint4 *st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+#pragma unroll
+      for (int q = 0; q < NPOL; q++) {
+        i4v X[NB], W[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+          const uint2 r = ((const uint2 *)(st + (cw * 8 + 2 * s + h) * NA + 32 * b + n))[q0 + q];
+          const uint32_t y0 = r.x ^ 0x88888888u, y1 = r.y ^ 0x88888888u;
+          const uint32_t ur0 = y0 & 0x0F0F0F0Fu, ur1 = y1 & 0x0F0F0F0Fu;
+          const uint32_t ui0 = (y0 >> 4) & 0x0F0F0F0Fu, ui1 = (y1 >> 4) & 0x0F0F0F0Fu;
+          sr[q][b] = __builtin_amdgcn_sad_u8(ur1, 0u, __builtin_amdgcn_sad_u8(ur0, 0u, sr[q][b]));
+          si[q][b] = __builtin_amdgcn_sad_u8(ui1, 0u, __builtin_amdgcn_sad_u8(ui0, 0u, si[q][b]));
+          X[b] = (i4v){(int)ur0, (int)ur1, (int)ui0, (int)ui1};
+          const uint32_t nr0 = (0x80808080u - ur0) ^ 0x80808080u, nr1 = (0x80808080u - ur1) ^ 0x80808080u;
+          W[b] = (i4v){(int)ui0, (int)ui1, (int)nr0, (int)nr1};
+        }
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          const int J = tile_j<NB>(t), I = tile_i<NB>(t);
+          accr[q][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(X[J], X[I], accr[q][t], 0, 0, 0);
+          acci[q][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(X[J], W[I], acci[q][t], 0, 0, 0);
+        }
+      }
+    }
+  };
+
+  u4v ra[4], rb[4];                         // units u + 1 and u + 2, in flight while unit u is computed
+  load(0, ra);
+  load(1, rb);
+  store(lds[0], ra);
+  load(2, ra);
+  __syncthreads();
+#pragma unroll 1
+  for (int u = 0; u < nunit; u += 2) {
+    store(lds[1], rb);
+    load(u + 3, rb);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(lds[0]);
+    __syncthreads();
+    if (u + 1 >= nunit) break;
+    store(lds[0], ra);
+    load(u + 4, ra);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(lds[1]);
+    __syncthreads();
+  }
+
+  // The sums leave by way of LDS, eight rows of a tile at a time, so that the CH
+  // channels' visibilities of a baseline (64 or 128 bytes) are written together; a
+  // pitch of one entry more than a baseline has spreads them over the banks.
+  constexpr int E8 = 2 * CH, PITCH = E8 + 1, NBUF = CH == 4 ? 2 : 1;
+  static_assert(NBUF * 256 * PITCH * sizeof(float2) <= sizeof(lds), "the rows in transit");
+  float2 *vis = (float2 *)(a.out + slice * a.slice_floats);
+  const int N128 = 128 * nunit * XU;
+  int S[NPOL][NB], E[NPOL][NB];
+#pragma unroll
+  for (int q = 0; q < NPOL; q++)
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      const int s0 = (int)(sr[q][b] + si[q][b]), e0 = (int)sr[q][b] - (int)si[q][b];
+      S[q][b] = s0 + __shfl_xor(s0, 32, 64);
+      E[q][b] = e0 + __shfl_xor(e0, 32, 64);
+    }
+  int turn = 0;
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    const int J = tile_j<NB>(t), I = tile_i<NB>(t);
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      if (32 * J + 8 * m >= a.nant || 32 * I >= a.nant) continue;
+      float2 *buf = (float2 *)lds + (NBUF == 2 ? (turn++ & 1) : 0) * 256 * PITCH;
+#pragma unroll
+      for (int q = 0; q < NPOL; q++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+          const int v = 4 * m + x, row = 4 * h + x, jl = 8 * m + row;
+          const int Sj = __shfl(S[q][J], jl, 64), Ej = __shfl(E[q][J], jl, 64);
+          const int re = accr[q][t][v] - 8 * Sj - 8 * S[q][I] + N128;
+          const int im = acci[q][t][v] - 8 * Ej + 8 * E[q][I];
+          buf[(row * 32 + n) * PITCH + cw * 2 + q0 + q] = make_float2((float)re, (float)im);
+        }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 256 * E8 / XF; k++) {
+        const int e = tid + k * XF, i = 32 * I + (e / E8) % 32, j = 32 * J + 8 * m + e / E8 / 32;
+        if (i < a.nant && j <= i)
+          vis[((long)i * (i + 1) / 2 + j) * a.nchan * 2 + c0 * 2 + e % E8] = buf[(e / E8) * PITCH + e % E8];
+      }
+      if (NBUF == 1) __syncthreads();
+    }
+  }
+}
+
 extern "C" size_t bfk_xcorr_vis_bytes(int nant, int nchan) {
   return (size_t)nant * (nant + 1) / 2 * nchan * 2 * 2 * sizeof(float);
 }
@@ -347,9 +508,32 @@ extern "C" size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice) {
   return nslice > 1 ? (size_t)nslice * bfk_xcorr_vis_bytes(nant, nchan) : 0;
 }
 
-// d_turn: the input's size; d_part: bfk_xcorr_part_bytes (nslice > 1).
+// d_turn: the input's size; d_part: bfk_xcorr_part_bytes of nslice, or of nfused where
+// that (bfk_xcorr_fused_slices) is given and the fused kernel runs.
+// Time slices of the fused kernel, 0 where it does not run: above 64 antennas, with
+// sums that FP32 may not hold, and where the turned copy is faster.  us alone and
+// among others, turned and fused: up to 32 antennas always (32 x 384 x 4096 52/54
+// and 34/34; 10 x 64 x 1024 11.0/9.6 and 11.4/6.8; 20 x 16 x 128 7.8/6.5 and
+// 7.6/3.7).  Up to 64 with antennas outermost a thread's 16 bytes cost a 128-byte
+// line through the L1, so only blocks of some size gain (64 x 384 x 4096 124/129 and
+// 87/91, 45 x 96 x 4096 (35 MB) 33/21 and 28/21, 64 x 128 x 1024 (17 MB) 24/16 and
+// 29/13), with groups outermost smaller ones too (64 x 384 x 4096 125/127 and 57/51,
+// 63 x 48 x 2048 (12 MB) 21/12 and 24/8.6, 64 x 24 x 2048 18/9.5 and 21/8.0), and the
+// shortest, which its one launch bounds (60 x 16 x 128 9.9/6.6 and 12/4.3).  Slices
+// fill the CUs while each has 128 (256 above 32 antennas) packets: 64 x 384 x 512
+// in one 30/13, in two 30/19; 16 x 384 x 1024 in one, two and four 21/9, 16/7, 13/7.
+extern "C" int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order) {
+  if (nant > 64 || npkt > 65536) return 0;
+  const long bytes = (long)npkt * nant * nchan * 4;
+  if (nant > 32 && npkt > 64 && bytes < (order == 0 ? 32000000 : 10000000)) return 0;
+  const int wgs = nchan / (nant <= 32 ? 8 : 4), most = npkt / (nant <= 32 ? 128 : 256);
+  int s = wgs >= 192 ? 1 : 256 / wgs;
+  if (s > most) s = most;
+  return s < 1 ? 1 : s;
+}
+
 extern "C" int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t *d_in, uint8_t *d_turn,
-                         float *d_part, int nslice, float *d_vis, void *stream) {
+                         float *d_part, int nslice, int nfused, float *d_vis, void *stream) {
   if (nant < 1 || nant > 96 || nchan < 8 || nchan % 8 || npkt < XUP || npkt % XUP || order < 0 || order > 1) {
     bfk_set_error("bfk_xcorr: unsupported shape nant=%d nchan=%d npkt=%d order=%d", nant, nchan, npkt, order);
     return -1;
@@ -358,12 +542,36 @@ extern "C" int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t
     bfk_set_error("bfk_xcorr: block above 2 GiB");
     return -1;
   }
+  if (nfused && (nfused != bfk_xcorr_fused_slices(nant, nchan, npkt, order) || (nfused > 1 && !d_part))) {
+    bfk_set_error("bfk_xcorr: %d slices of the fused kernel (partials %p)", nfused, (void *)d_part);
+    return -1;
+  }
   if (nslice < 1 || nslice > npkt / XUP || (nslice > 1 && !d_part) || !d_turn) {
     bfk_set_error("bfk_xcorr: %d slices of %d units (partials %p)", nslice, npkt / XUP, (void *)d_part);
     return -1;
   }
   hipStream_t s = (hipStream_t)stream;
   const uint32_t in_bytes = (uint32_t)((size_t)npkt * nant * nchan * 4);
+  const long n4 = (long)(bfk_xcorr_vis_bytes(nant, nchan) / sizeof(float4));
+  if (nfused) {
+    XcArgs a;
+    a.in = d_in;
+    a.out = nfused > 1 ? d_part : d_vis;
+    a.nant = nant;
+    a.nchan = nchan;
+    a.npkt = npkt;
+    a.nslice = nfused;
+    a.in_bytes = in_bytes;
+    a.slice_floats = 4 * n4;
+    const int ch = nant <= 32 ? 8 : 4;
+    const dim3 grid((unsigned)((nchan / ch * nfused + 7) / 8 * 8));
+    if (ch == 8) hipLaunchKernelGGL((xc_fused_kernel<1, 8>), grid, dim3(XF), 0, s, a, order);
+    else hipLaunchKernelGGL((xc_fused_kernel<2, 4>), grid, dim3(XF), 0, s, a, order);
+    if (nfused > 1)
+      hipLaunchKernelGGL(xc_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, (const float4 *)d_part,
+                         (float4 *)d_vis, n4, nfused);
+    return bfk_check(hipGetLastError(), "xc_fused_kernel");
+  }
   const long nturn = (long)(npkt / XUP) * ((nchan + TCH - 1) / TCH) * ((nant + TA16 - 1) / TA16);
   hipLaunchKernelGGL(xc_turn_kernel, dim3((unsigned)nturn), dim3(256), 0, s, d_in, d_turn, nant, nchan, npkt, order,
                      in_bytes);
@@ -389,7 +597,6 @@ extern "C" int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t
   else if (nant <= 64) hipLaunchKernelGGL((xc_kernel<2, 2, XPD>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((xc_kernel<3, 2, XPD>), grid, block, 0, s, a);
   if (nslice > 1) {
-    const long n4 = a.slice_floats / 4;
     hipLaunchKernelGGL(xc_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s,
                        (const float4 *)d_part, (float4 *)d_vis, n4, nslice);
   }

@@ -5,7 +5,8 @@
  * (dsaX_bfCorr.cu:472-569: copy, reorder, four batched GEMMs, two reorder
  * kernels, with cudaMalloc/cublasCreate per call) by a turn of the packed
  * block into (channel, pol) planes, one correlation launch over time slices
- * and the sum of the slices, on device buffers the plan owns.
+ * and the sum of the slices, on device buffers the plan owns; or, up to 64
+ * antennas, by a correlation launch that reads the block itself.
  */
 #include <hip/hip_runtime_api.h>
 #include <stdlib.h>
@@ -18,11 +19,13 @@
 size_t bfk_xcorr_vis_bytes(int nant, int nchan);
 size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice);
 int bfk_xcorr_default_slices(int nchan, int npkt);
+int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order);
 int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t *d_in, uint8_t *d_turn, float *d_part,
-              int nslice, float *d_vis, void *stream);
+              int nslice, int nfused, float *d_vis, void *stream);
 
 struct dsaxbf_xengine {
   int nant, nchan, npkt, order, device, nslice;
+  int nfused;           /* slices of the kernel that reads the block itself; 0: it does not run */
   hipStream_t stream;
   uint8_t *d_in, *d_turn;
   float *d_vis, *d_part;
@@ -30,6 +33,10 @@ struct dsaxbf_xengine {
 
 size_t dsaxbf_xengine_vis_bytes(int nant, int nchan) {
   return nant < 1 || nchan < 1 ? 0 : bfk_xcorr_vis_bytes(nant, nchan);
+}
+
+static size_t part_bytes(const dsaxbf_xengine *x, int nslice, int nfused) {
+  return bfk_xcorr_part_bytes(x->nant, x->nchan, nslice > nfused ? nslice : nfused);
 }
 
 void dsaxbf_xengine_destroy(dsaxbf_xengine *x) {
@@ -66,7 +73,8 @@ int dsaxbf_xengine_create(dsaxbf_xengine **out, int nant, int nchan, int npkt, i
   x->order = input_order;
   x->device = device;
   x->nslice = bfk_xcorr_default_slices(nchan, npkt);
-  const size_t nin = (size_t)npkt * nant * nchan * 4, npart = bfk_xcorr_part_bytes(nant, nchan, x->nslice);
+  x->nfused = bfk_xcorr_fused_slices(nant, nchan, npkt, input_order);
+  const size_t nin = (size_t)npkt * nant * nchan * 4, npart = part_bytes(x, x->nslice, x->nfused);
   hipError_t e = hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void **)&x->d_in, nin);
   if (e == hipSuccess) e = hipMalloc((void **)&x->d_turn, nin);
@@ -84,7 +92,7 @@ void *dsaxbf_xengine_stream(dsaxbf_xengine *x) { return x ? (void *)x->stream : 
 
 int dsaxbf_xengine_execute(dsaxbf_xengine *x, const uint8_t *d_in, float *d_vis, void *stream) {
   if (!x || !d_in || !d_vis) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
-  int rc = bfk_xcorr(x->nant, x->nchan, x->npkt, x->order, d_in, x->d_turn, x->d_part, x->nslice, d_vis,
+  int rc = bfk_xcorr(x->nant, x->nchan, x->npkt, x->order, d_in, x->d_turn, x->d_part, x->nslice, x->nfused, d_vis,
                      stream ? stream : (void *)x->stream);
   return rc ? dsaxbf_fail(rc, "%s", bfk_last_error()) : DSAXBF_OK;
 }
@@ -92,6 +100,8 @@ int dsaxbf_xengine_execute(dsaxbf_xengine *x, const uint8_t *d_in, float *d_vis,
 int dsaxbf_xengine_set_slices(dsaxbf_xengine *x, int nslice) {
   dsaxbf_clear_error();
   if (!x) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
+  /* (a number of slices asks for the turned copy and those slices) */
+  const int nfused = nslice ? 0 : bfk_xcorr_fused_slices(x->nant, x->nchan, x->npkt, x->order);
   if (nslice == 0) nslice = bfk_xcorr_default_slices(x->nchan, x->npkt);
   if (nslice < 1 || nslice > x->npkt / 32)
     return dsaxbf_fail(DSAXBF_EINVAL, "nslice=%d outside 1..%d", nslice, x->npkt / 32);
@@ -99,12 +109,13 @@ int dsaxbf_xengine_set_slices(dsaxbf_xengine *x, int nslice) {
   hipError_t e = hipStreamSynchronize(x->stream);
   if (e != hipSuccess) return dsaxbf_fail(DSAXBF_EHIP, "correlator stream: %s", hipGetErrorString(e));
   float *part = NULL;
-  const size_t npart = bfk_xcorr_part_bytes(x->nant, x->nchan, nslice);
+  const size_t npart = part_bytes(x, nslice, nfused);
   if (npart && hipMalloc((void **)&part, npart) != hipSuccess)
     return dsaxbf_fail(DSAXBF_ENOMEM, "partial visibilities (%zu bytes)", npart);
   hipFree(x->d_part);
   x->d_part = part;
   x->nslice = nslice;
+  x->nfused = nfused;
   return DSAXBF_OK;
 }
 

@@ -397,7 +397,8 @@ void *dsaxbf_xengine_stream(dsaxbf_xengine *x);   /* the plan's hipStream_t */
  * block turned into (channel, pol) planes of 64-sample units (plan-owned, the
  * input's size), the correlation over time slices, and the sum of the
  * slices' partial visibilities (plan-owned) when there is more than one
- * slice. */
+ * slice.  Up to 64 antennas, unless slices are set, the correlation may read
+ * the block itself instead, in slices of its own. */
 int dsaxbf_xengine_execute(dsaxbf_xengine *x, const uint8_t *d_in, float *d_vis,
                            void *stream);
 /* Time slices the correlation runs in (1 .. npkt/32; 0 = the library's

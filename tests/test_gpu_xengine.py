@@ -115,3 +115,26 @@ def test_xengine_rejects_bad_shapes(bf):
         with pytest.raises(bf.BeamformerError):
             x.slices = n
     x.close()
+
+
+@pytest.mark.parametrize("nant,nchan,npkt,order", [
+    (1, 8, 128, 0), (17, 24, 1056, 1), (32, 40, 640, 0), (8, 520, 96, 1), (33, 24, 64, 0), (64, 8, 32, 1),
+    (64, 72, 2016, 0), (45, 96, 2080, 0), (64, 48, 864, 1), (50, 104, 2048, 1)])
+def test_xengine_reads_the_block_itself(bf, orc, nant, nchan, npkt, order):
+    """The correlation that reads the untransposed block (up to 32 antennas, short
+    and large blocks to 64), in one and several slices of even and odd numbers of
+    units: the turned path's visibilities (a plan with slices set) bit for bit,
+    the oracle's on the first group, and each block its own after another."""
+    cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=8, input_order=order)
+    assert bf.lib.bfk_xcorr_fused_slices(nant, nchan, npkt, order)
+    plans = [bf.XEngine(nant, nchan, npkt, order) for _ in range(2)]
+    plans[1].slices = plans[1].slices
+    for seed in (1, 2):
+        block = np.random.default_rng(seed).integers(0, 256, bf.input_bytes(cfg), dtype=np.uint8)
+        vis = [x.process_block(block) for x in plans]
+        assert np.array_equal(vis[0], vis[1])
+    shape = (npkt, nant, nchan // 8, 32) if order == 0 else (npkt, nchan // 8, nant, 32)
+    group = np.ascontiguousarray(block.reshape(shape)[(slice(None),) * (2 - order) + (0,)])
+    assert np.array_equal(vis[0][:, :8], orc.xcorr(nant, 8, npkt, group.ravel(), 0))
+    for x in plans:
+        x.close()
