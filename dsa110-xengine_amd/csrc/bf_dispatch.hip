@@ -119,7 +119,12 @@ static TileCost variant_cost(const bfk_dims *d) {
                                          {{36, 50, 54}, {28, 43, 44}, {22, 34, 35}, {26, 42, 46}}};
   static const TileTimes half[3] = {{22, 42, 37}, {48, 87, 70}, {133, 256, 185}};      // 128 beams
   static const TileTimes quarter[3] = {{17, 33, 26}, {35, 67, 45}, {106, 222, 137}};   // 64 beams
-  const TileTimes &t = beams == 256 ? shared[group][d->prec] : beams == 128 ? half[k] : quarter[k];
+  TileTimes t = beams == 256 ? shared[group][d->prec] : beams == 128 ? half[k] : quarter[k];
+  if (beams == 256 && d->nbeam <= 128) {            // one beam tile a wave (64 x 384 x 2048 -> 100, FP6: 112 -> 85)
+    t.t1 *= 0.7f;
+    t.t2 *= 0.7f;
+    t.per512 *= 0.7f;
+  }
   const float steady = (float)n * t.per512 / 512;
   const float alone = n <= 256   ? t.t1
                       : n <= 512 ? beams == 256 ? t.t2 : fminf(t.t2, t.t1 + (t.t2 - t.t1) * (float)(n - 256) / 192)

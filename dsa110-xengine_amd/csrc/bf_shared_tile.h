@@ -136,12 +136,12 @@ __device__ __forceinline__ void det_final(const float (&sd)[NP][4], float sc, fl
 // scalar: no 64-bit address arithmetic per load.
 // (For FP16 this block order measured faster than the deferred-detect chains
 // that FP8 uses: those need A_im derived once per beam tile.)
-template <bool PF>
-__device__ __forceinline__ void unit16(Acc<BTW> &A, WFrag<0, BTW, 1> &W, const uint8_t *unit, int lane,
+template <bool PF, int NB>
+__device__ __forceinline__ void unit16(Acc<NB> &A, WFrag<0, NB, 1> &W, const uint8_t *unit, int lane,
                                        const WSrc &src, uint32_t wnext) {
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-  for (int bt = 0; bt < BTW; bt++) { A.r[bt] = (f16v){}; A.i[bt] = (f16v){}; }
+  for (int bt = 0; bt < NB; bt++) { A.r[bt] = (f16v){}; A.i[bt] = (f16v){}; }
 #pragma unroll
   for (int s = 0; s < 8; s++) {
     const uint4 r = *(const uint4 *)(unit + (s * 64 + lane) * 16);
@@ -149,14 +149,14 @@ __device__ __forceinline__ void unit16(Acc<BTW> &A, WFrag<0, BTW, 1> &W, const u
     const uint4 m = make_uint4(r.y ^ 0x80008000u, r.x, r.w ^ 0x80008000u, r.z);
     const h8v are = __builtin_bit_cast(h8v, r), aim = __builtin_bit_cast(h8v, m);
 #pragma unroll
-    for (int bt = 0; bt < BTW; bt++) {
+    for (int bt = 0; bt < NB; bt++) {
       A.r[bt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(are, W.w[bt][0][s], A.r[bt], 0, 0, 0);
       A.i[bt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aim, W.w[bt][0][s], A.i[bt], 0, 0, 0);
     }
     if constexpr (PF) {
       __builtin_amdgcn_sched_barrier(0x386);
 #pragma unroll
-      for (int bt = 0; bt < BTW; bt++) W.load_one_rb(src, wnext, bt, s);
+      for (int bt = 0; bt < NB; bt++) W.load_one_rb(src, wnext, bt, s);
       __builtin_amdgcn_sched_barrier(0x386);
     }
   }
@@ -172,8 +172,8 @@ __device__ __forceinline__ void unit16(Acc<BTW> &A, WFrag<0, BTW, 1> &W, const u
 // of detect1).  With PF, each K step of W[BT] is reloaded from row wnext
 // right after its last MFMA (the rolling prefetch of unit16).  Scheduling
 // barriers keep this interleave as written.
-template <int PREC, int BT, bool PF, int NP>
-__device__ __forceinline__ void chain8(f16v &cr, f16v &ci, WFrag<PREC, BTW, 1> &W, const i8v (&are)[2],
+template <int PREC, int BT, bool PF, int NP, int NB>
+__device__ __forceinline__ void chain8(f16v &cr, f16v &ci, WFrag<PREC, NB, 1> &W, const i8v (&are)[2],
                                        const i8v (&aim)[2], const WSrc &src, uint32_t wnext,
                                        const Pending &pd, float (&into)[NP]) {
   constexpr int NPART = PREC == 3 ? 3 : 2;
@@ -211,10 +211,10 @@ __device__ __forceinline__ void chain8(f16v &cr, f16v &ci, WFrag<PREC, BTW, 1> &
   det_final<NP>(sd, pd.sc, into);
 }
 
-// One FP8 or FP6 unit, both beam tiles: chain 0 detects the pending chain
+// One FP8 or FP6 unit, both beam tiles (or the only one): chain 0 detects the pending chain
 // into into0, chain 1 detects chain 0 into into1, and chain 1 is left pending.
-template <int PREC, bool PF, int NP>
-__device__ __forceinline__ void unit8(Pending &pd, WFrag<PREC, BTW, 1> &W, const uint8_t *unit, int lane,
+template <int PREC, bool PF, int NP, int NB>
+__device__ __forceinline__ void unit8(Pending &pd, WFrag<PREC, NB, 1> &W, const uint8_t *unit, int lane,
                                       const WSrc &src, uint32_t wnext, float (&into0)[NP], float (&into1)[NP]) {
   f16v cr, ci;
   __builtin_amdgcn_s_setprio(1);
@@ -236,9 +236,11 @@ __device__ __forceinline__ void unit8(Pending &pd, WFrag<PREC, BTW, 1> &W, const
   }
   chain8<PREC, 0, PF, NP>(cr, ci, W, are, aim, src, wnext, pd, into0);
   pd.r = cr; pd.i = ci; pd.sc = W.sc[0];
-  chain8<PREC, 1, PF, NP>(cr, ci, W, are, aim, src, wnext, pd, into1);
+  if constexpr (NB == 2) {
+    chain8<PREC, 1, PF, NP>(cr, ci, W, are, aim, src, wnext, pd, into1);
+    pd.r = cr; pd.i = ci; pd.sc = W.sc[1];
+  }
   __builtin_amdgcn_s_setprio(0);
-  pd.r = cr; pd.i = ci; pd.sc = W.sc[1];
 }
 
 template <int PREC> constexpr int abuf_bytes() { return PREC == 0 ? AB16 : 2 * AB8; }   // double buffers
@@ -255,12 +257,11 @@ static_assert(2 * 4096 <= AB8, "FP6 operands of one (channel, pol) fit the FP8 h
 //      pol 1), so one row is held at a time and the second is loaded in place
 //      once, during step 7's second unit, with the rolling path's registers.
 //      The powers are summed in another order than the rolling path's.
-template <int PREC, int TAVG, int GROUP = 0>
-__device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *stage, uint8_t *abuf) {
+template <int PREC, int TAVG, int GROUP, int NB>
+__device__ __forceinline__ void shared_tile_of(const BfArgs &a, const TileId &t, uint8_t *stage, uint8_t *abuf) {
   static_assert(GROUP != 1 || PREC == 1 || PREC == 2, "FP16 and three-part FP6 cannot hold both rows");
   constexpr int UNIT = PREC == 0 ? AB16 / 2 : AB8 / 2;    // operand bytes per unit
   constexpr int NP = TAVG <= 32 ? 32 / TAVG : 1;
-  const TileId t = tile_id(a, L);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: weight rows stay scalar
@@ -270,14 +271,15 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
   src.vl = (uint32_t)lane * (PREC == 0 ? 16u : 32u);
   src.vn4 = (uint32_t)(lane & 31) * 4u;
   const int n = lane & 31, h = lane >> 5;
-  const int btw = (t.bset * NW + wave) * BTW;
+  const int btw = t.bset * NW * BTW + wave * NB;
+  const bool live = NB == 2 || btw * 32 < a.nbeam;   // (a wave without beams only stages and unpacks)
 
   // Weights of (channel, pol) 0 are loaded right after the staging loads:
   // their latency overlaps the staging, and the stage stores (which wait for
   // every older load) do not wait for them.  The second unit of each (channel,
   // pol) prefetches the next one's in place (the last one reloads itself).
-  WFrag<PREC, BTW, 1> W;
-  WFrag<PREC, BTW, 1> W1;                 // pol 1's weights (GROUP 1)
+  WFrag<PREC, NB, 1> W;
+  WFrag<PREC, NB, 1> W1;                 // pol 1's weights (GROUP 1)
 
   // (a) stage: the two (packet, antenna quad) tasks of each thread, every
   // load issued before the first store.  Buffer loads without branches: a
@@ -323,11 +325,11 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
   }
   __syncthreads();
 
-  float part[2][BTW][NP];
+  float part[2][NB][NP];
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int bt = 0; bt < BTW; bt++)
+    for (int bt = 0; bt < NB; bt++)
 #pragma unroll
       for (int j = 0; j < NP; j++) part[i][bt][j] = 0.f;
 
@@ -344,15 +346,19 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
     auto cqof = [](int k) { return 2 * (k & 7) + (k >> 3); };
     auto step = [&](int k, auto prefetch) {
       const int cq = cqof(k);
-      Acc<BTW> A;
+      Acc<NB> A;
       unpack_unit_f16(stage, abuf + UNIT, 2 * cq + 1, tid);
-      unit16<false>(A, W, abuf, lane, src, 0);
-      detect<TAVG>(A, W.sc, part[0]);
+      if (live) {
+        unit16<false>(A, W, abuf, lane, src, 0);
+        detect<TAVG>(A, W.sc, part[0]);
+      }
       __syncthreads();
       if (k < 15) unpack_unit_f16(stage, abuf, 2 * cqof(k + 1), tid);
-      unit16<decltype(prefetch)::value>(A, W, abuf + UNIT, lane, src, w1 * a.nbt + btw);
-      detect<TAVG>(A, W.sc, part[1]);
-      if constexpr (decltype(prefetch)::value) W.load_scale_rb(src, w1 * a.nbeam_pad + btw * 32);
+      if (live) {
+        unit16<decltype(prefetch)::value>(A, W, abuf + UNIT, lane, src, w1 * a.nbt + btw);
+        detect<TAVG>(A, W.sc, part[1]);
+        if constexpr (decltype(prefetch)::value) W.load_scale_rb(src, w1 * a.nbeam_pad + btw * 32);
+      }
       __syncthreads();
     };
     unpack_unit_f16(stage, abuf, 0, tid);
@@ -367,15 +373,19 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
     __syncthreads();
     for (int cq = 0; cq < 16; cq++) {
       const uint32_t wn = weight_row(a, t.g, cq < 15 ? cq + 1 : cq);
-      Acc<BTW> A;
+      Acc<NB> A;
       unpack_unit_f16(stage, abuf + UNIT, 2 * cq + 1, tid);
-      unit16<false>(A, W, abuf, lane, src, 0);
-      detect<TAVG>(A, W.sc, part[0]);
+      if (live) {
+        unit16<false>(A, W, abuf, lane, src, 0);
+        detect<TAVG>(A, W.sc, part[0]);
+      }
       __syncthreads();
       if (cq < 15) unpack_unit_f16(stage, abuf, 2 * cq + 2, tid);
-      unit16<true>(A, W, abuf + UNIT, lane, src, wn * a.nbt + btw);
-      detect<TAVG>(A, W.sc, part[1]);
-      W.load_scale_rb(src, wn * a.nbeam_pad + btw * 32);
+      if (live) {
+        unit16<true>(A, W, abuf + UNIT, lane, src, wn * a.nbt + btw);
+        detect<TAVG>(A, W.sc, part[1]);
+        W.load_scale_rb(src, wn * a.nbeam_pad + btw * 32);
+      }
       __syncthreads();
     }
   } else {
@@ -393,11 +403,13 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
     unpack_cq(abuf, 0);
     __syncthreads();
     if constexpr (GROUP == 1) {
-      auto step = [&](int cq, WFrag<PREC, BTW, 1> &Wc) {
+      auto step = [&](int cq, WFrag<PREC, NB, 1> &Wc) {
         if (cq < 15) unpack_cq(abuf + ((cq + 1) & 1) * AB8, cq + 1);
         const uint8_t *ab = abuf + (cq & 1) * AB8;
-        unit8<PREC, false, NP>(pd, Wc, ab, lane, src, 0, part[1][1], part[0][0]);
-        unit8<PREC, false, NP>(pd, Wc, ab + UNIT, lane, src, 0, part[0][1], part[1][0]);
+        if (live) {
+          unit8<PREC, false, NP>(pd, Wc, ab, lane, src, 0, part[1][NB - 1], part[0][0]);
+          unit8<PREC, false, NP>(pd, Wc, ab + UNIT, lane, src, 0, part[0][NB - 1], part[1][0]);
+        }
         __syncthreads();
       };
       for (int cq = 0; cq < 16; cq += 2) {
@@ -411,10 +423,12 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
       auto step = [&](int k, auto prefetch) {
         if (k < 15) unpack_cq(abuf + ((k + 1) & 1) * AB8, 2 * ((k + 1) & 7) + ((k + 1) >> 3));
         const uint8_t *ab = abuf + (k & 1) * AB8;
-        unit8<PREC, false, NP>(pd, W, ab, lane, src, 0, part[1][1], part[0][0]);
-        unit8<PREC, decltype(prefetch)::value, NP>(pd, W, ab + UNIT, lane, src, w1 * a.nbt + btw, part[0][1],
-                                                   part[1][0]);
-        if constexpr (decltype(prefetch)::value) W.load_scale_rb(src, w1 * a.nbeam_pad + btw * 32);
+        if (live) {
+          unit8<PREC, false, NP>(pd, W, ab, lane, src, 0, part[1][NB - 1], part[0][0]);
+          unit8<PREC, decltype(prefetch)::value, NP>(pd, W, ab + UNIT, lane, src, w1 * a.nbt + btw, part[0][NB - 1],
+                                                     part[1][0]);
+          if constexpr (decltype(prefetch)::value) W.load_scale_rb(src, w1 * a.nbeam_pad + btw * 32);
+        }
         __syncthreads();
       };
 #pragma unroll 1
@@ -427,9 +441,11 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
         const uint32_t wn = weight_row(a, t.g, cq < 15 ? cq + 1 : cq);
         if (cq < 15) unpack_cq(abuf + ((cq + 1) & 1) * AB8, cq + 1);
         const uint8_t *ab = abuf + (cq & 1) * AB8;
-        unit8<PREC, false, NP>(pd, W, ab, lane, src, 0, part[1][1], part[0][0]);
-        unit8<PREC, true, NP>(pd, W, ab + UNIT, lane, src, wn * a.nbt + btw, part[0][1], part[1][0]);
-        W.load_scale_rb(src, wn * a.nbeam_pad + btw * 32);
+        if (live) {
+          unit8<PREC, false, NP>(pd, W, ab, lane, src, 0, part[1][NB - 1], part[0][0]);
+          unit8<PREC, true, NP>(pd, W, ab + UNIT, lane, src, wn * a.nbt + btw, part[0][NB - 1], part[1][0]);
+          W.load_scale_rb(src, wn * a.nbeam_pad + btw * 32);
+        }
         __syncthreads();
       }
     }
@@ -438,11 +454,27 @@ __device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *sta
     for (int j = 0; j < NP; j++) sd[j][0] = sd[j][1] = sd[j][2] = sd[j][3] = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; v++) det_elem<NP>(pd, v, sd);
-    det_final<NP>(sd, pd.sc, part[1][1]);
+    det_final<NP>(sd, pd.sc, part[1][NB - 1]);
   }
 
   // (c)
-  tile_output<TAVG>(a, t, btw, n, h, part, 0, 2);
+  if (live) tile_output<TAVG>(a, t, btw, n, h, part, 0, 2);
+}
+
+// A set of at most four beam tiles takes one a wave (waves without beams only stage
+// and unpack), else two: with two, half the waves of 128 beams or fewer multiplied
+// zeros.  us alone and among other blocks, 64 antennas x 384 channels x 2048 samples,
+// fine weights: 100 beams in FP6 112/144 and 85/93, in three-part FP6 150/233 and
+// 103/116, 30 beams 136/227 and 81/84; in FP8, were it run for them, 100 beams 136/154 and
+// 93/100 (128-beam classic tiles 98/107) and 60 beams 135/153 and 83/85 (64-beam classic
+// tiles 66/69).
+template <int PREC, int TAVG, int GROUP = 0>
+__device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *stage, uint8_t *abuf) {
+  const TileId t = tile_id(a, L);
+  if ((a.nbeam + 31) / 32 - t.bset * NW * BTW <= NW)
+    shared_tile_of<PREC, TAVG, GROUP == 1 ? 0 : GROUP, 1>(a, t, stage, abuf);   // (0 and 1: the same results)
+  else
+    shared_tile_of<PREC, TAVG, GROUP, BTW>(a, t, stage, abuf);
 }
 }  // namespace shared
 #endif

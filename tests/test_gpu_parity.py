@@ -913,3 +913,28 @@ def test_packed_blocks_on_several_streams_and_in_a_graph(bf):
     plan.close()
     for s in streams:
         ok(hip.hipStreamDestroy(s))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("tavg", [8, 32, 64])
+def test_short_beam_sets_of_shared_tiles(bf, prec, tavg):
+    """Shared tiles of a set of at most four beam tiles (one a wave, waves without
+    beams idle) give each beam the bits it has in a full set: the first beams of a
+    plan with whole 256-beam sets, fine and group weights, both input orders."""
+    for i, (nbeam, whole) in enumerate([(1, 256), (33, 256), (96, 256), (128, 256), (300, 512), (384, 512)]):
+        for fine in (0, 1):
+            got = []
+            for nb in (nbeam, whole):
+                cfg = bf.config(nant=61, nchan=24, npkt=96, nbeam=nb, tavg=tavg, precision=prec, weight_mode=fine,
+                                angle_mode=bf.ANGLE_SIN, input_order=i & 1)
+                antpos, cal, theta = bf.synth_geometry(61, cfg.ncal, whole, 9)
+                plan = bf.Plan(cfg)
+                plan.set_weights(antpos, cal, bf.reference_freqs(1498.75, 24), theta[:nb])
+                plan.variant = 5                       # (pinned: BFK_VAR_SHARED_256)
+                block = bf.synth_block(cfg, 70 + i)
+                out, power, bp = plan.process_block(block, np.full(nb, 3e-5, np.float32), want_power=True, want_beam_power=True)
+                got.append((out[:, :nbeam], power[:, :nbeam], bp[:nbeam]))
+                plan.close()
+            for a, b in zip(*got):
+                assert np.array_equal(a, b)
