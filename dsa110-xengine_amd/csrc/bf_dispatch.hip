@@ -189,7 +189,8 @@ static TileCost packed_cost(const bfk_dims *d) {
   float sum = 0.f, end = 0.f;
   for (int i = 0; i < nset; i++) {
     const int split = bfk_packed_split(live, i);
-    const float t = p[split == 1 ? 0 : split == 2 ? 1 : 2][d->prec];
+    const float t = p[split == 1 ? 0 : split == 2 ? 1 : 2][d->prec] *
+                    (split == 1 && live < 8 * i + 8 ? 0.28f + 0.09f * (float)(live - 8 * i) : 1.f);
     sum += t;
     for (long n = tiles; n > 0;) {
       if (ncu == 1 && n >= 256) {
@@ -225,10 +226,18 @@ static TileCost packed_cost(const bfk_dims *d) {
 }
 extern "C" int bfk_use_packed(const bfk_dims *d) {
   if (d->pinned || !bfk_packed_bytes(d) || !bfk_variant_supported(d, d->variant)) return 0;
-  // (fine weights of 256-beam tiles contend for the L2 among others)
+  // (256-beam tiles: fine weights contend for the L2 among others; zeros take the
+  // place of missing beam tiles, and five of eight this part of the time)
   static const float contend[4] = {1.05f, 1.1f, 1.25f, 1.27f};
+  static const float five[2][4] = {{0.87f, 0.9f, 0.85f, 0.95f}, {0.67f, 0.74f, 0.81f, 0.8f}};
   TileCost v = variant_cost(d);
-  if (d->variant == BFK_VAR_SHARED_256 && d->wmode != 0) v.among *= contend[d->prec];
+  if (d->variant == BFK_VAR_SHARED_256) {
+    const bool group = d->wmode == 0;
+    const int live = (d->nbeam + 31) / 32, nset = (live + 7) / 8;
+    const float part = 1.f - (1.f - five[group][d->prec]) / 3 * (float)(8 * nset - live) / (float)nset;
+    v.alone *= part;
+    v.among *= part * (group ? 1.f : contend[d->prec]);
+  }
   spread_tiles(d, &v);
   const TileCost k = packed_cost(d);
   return k.alone < 1.05f * v.alone && k.among < 1.05f * v.among && k.alone * k.among < 0.95f * v.alone * v.among;

@@ -93,18 +93,15 @@ __global__ __launch_bounds__(256) void bf_pack_kernel(BfArgs a, int nb2, uint8_t
 struct PSet {
   int bt0, split;
 };
-// Set i of `live` beam tiles: eights, then what remains in the fewest wave times:
-// up to 2 tiles on four waves each, 4 on two, 5 and 6 as 4 and the rest.
+// Set i of `live` beam tiles: eights, then what remains: up to 2 tiles on four waves
+// each, 3 and 4 on two, more as an eight (140 beams, five tiles, as one such set, or as
+// four and one: 256 antennas x 384 channels x 2048 samples in FP8 276 and 333 us among
+// other blocks, in FP16 321 and 431).
 __host__ __device__ inline PSet packed_set(int live, int i) {
   const int full = live / 8, rem = live % 8;
-  if (i < full || rem == 7) return {i * 8, 1};
-  if (i > full) return {full * 8 + 4, 4};
-  return {full * 8, rem <= 2 ? 4 : 2};
+  return {i * 8, i < full || rem > 4 ? 1 : rem <= 2 ? 4 : 2};
 }
-__host__ __device__ inline int packed_sets(int live) {
-  const int rem = live % 8;
-  return live / 8 + (rem > 0) + (rem == 5 || rem == 6);
-}
+__host__ __device__ inline int packed_sets(int live) { return (live + 7) / 8; }
 
 template <int PREC, int TAVG, int NKC, int SPLIT>
 __device__ __forceinline__ void packed_tile(const BfArgs &a, TileId t, int tb2, int nb2, int bt0, const uint8_t *packed,

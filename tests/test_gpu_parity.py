@@ -826,7 +826,7 @@ def _use_packed(bf, cfg):
 PACKED = [(70, 104, 640, 150, 0, 1), (66, 112, 608, 290, 0, 1), (67, 120, 768, 100, 1, 0), (68, 104, 640, 190, 1, 1),
           (65, 56, 640, 290, 2, 0), (65, 96, 704, 70, 2, 1), (67, 104, 640, 1, 3, 1), (127, 112, 672, 224, 3, 1),
           (132, 112, 736, 70, 0, 1), (133, 112, 608, 256, 0, 0), (130, 64, 512, 100, 1, 1), (129, 72, 480, 400, 1, 0),
-          (131, 48, 448, 190, 2, 1), (256, 104, 640, 1, 2, 1)]
+          (131, 104, 640, 190, 2, 1), (256, 104, 640, 1, 2, 1)]
 
 
 @pytest.mark.gpu
