@@ -244,7 +244,9 @@ int dsaxbf_beam_power(dsaxbf_plan *plan, float *d_beam_power, void *stream);
  * supports it, and dsaxbf_set_variant rejects it.
  * A plan whose variant nobody set runs, where its tiles would leave the chip
  * part idle, smaller work items in the variant's place (one 32-beam tile and one
- * channel and pol per wave) with the variant's bits.
+ * channel and pol per wave) with the variant's bits.  Above 64 antennas such a
+ * plan may first repack the block into a buffer of its own (one byte a
+ * sample, antennas padded to 128 or 256; without the memory the variant runs); executes of one plan that overlap take it in turn.
  * No counterpart in the reference (its five kernels per int have one fixed
  * launch shape, dsaX_beamformer.cu:955-1003). */
 enum {
@@ -263,7 +265,8 @@ int dsaxbf_get_variant(const dsaxbf_plan *plan);
 
 /* Autotuner: times every variant the shape supports (the plan's own device
  * buffers, current weights; reps launches each after one warm-up) and keeps
- * the fastest (or the smaller work items above, where they are no slower).  ms, if not NULL, receives DSAXBF_NVARIANT mean launch times in
+ * the fastest (or what an unset plan runs in its place, above, where that is no
+ * slower).  ms, if not NULL, receives DSAXBF_NVARIANT mean launch times in
  * milliseconds (-1 for a variant that cannot run this shape).  Synchronous;
  * requires dsaxbf_set_weights (or -s mode).  No counterpart in the reference. */
 int dsaxbf_autotune(dsaxbf_plan *plan, int reps, float *ms);
