@@ -257,11 +257,20 @@ static_assert(2 * 4096 <= AB8, "FP6 operands of one (channel, pol) fit the FP8 h
 //      pol 1), so one row is held at a time and the second is loaded in place
 //      once, during step 7's second unit, with the rolling path's registers.
 //      The powers are summed in another order than the rolling path's.
-template <int PREC, int TAVG, int GROUP, int NB>
-__device__ __forceinline__ void shared_tile_of(const BfArgs &a, const TileId &t, uint8_t *stage, uint8_t *abuf) {
+// NB: beam tiles a wave: two, or, for blocks of at most 128 beams, one (waves without
+//   beams then only stage and unpack).  With two, half the waves of such a block
+//   multiplied zeros.  us alone and among other blocks, 64 antennas x 384 channels x
+//   2048 samples, fine weights: 100 beams in FP6 112/144 and 85/93, in three-part FP6
+//   150/233 and 103/116, 30 beams 136/227 and 81/84; in FP8, were it run for them, 100
+//   beams 136/154 and 93/100 (128-beam classic tiles 98/107) and 60 beams 135/153 and
+//   83/85 (64-beam classic tiles 66/69).  Larger blocks' last sets gain nothing from it
+//   (300 beams 177 and 177).
+template <int PREC, int TAVG, int GROUP = 0, int NB = BTW>
+__device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *stage, uint8_t *abuf) {
   static_assert(GROUP != 1 || PREC == 1 || PREC == 2, "FP16 and three-part FP6 cannot hold both rows");
   constexpr int UNIT = PREC == 0 ? AB16 / 2 : AB8 / 2;    // operand bytes per unit
   constexpr int NP = TAVG <= 32 ? 32 / TAVG : 1;
+  const TileId t = tile_id(a, L);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: weight rows stay scalar
@@ -459,22 +468,6 @@ __device__ __forceinline__ void shared_tile_of(const BfArgs &a, const TileId &t,
 
   // (c)
   if (live) tile_output<TAVG>(a, t, btw, n, h, part, 0, 2);
-}
-
-// A set of at most four beam tiles takes one a wave (waves without beams only stage
-// and unpack), else two: with two, half the waves of 128 beams or fewer multiplied
-// zeros.  us alone and among other blocks, 64 antennas x 384 channels x 2048 samples,
-// fine weights: 100 beams in FP6 112/144 and 85/93, in three-part FP6 150/233 and
-// 103/116, 30 beams 136/227 and 81/84; in FP8, were it run for them, 100 beams 136/154 and
-// 93/100 (128-beam classic tiles 98/107) and 60 beams 135/153 and 83/85 (64-beam classic
-// tiles 66/69).
-template <int PREC, int TAVG, int GROUP = 0>
-__device__ __forceinline__ void shared_tile(const BfArgs &a, int L, uint8_t *stage, uint8_t *abuf) {
-  const TileId t = tile_id(a, L);
-  if ((a.nbeam + 31) / 32 - t.bset * NW * BTW <= NW)
-    shared_tile_of<PREC, TAVG, GROUP == 1 ? 0 : GROUP, 1>(a, t, stage, abuf);   // (0 and 1: the same results)
-  else
-    shared_tile_of<PREC, TAVG, GROUP, BTW>(a, t, stage, abuf);
 }
 }  // namespace shared
 #endif
