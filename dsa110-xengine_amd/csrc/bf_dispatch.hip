@@ -65,7 +65,7 @@ extern "C" int bfk_beamform_classic(const bfk_dims *d, const uint8_t *d_in, cons
                                     float *d_power, float *d_bpart, void *stream);
 extern "C" int bfk_beamform_shared(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                                    const float *d_wscale, const float *d_scale, uint8_t *d_out,
-                                   float *d_power, float *d_bpart, void *stream);
+                                   float *d_power, float *d_bpart, int in_order, void *stream);
 extern "C" int bfk_beamform_shared8(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                                    const float *d_wscale, const float *d_scale, uint8_t *d_out,
                                    float *d_power, float *d_bpart, void *stream);
@@ -251,6 +251,15 @@ extern "C" int bfk_variant_supported(const bfk_dims *d, int v) {
   return bfk_classic_beams(v, d->nkc) > 0;
 }
 
+// FP8 blocks of 65 to 128 beams that the 128-beam classic tiles would take run shared
+// tiles of one beam tile a wave, in the same order (64 antennas x 384 channels x 2048
+// samples -> 100 beams, fine weights 97/106 -> 92/99 us alone and among other blocks;
+// x 4096 -> 128, group weights 188/206 -> 176/190; FP16 103/108 with either).
+static bool short_shared(const bfk_dims *d) {
+  return !d->pinned && d->variant == BFK_VAR_CLASSIC_128S && d->prec == 1 && d->nkc == 1 && d->nbeam > 64 && d->nbeam <= 128;
+}
+extern "C" int bfk_unset_differs(const bfk_dims *d) { return bfk_spread_tiles(d) || short_shared(d); }
+
 extern "C" int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                             const float *d_wscale, const float *d_scale, uint8_t *d_out,
                             float *d_power, float *d_bpart, float *d_beam_power, void *d_psum,
@@ -278,8 +287,10 @@ extern "C" int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *
     return bfk_beamform_spread(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, d_beam_power, d_psum,
                                nbw, pol_outer, stream);
   }
+  if (short_shared(d))
+    return bfk_beamform_shared(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, 1, stream);
   if (d->variant == BFK_VAR_SHARED_256)
-    return d->nkc == 1 ? bfk_beamform_shared(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, stream)
+    return d->nkc == 1 ? bfk_beamform_shared(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, 0, stream)
                        : bfk_beamform_shared8(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, stream);
   return bfk_beamform_classic(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, stream);
 }

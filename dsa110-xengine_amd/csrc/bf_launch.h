@@ -94,6 +94,9 @@ int bfk_variant_supported(const bfk_dims *d, int v);
  * the variant, for blocks whose tiles would leave the chip part idle) that
  * bfk_beamform runs in the variant's place unless it is pinned, or 0. */
 int bfk_spread_tiles(const bfk_dims *d);
+/* 1 if bfk_beamform runs something else than the variant where none is pinned
+ * (without a repacked block). */
+int bfk_unset_differs(const bfk_dims *d);
 
 /* Batched classic launches: all blocks of a batch in one launch per kernel
  * instantiation (precision, tavg, antenna chunks, beam tiles per wave).

@@ -76,10 +76,10 @@ static void launch_g(int tavg, dim3 grid, hipStream_t s, const BfArgs &a) {
 // spill with both, so they hold one row at a time, pol-outer.  One beam tile a
 // wave has no use for both rows: it reloads them, with the same results.
 template <int PREC>
-static void launch(int tavg, dim3 grid, hipStream_t s, const BfArgs &a) {
+static void launch(int tavg, dim3 grid, hipStream_t s, const BfArgs &a, bool in_order) {
   constexpr int G = PREC == 1 || PREC == 2 ? 1 : 2;
   if (a.nbeam <= BSET / 2) {
-    if (a.wmode != 0 || (G == 1 && tavg >= 32)) launch_g<PREC, 0, 1>(tavg, grid, s, a);
+    if (a.wmode != 0 || in_order || (G == 1 && tavg >= 32)) launch_g<PREC, 0, 1>(tavg, grid, s, a);
     else launch_g<PREC, 2, 1>(tavg, grid, s, a);
   } else if (a.wmode != 0) {
     launch_g<PREC, 0, BTW>(tavg, grid, s, a);
@@ -109,16 +109,18 @@ static int shared_shape_ok(const bfk_dims *d) {
   return 1;
 }
 
+// in_order (at most 128 beams): the powers summed with pol fastest, as the classic
+// tiles do, whatever the weights.
 extern "C" int bfk_beamform_shared(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                                    const float *d_wscale, const float *d_scale, uint8_t *d_out,
-                                   float *d_power, float *d_bpart, void *stream) {
+                                   float *d_power, float *d_bpart, int in_order, void *stream) {
   if (!shared_shape_ok(d)) return -1;
   const BfArgs a = bf_make_args(d, d_in, d_wfrag, d_wscale, d_scale, d_out, d_power, d_bpart, BSET);
   const dim3 grid((a.ntiles + 7) / 8 * 8);
-  if (d->prec == 0) launch<0>(d->tavg, grid, (hipStream_t)stream, a);
-  else if (d->prec == 1) launch<1>(d->tavg, grid, (hipStream_t)stream, a);
-  else if (d->prec == 2) launch<2>(d->tavg, grid, (hipStream_t)stream, a);
-  else launch<3>(d->tavg, grid, (hipStream_t)stream, a);
+  if (d->prec == 0) launch<0>(d->tavg, grid, (hipStream_t)stream, a, in_order);
+  else if (d->prec == 1) launch<1>(d->tavg, grid, (hipStream_t)stream, a, in_order);
+  else if (d->prec == 2) launch<2>(d->tavg, grid, (hipStream_t)stream, a, in_order);
+  else launch<3>(d->tavg, grid, (hipStream_t)stream, a, in_order);
   return bfk_check(hipGetLastError(), "bf_shared_kernel");
 }
 

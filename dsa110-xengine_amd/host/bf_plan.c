@@ -480,7 +480,7 @@ int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_sca
     }
     p->dims.variant = unpinned ? best : v;
     p->dims.pinned = !unpinned;
-    if (unpinned && (!spread_wins || !(bfk_spread_tiles(&p->dims) || (p->d_packed && bfk_use_packed(&p->dims))))) break;
+    if (unpinned && (!spread_wins || !(bfk_unset_differs(&p->dims) || (p->d_packed && bfk_use_packed(&p->dims))))) break;
     float t = 0.f;
     he = hipSuccess;
     for (int r = -1; r < reps && rc == DSAXBF_OK && he == hipSuccess; r++) {

@@ -938,3 +938,27 @@ def test_short_beam_sets_of_shared_tiles(bf, prec, tavg):
                 plan.close()
             for a, b in zip(*got):
                 assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tavg", [8, 32, 64])
+def test_fp8_blocks_of_65_to_128_beams(bf, tavg):
+    """FP8 blocks too large for spread tiles and of 65 to 128 beams run shared tiles
+    of one beam tile a wave: the pinned variant's bits, three and four beam tiles,
+    fine and group weights, both input orders."""
+    for i, nbeam in enumerate((65, 96, 128)):
+        for fine in (0, 1):
+            cfg = bf.config(nant=60, nchan=256, npkt=640, nbeam=nbeam, tavg=tavg, precision=1, weight_mode=fine,
+                            angle_mode=bf.ANGLE_SIN, input_order=i & 1)
+            antpos, cal, theta = bf.synth_geometry(60, cfg.ncal, nbeam, 4)
+            block = np.random.default_rng(i).integers(0, 256, bf.input_bytes(cfg), dtype=np.uint8)
+            got = []
+            for pin in (False, True):
+                plan = bf.Plan(cfg)
+                plan.set_weights(antpos, cal, bf.reference_freqs(1498.75, 256), theta)
+                if pin:
+                    plan.variant = plan.variant
+                got.append(plan.process_block(block, np.full(nbeam, 3e-5, np.float32), want_power=True, want_beam_power=True))
+                plan.close()
+            for a, b in zip(*got):
+                assert np.array_equal(a, b)
