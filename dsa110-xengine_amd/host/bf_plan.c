@@ -33,7 +33,7 @@ struct dsaxbf_plan {
   void *d_packed;       /* the repacked block (or NULL), and its last use */
   hipEvent_t packed_done;
   pthread_mutex_t packed_lock;
-  void *d_psum;         /* of launches that sum the beam powers themselves, or NULL */
+  void *d_psum;         /* of launches that sum the beam powers themselves (behind d_wargs), or NULL */
   void *d_scratch;      /* the device's static scratch array (dsaxbf_execute_noalloc) */
   int have_weights;
 };
@@ -77,9 +77,15 @@ static void fill_dims(const dsaxbf_config *c, bfk_dims *d) {
                                : BFK_VAR_CLASSIC_64;
 }
 
-/* calibration (16 bytes an antenna and weight channel), frequencies, angles, positions */
+/* calibration (16 bytes an antenna and weight channel), frequencies, angles,
+ * positions; then, in whole cache lines, bfk_psum_bytes */
 static size_t wargs_bytes(const bfk_dims *d) {
-  return (size_t)d->nant * d->ncal * 16 + ((size_t)d->nchan + d->nbeam) * sizeof(double) + d->nant * sizeof(float);
+  return ((size_t)d->nant * d->ncal * 16 + ((size_t)d->nchan + d->nbeam) * sizeof(double) + d->nant * sizeof(float) + 127) &
+         ~(size_t)127;
+}
+/* what dsaxbf_set_weights copies: those and the zeros that the counters start with */
+static size_t wcopy_bytes(const bfk_dims *d) {
+  return wargs_bytes(d) + (bfk_psum_bytes(d) ? BFK_COUNTS * sizeof(unsigned) : 0);
 }
 
 void dsaxbf_destroy(dsaxbf_plan *p) {
@@ -94,7 +100,6 @@ void dsaxbf_destroy(dsaxbf_plan *p) {
   hipFree(p->d_beam_power);
   hipFree(p->d_scale);
   hipFree(p->d_bpart);
-  hipFree(p->d_psum);
   hipFree(p->d_packed);
   if (p->packed_done) hipEventDestroy(p->packed_done);
   pthread_mutex_destroy(&p->packed_lock);
@@ -135,12 +140,8 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_beam_power, (size_t)cfg->nbeam * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_scale, (size_t)cfg->nbeam * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_bpart, bfk_bpart_bytes(d));
-  if (e == hipSuccess) e = hipMalloc(&p->d_wargs, wargs_bytes(d));
-  if (bfk_psum_bytes(d)) {
-    if (e == hipSuccess) e = hipMalloc(&p->d_psum, bfk_psum_bytes(d));
-    /* (done by the first execute: dsaxbf_set_weights waits for this stream) */
-    if (e == hipSuccess) e = hipMemsetAsync(p->d_psum, 0, BFK_COUNTS * sizeof(unsigned), p->stream);
-  }
+  if (e == hipSuccess) e = hipMalloc(&p->d_wargs, wargs_bytes(d) + bfk_psum_bytes(d));
+  if (e == hipSuccess && bfk_psum_bytes(d)) p->d_psum = (char *)p->d_wargs + wargs_bytes(d);
   if (e != hipSuccess) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "device allocation failed: %s", hipGetErrorString(e));
@@ -153,7 +154,7 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
       (void)hipGetLastError();
     }
   }
-  p->h_wargs = malloc(wargs_bytes(d));
+  p->h_wargs = calloc(1, wcopy_bytes(d));
   if (!p->h_wargs) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "host allocation failed");
@@ -196,7 +197,7 @@ int dsaxbf_set_weights(dsaxbf_plan *p, const float *antpos, const float *cal,
     theta[b] = theta_rad ? theta_rad[b] : sep_arcmin * (double)(d->nbeam / 2 - 1 - b) * M_PI / 10800.0;
   const double *d_freqs = (const double *)((char *)p->d_wargs + ncal), *d_theta = d_freqs + d->nchan;
   int rc = DSAXBF_OK;
-  hipError_t e = hipMemcpyAsync(p->d_wargs, p->h_wargs, wargs_bytes(d), hipMemcpyHostToDevice, p->stream);
+  hipError_t e = hipMemcpyAsync(p->d_wargs, p->h_wargs, wcopy_bytes(d), hipMemcpyHostToDevice, p->stream);
   if (e != hipSuccess) {
     rc = dsaxbf_fail(DSAXBF_EHIP, "weights upload: %s", hipGetErrorString(e));
   } else {
