@@ -518,14 +518,20 @@ extern "C" size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice) {
 // line through the L1, so only blocks of some size gain (64 x 384 x 4096 124/129 and
 // 87/91, 45 x 96 x 4096 (35 MB) 33/21 and 28/21, 64 x 128 x 1024 (17 MB) 24/16 and
 // 29/13), with groups outermost smaller ones too (64 x 384 x 4096 125/127 and 57/51,
-// 63 x 48 x 2048 (12 MB) 21/12 and 24/8.6, 64 x 24 x 2048 18/9.5 and 21/8.0), and the
-// shortest, which its one launch bounds (60 x 16 x 128 9.9/6.6 and 12/4.3).  Slices
+// 63 x 48 x 2048 (12 MB) 21/12 and 24/8.6, 64 x 24 x 2048 18/9.5 and 21/8.0), wide
+// short ones in their one slice (antennas outermost 40 x 384 x 256 15.5/8.0 and 14.3/6.8,
+// 64 x 384 x 384 26/16 and 25/11, 64 x 200 x 256 14.9/9.0 and 18.5/7.9; groups outermost
+// 61 x 264 x 256 18.7/10.3 and 15.5/6.3, 64 x 160 x 256 14.3/8.2 and 15.2/5.7, 64 x 96 x
+// 256 12.3/6.6 and 14.8/5.4), and the shortest, which its one launch bounds (60 x 16 x
+// 128 9.9/6.6 and 12/4.3).  Slices
 // fill the CUs while each has 128 (256 above 32 antennas) packets: 64 x 384 x 512
 // in one 30/13, in two 30/19; 16 x 384 x 1024 in one, two and four 21/9, 16/7, 13/7.
 extern "C" int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order) {
   if (nant > 64 || npkt > 65536) return 0;
   const long bytes = (long)npkt * nant * nchan * 4;
-  if (nant > 32 && npkt > 64 && bytes < (order == 0 ? 32000000 : 10000000)) return 0;
+  if (nant > 32 && npkt > 64 && !(npkt <= 256 && nchan >= (order == 0 ? 300 : 160)) &&
+      bytes < (order == 0 ? 32000000 : 10000000))
+    return 0;
   const int wgs = nchan / (nant <= 32 ? 8 : 4), most = npkt / (nant <= 32 ? 128 : 256);
   int s = wgs >= 192 ? 1 : 256 / wgs;
   if (s > most) s = most;

@@ -119,7 +119,7 @@ def test_xengine_rejects_bad_shapes(bf):
 
 @pytest.mark.parametrize("nant,nchan,npkt,order", [
     (1, 8, 128, 0), (17, 24, 1056, 1), (32, 40, 640, 0), (8, 520, 96, 1), (33, 24, 64, 0), (64, 8, 32, 1),
-    (64, 72, 2016, 0), (45, 96, 2080, 0), (64, 48, 864, 1), (50, 104, 2048, 1)])
+    (64, 72, 2016, 0), (45, 96, 2080, 0), (64, 48, 864, 1), (50, 104, 2048, 1), (34, 304, 96, 0), (61, 160, 256, 1)])
 def test_xengine_reads_the_block_itself(bf, orc, nant, nchan, npkt, order):
     """The correlation that reads the untransposed block (up to 32 antennas, short
     and large blocks to 64), in one and several slices of even and odd numbers of
