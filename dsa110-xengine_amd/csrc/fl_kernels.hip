@@ -452,11 +452,12 @@ __device__ inline float fl_unkey(uint32_t k) {
 // keys: few waves issue an instruction only every eight cycles or so.)  Every
 // thread of the workgroup calls it (it has barriers), teams with data and FlSel
 // of their own.
-struct FlSel {
+struct alignas(16) FlSel {
   uint32_t hist[256];
   uint32_t lo[4], hi[4];             // per wave, then the range in [0]
   uint32_t k;
 };
+static_assert(alignof(FlSel) == 16, "hist is read 16 bytes at a time, in every element of an array");
 template <class G> __device__ inline uint32_t fl_kth(G get, int n, int k, int tid, FlSel &t) {
   const int lane = tid & 63;
   uint32_t lo = 0xFFFFFFFFu, hi = 0;
