@@ -31,7 +31,8 @@ __global__ __launch_bounds__(64 * STUFF_WAVES) void bf_stuff_kernel(bfk_dims d, 
                                                                     float *__restrict__ bpart) {
   constexpr int ABIT = ORDER == 0 ? 3 : 1;   // lane bits: antennas from here on, groups from GBIT, 16-byte half 0
   constexpr int GBIT = ORDER == 0 ? 1 : 4;
-  __shared__ int S[256][4][8];               // [antenna][group][4 packets]
+  __shared__ __attribute__((aligned(16))) int S[256][4][8];   // [antenna][group][4 packets]
+  static_assert(__alignof__(S) == 16, "S is written 16 bytes at a time");
   __shared__ int part[STUFF_WAVES][4][8];
   __shared__ float IB[4][10];                // up to 8 bins, then the two 32-sample halves
   const int nblk = d.nsamp / 64, t64 = blockIdx.x % nblk, g0 = blockIdx.x / nblk * 4;
