@@ -83,10 +83,6 @@ static size_t wargs_bytes(const bfk_dims *d) {
   return ((size_t)d->nant * d->ncal * 16 + ((size_t)d->nchan + d->nbeam) * sizeof(double) + d->nant * sizeof(float) + 127) &
          ~(size_t)127;
 }
-/* what dsaxbf_set_weights copies: those and the zeros that the counters start with */
-static size_t wcopy_bytes(const bfk_dims *d) {
-  return wargs_bytes(d) + (bfk_psum_bytes(d) ? BFK_COUNTS * sizeof(unsigned) : 0);
-}
 
 void dsaxbf_destroy(dsaxbf_plan *p) {
   if (!p) return;
@@ -141,7 +137,12 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_scale, (size_t)cfg->nbeam * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_bpart, bfk_bpart_bytes(d));
   if (e == hipSuccess) e = hipMalloc(&p->d_wargs, wargs_bytes(d) + bfk_psum_bytes(d));
-  if (e == hipSuccess && bfk_psum_bytes(d)) p->d_psum = (char *)p->d_wargs + wargs_bytes(d);
+  if (e == hipSuccess && bfk_psum_bytes(d)) {
+    p->d_psum = (char *)p->d_wargs + wargs_bytes(d);
+    /* the counters' only zeros: every launch leaves them zero, and any launch comes
+       after dsaxbf_set_weights, which waits for this stream */
+    e = hipMemsetAsync(p->d_psum, 0, BFK_COUNTS * sizeof(unsigned), p->stream);
+  }
   if (e != hipSuccess) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "device allocation failed: %s", hipGetErrorString(e));
@@ -154,7 +155,7 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
       (void)hipGetLastError();
     }
   }
-  p->h_wargs = calloc(1, wcopy_bytes(d));
+  p->h_wargs = calloc(1, wargs_bytes(d));
   if (!p->h_wargs) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "host allocation failed");
@@ -197,7 +198,7 @@ int dsaxbf_set_weights(dsaxbf_plan *p, const float *antpos, const float *cal,
     theta[b] = theta_rad ? theta_rad[b] : sep_arcmin * (double)(d->nbeam / 2 - 1 - b) * M_PI / 10800.0;
   const double *d_freqs = (const double *)((char *)p->d_wargs + ncal), *d_theta = d_freqs + d->nchan;
   int rc = DSAXBF_OK;
-  hipError_t e = hipMemcpyAsync(p->d_wargs, p->h_wargs, wcopy_bytes(d), hipMemcpyHostToDevice, p->stream);
+  hipError_t e = hipMemcpyAsync(p->d_wargs, p->h_wargs, wargs_bytes(d), hipMemcpyHostToDevice, p->stream);
   if (e != hipSuccess) {
     rc = dsaxbf_fail(DSAXBF_EHIP, "weights upload: %s", hipGetErrorString(e));
   } else {

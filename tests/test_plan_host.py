@@ -1,0 +1,72 @@
+"""The host side of plans, batches and the correlator's plan without a GPU:
+host/bf_plan.c, host/bf_batch.c and host/xc_plan.c linked with tests/hip_stub.c,
+whose device memory is host memory and whose launches, events and waits are a
+log.  Checks what the plans share between calls, streams and threads."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from conftest import ROOT
+
+HOST = os.path.join(ROOT, "dsa110-xengine_amd", "host")
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory, bf):
+    so = str(tmp_path_factory.mktemp("stub") / "plan.so")
+    src = [os.path.join(HOST, f) for f in ("bf_plan.c", "bf_batch.c", "xc_plan.c", "bf_host.c")]
+    subprocess.run(["gcc", "-O1", "-fPIC", "-shared", "-std=gnu11", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + HOST, "-Wl,-Bsymbolic", "-o", so, *src,
+                    os.path.join(ROOT, "tests", "hip_stub.c"), "-lpthread", "-lm"], check=True)
+    L = C.CDLL(so)
+    L.stub_log.restype = C.c_char_p
+    for f in ("dsaxbf_execute", "dsaxbf_set_variant", "dsaxbf_set_weights", "dsaxbf_destroy", "dsaxbf_get_stream"):
+        getattr(L, f).argtypes = None
+    L.dsaxbf_get_stream.restype = C.c_void_p
+    return L
+
+
+def _set(lib, **values):
+    for k, v in values.items():
+        t = {"stub_capturing": C.c_void_p, "stub_live": C.c_long, "stub_psum_bytes": C.c_size_t,
+             "stub_packed_bytes": C.c_size_t}.get(k, C.c_int)
+        t.in_dll(lib, k).value = v
+
+
+def _plan(lib, bf, psum=0, packed=0):
+    _set(lib, stub_psum_bytes=psum, stub_packed_bytes=packed)
+    cfg = bf.config(nant=64, nchan=384, npkt=32, nbeam=64, tavg=32, weight_mode=bf.WEIGHTS_FINE)
+    p = C.c_void_p()
+    assert lib.dsaxbf_create(C.byref(p), C.byref(cfg)) == 0
+    return p, cfg
+
+
+def _weights(lib, p, cfg, v=1.0):
+    arr = [np.full(n, v, t) for n, t in ((cfg.nant, np.float32), (cfg.nant * cfg.ncal * 4, np.float32),
+                                         (cfg.nchan, np.float64), (cfg.nbeam, np.float64))]
+    assert lib.dsaxbf_set_weights(p, *(C.c_void_p(a.ctypes.data) for a in arr), C.c_double(0)) == 0
+
+
+ANY = C.c_void_p(64)         # a device pointer that the stub does not look behind
+
+
+def _execute(lib, p, stream=None, power=True):
+    return lib.dsaxbf_execute(p, ANY, ANY, ANY, None, ANY if power else None, stream)
+
+
+def test_counters_are_zero_from_the_start_and_left_alone(lib, bf):
+    """The counters of a launch that sums the beam powers are zero before the first
+    launch, and dsaxbf_set_weights does not write them: a launch in flight on
+    another stream would lose its count, and all later ones would sum too early."""
+    p, cfg = _plan(lib, bf, psum=4096)
+    _weights(lib, p, cfg)
+    assert _execute(lib, p) == 0
+    count = (C.c_uint32 * 32).from_address(C.c_void_p.in_dll(lib, "stub_psum").value)
+    assert not any(count)
+    count[3] = 7                                   # a launch has counted seven workgroups
+    _weights(lib, p, cfg)
+    assert count[3] == 7 and sum(count) == 7
+    lib.dsaxbf_destroy(p)
