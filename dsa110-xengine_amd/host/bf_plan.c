@@ -32,8 +32,10 @@ struct dsaxbf_plan {
   void *d_wargs, *h_wargs;  /* dsaxbf_set_weights' arguments, on the device and packed for it */
   void *d_packed;       /* the repacked block (or NULL), and its last use */
   hipEvent_t packed_done;
-  pthread_mutex_t packed_lock;
   void *d_psum;         /* of launches that sum the beam powers themselves (behind d_wargs), or NULL */
+  hipEvent_t psum_ready, psum_done;   /* the last such launch on the plan's stream, and on another */
+  int psum_elsewhere;   /* psum_done is of a launch that the plan's stream does not follow yet */
+  pthread_mutex_t turn; /* of the launches that use d_packed or d_psum */
   void *d_scratch;      /* the device's static scratch array (dsaxbf_execute_noalloc) */
   int have_weights;
 };
@@ -84,6 +86,12 @@ static size_t wargs_bytes(const bfk_dims *d) {
          ~(size_t)127;
 }
 
+/* what the first dsaxbf_set_weights, before any launch, copies: those and the zeros
+ * that the counters start with (every launch leaves them zero) */
+static size_t wfirst_bytes(const bfk_dims *d) {
+  return wargs_bytes(d) + (bfk_psum_bytes(d) ? BFK_COUNTS * sizeof(unsigned) : 0);
+}
+
 void dsaxbf_destroy(dsaxbf_plan *p) {
   if (!p) return;
   hipSetDevice(p->cfg.device);
@@ -98,7 +106,9 @@ void dsaxbf_destroy(dsaxbf_plan *p) {
   hipFree(p->d_bpart);
   hipFree(p->d_packed);
   if (p->packed_done) hipEventDestroy(p->packed_done);
-  pthread_mutex_destroy(&p->packed_lock);
+  if (p->psum_ready) hipEventDestroy(p->psum_ready);
+  if (p->psum_done) hipEventDestroy(p->psum_done);
+  pthread_mutex_destroy(&p->turn);
   hipFree(p->d_wargs);
   free(p->h_wargs);
   if (p->stream) hipStreamDestroy(p->stream);
@@ -123,7 +133,7 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   dsaxbf_plan *p = calloc(1, sizeof(*p));
   if (!p) return dsaxbf_fail(DSAXBF_ENOMEM, "plan allocation failed");
   p->cfg = *cfg;
-  pthread_mutex_init(&p->packed_lock, NULL);
+  pthread_mutex_init(&p->turn, NULL);
   fill_dims(cfg, &p->dims);
   const bfk_dims *d = &p->dims;
   size_t nin = dsaxbf_input_bytes(cfg), nout = dsaxbf_output_bytes(cfg);
@@ -139,9 +149,8 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   if (e == hipSuccess) e = hipMalloc(&p->d_wargs, wargs_bytes(d) + bfk_psum_bytes(d));
   if (e == hipSuccess && bfk_psum_bytes(d)) {
     p->d_psum = (char *)p->d_wargs + wargs_bytes(d);
-    /* the counters' only zeros: every launch leaves them zero, and any launch comes
-       after dsaxbf_set_weights, which waits for this stream */
-    e = hipMemsetAsync(p->d_psum, 0, BFK_COUNTS * sizeof(unsigned), p->stream);
+    e = hipEventCreateWithFlags(&p->psum_ready, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&p->psum_done, hipEventDisableTiming);
   }
   if (e != hipSuccess) {
     dsaxbf_destroy(p);
@@ -155,7 +164,7 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
       (void)hipGetLastError();
     }
   }
-  p->h_wargs = calloc(1, wargs_bytes(d));
+  p->h_wargs = calloc(1, wfirst_bytes(d));
   if (!p->h_wargs) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "host allocation failed");
@@ -198,7 +207,8 @@ int dsaxbf_set_weights(dsaxbf_plan *p, const float *antpos, const float *cal,
     theta[b] = theta_rad ? theta_rad[b] : sep_arcmin * (double)(d->nbeam / 2 - 1 - b) * M_PI / 10800.0;
   const double *d_freqs = (const double *)((char *)p->d_wargs + ncal), *d_theta = d_freqs + d->nchan;
   int rc = DSAXBF_OK;
-  hipError_t e = hipMemcpyAsync(p->d_wargs, p->h_wargs, wargs_bytes(d), hipMemcpyHostToDevice, p->stream);
+  hipError_t e = hipMemcpyAsync(p->d_wargs, p->h_wargs, p->have_weights ? wargs_bytes(d) : wfirst_bytes(d),
+                                hipMemcpyHostToDevice, p->stream);
   if (e != hipSuccess) {
     rc = dsaxbf_fail(DSAXBF_EHIP, "weights upload: %s", hipGetErrorString(e));
   } else {
@@ -305,6 +315,33 @@ int dsaxbf_get_weights(dsaxbf_plan *p, double *w) {
   return DSAXBF_OK;
 }
 
+static int capturing(hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
+/* Stream s waits for the last launches that used d_packed, or d_psum (the caller
+ * holds the turn). */
+static hipError_t wait_turn(dsaxbf_plan *p, int packed, int psum, hipStream_t s) {
+  hipError_t e = packed ? hipStreamWaitEvent(s, p->packed_done, 0) : hipSuccess;
+  if (psum && s != p->stream) {
+    if (e == hipSuccess) e = hipEventRecord(p->psum_ready, p->stream);
+    if (e == hipSuccess) e = hipStreamWaitEvent(s, p->psum_ready, 0);
+  }
+  if (psum && p->psum_elsewhere && e == hipSuccess) e = hipStreamWaitEvent(s, p->psum_done, 0);
+  if (psum && s == p->stream && e == hipSuccess) p->psum_elsewhere = 0;
+  return e;
+}
+/* ... and the launch just queued on s is the last. */
+static void end_turn(dsaxbf_plan *p, int packed, int psum, hipStream_t s) {
+  hipError_t e = packed ? hipEventRecord(p->packed_done, s) : hipSuccess;
+  if (psum && s != p->stream) {
+    p->psum_elsewhere = 1;
+    if (e == hipSuccess) e = hipEventRecord(p->psum_done, s);
+  }
+  if (e != hipSuccess) hipStreamSynchronize(s);
+}
+
 /* One block on device buffers with the per-unit beam-power partial sums in
  * bpart (kernel launches only). */
 static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, void *packed, const uint8_t *d_in, const float *d_scale,
@@ -313,30 +350,32 @@ static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, void *packed, 
   const bfk_dims *d = &p->dims;
   if (!p->have_weights && d->stuff != DSAXBF_STUFF_ANTS)
     return dsaxbf_fail(DSAXBF_ESTATE, "execute before dsaxbf_set_weights");
-  void *s = stream ? stream : (void *)p->stream;
+  hipStream_t s = stream ? (hipStream_t)stream : p->stream;
   int rc, summed = 0;
   if (d->stuff != DSAXBF_STUFF_ANTS) {
-    /* The repacked block: executes of the plan that overlap, on several streams or
-       from several threads, take it in turn.  A graph's replays would not wait for
-       each other, so under capture the block runs without. */
-    if (packed) {
-      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-      if (!bfk_use_packed(d) || hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
-        packed = NULL;
-    }
-    if (packed) {
-      pthread_mutex_lock(&p->packed_lock);
-      if (hipStreamWaitEvent(s, p->packed_done, 0) != hipSuccess) {
-        pthread_mutex_unlock(&p->packed_lock);
-        return dsaxbf_fail(DSAXBF_EHIP, "waiting for the repacked block");
+    /* The repacked block, and the sums and counters of a launch that adds the beam
+       powers itself: executes of the plan that overlap, on several streams or from
+       several threads, take them in turn.  The plan's own stream is its own order,
+       so that a run on it records no event for the sums (and costs what it did).  A
+       graph's replays would not wait for each other, so under capture the block
+       runs without either. */
+    if (!d_beam_power || d->stuff != DSAXBF_STUFF_NONE || d->pinned) psum = NULL;
+    if (packed && !bfk_use_packed(d)) packed = NULL;
+    if ((packed || psum) && (capturing(s) || (psum && s != p->stream && capturing(p->stream)))) packed = psum = NULL;
+    const int mine = packed || psum;
+    if (mine) {
+      pthread_mutex_lock(&p->turn);
+      if (wait_turn(p, packed != NULL, psum != NULL, s) != hipSuccess) {
+        pthread_mutex_unlock(&p->turn);
+        return dsaxbf_fail(DSAXBF_EHIP, "waiting for the plan's buffers");
       }
     }
     /* (-q replaces beam 0's partial sums afterwards) */
     rc = bfk_beamform(d, d_in, p->d_wfrag, p->d_wscale, d_scale, d_out, d_power, bpart,
                       d->stuff == DSAXBF_STUFF_NONE ? d_beam_power : NULL, psum, &summed, packed, s);
-    if (packed) {
-      if (!rc && hipEventRecord(p->packed_done, s) != hipSuccess) hipStreamSynchronize(s);
-      pthread_mutex_unlock(&p->packed_lock);
+    if (mine) {
+      if (!rc) end_turn(p, packed != NULL, psum != NULL, s);
+      pthread_mutex_unlock(&p->turn);
     }
     if (rc) return dsaxbf_fail(rc, "%s", bfk_last_error());
   }

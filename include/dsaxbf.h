@@ -244,9 +244,12 @@ int dsaxbf_beam_power(dsaxbf_plan *plan, float *d_beam_power, void *stream);
  * supports it, and dsaxbf_set_variant rejects it.
  * A plan whose variant nobody set runs, where its tiles would leave the chip
  * part idle, smaller work items in the variant's place (one 32-beam tile and one
- * channel and pol per wave) with the variant's bits.  Above 64 antennas such a
+ * channel and pol per wave) with the variant's bits; the smallest blocks' launch
+ * also sums the beam powers, in counters of the plan.  Above 64 antennas such a
  * plan may first repack the block into a buffer of its own (one byte a
- * sample, antennas padded to 128 or 256; without the memory the variant runs); executes of one plan that overlap take it in turn.
+ * sample, antennas padded to 128 or 256; without the memory the variant runs).
+ * Executes of one plan that overlap take the counters and the buffer in turn;
+ * executes that are captured use neither.
  * No counterpart in the reference (its five kernels per int have one fixed
  * launch shape, dsaX_beamformer.cu:955-1003). */
 enum {

@@ -70,3 +70,69 @@ def test_counters_are_zero_from_the_start_and_left_alone(lib, bf):
     _weights(lib, p, cfg)
     assert count[3] == 7 and sum(count) == 7
     lib.dsaxbf_destroy(p)
+
+
+def _ordered(log):
+    """Whether each launch that uses plan-owned memory for one launch at a time
+    starts after the one before it has ended, by its stream's order and the events."""
+    clock, event, last, unordered = {}, {}, None, []
+    for i, line in enumerate(log.decode().splitlines()):
+        op, s, *rest = line.split()
+        seen = clock.setdefault(s, set())
+        if op == "record":
+            event[rest[0]] = set(seen)
+        elif op == "wait":
+            seen |= event.get(rest[0], set())
+        elif op == "launch" and rest[0] != "plain":
+            if last is not None and last not in seen:
+                unordered.append(line)
+            last = i
+            seen.add(i)
+    return not unordered
+
+
+STREAMS = [C.c_void_p(16 * k) for k in range(1, 4)]    # a caller's
+
+
+@pytest.mark.parametrize("kind", ["sums", "packed"])
+def test_launches_on_several_streams_take_the_plans_memory_in_turn(lib, bf, kind):
+    """Executes of one plan on its own stream and on others, in every order of two
+    and three: each launch that sums its beam powers, or reads the repacked block,
+    waits for the one before it; a run on the plan's own stream needs no event for
+    its sums."""
+    p, cfg = _plan(lib, bf, **{"psum" if kind == "sums" else "packed": 4096})
+    _weights(lib, p, cfg)
+    lib.stub_reset()
+    for a in (None, *STREAMS):
+        for b in (None, *STREAMS):
+            for c in (None, *STREAMS):
+                for s in (a, b, c):
+                    assert _execute(lib, p, s) == 0
+    log = lib.stub_log()
+    assert log.count(kind.encode()) == 3 * 64 and b"plain" not in log and _ordered(log)
+    lib.stub_reset()
+    for _ in range(3):
+        assert _execute(lib, p) == 0
+    if kind == "sums":
+        assert b"".join(line[:6] for line in lib.stub_log().splitlines()[-2:]) == b"launch" * 2
+    lib.dsaxbf_destroy(p)
+
+
+@pytest.mark.parametrize("kind", ["sums", "packed"])
+def test_captured_launches_use_none_of_it(lib, bf, kind):
+    """Under capture, whose replays would not wait for other launches, a block runs
+    without the plan's counters and repacked copy and records no event; so does one
+    on another stream while the plan's own is captured, whose end it could not wait
+    for."""
+    p, cfg = _plan(lib, bf, **{"psum" if kind == "sums" else "packed": 4096})
+    _weights(lib, p, cfg)
+    own = lib.dsaxbf_get_stream(p)
+    for captured, s, alone in [(STREAMS[0].value, STREAMS[0], True), (own, None, True), (own, STREAMS[1], kind == "sums")]:
+        assert _execute(lib, p, STREAMS[2]) == 0
+        _set(lib, stub_capturing=captured)
+        lib.stub_reset()
+        assert _execute(lib, p, s) == 0
+        ops = [" ".join(x.split()[::2]) for x in lib.stub_log().decode().splitlines()]
+        assert (ops == ["launch plain", "power"]) == alone
+        _set(lib, stub_capturing=None)
+    lib.dsaxbf_destroy(p)
