@@ -30,6 +30,7 @@ struct dsaxbf_plan {
   float *d_scale;
   float *d_bpart;       /* per-tile beam power sums of the last execute */
   void *d_wargs, *h_wargs;  /* dsaxbf_set_weights' arguments, on the device and packed for it */
+  pthread_mutex_t pointing; /* held by the call whose arguments they are */
   void *d_packed;       /* the repacked block (or NULL), and its last use */
   hipEvent_t packed_done;
   void *d_psum;         /* of launches that sum the beam powers themselves (behind d_wargs), or NULL */
@@ -109,6 +110,7 @@ void dsaxbf_destroy(dsaxbf_plan *p) {
   if (p->psum_ready) hipEventDestroy(p->psum_ready);
   if (p->psum_done) hipEventDestroy(p->psum_done);
   pthread_mutex_destroy(&p->turn);
+  pthread_mutex_destroy(&p->pointing);
   hipFree(p->d_wargs);
   free(p->h_wargs);
   if (p->stream) hipStreamDestroy(p->stream);
@@ -134,6 +136,7 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   if (!p) return dsaxbf_fail(DSAXBF_ENOMEM, "plan allocation failed");
   p->cfg = *cfg;
   pthread_mutex_init(&p->turn, NULL);
+  pthread_mutex_init(&p->pointing, NULL);
   fill_dims(cfg, &p->dims);
   const bfk_dims *d = &p->dims;
   size_t nin = dsaxbf_input_bytes(cfg), nout = dsaxbf_output_bytes(cfg);
@@ -197,6 +200,7 @@ int dsaxbf_set_weights(dsaxbf_plan *p, const float *antpos, const float *cal,
   /* one copy of all arguments, packed in memory that the plan keeps (the last
      call's copy and kernel have ended): four copies to memory allocated and freed
      here took 139 us a call of 64 antennas x 384 channels, against 90 */
+  pthread_mutex_lock(&p->pointing);
   const size_t ncal = (size_t)d->nant * d->ncal * 16;
   double *freqs = (double *)((char *)p->h_wargs + ncal), *theta = freqs + d->nchan;
   float *pos = (float *)(theta + d->nbeam);
@@ -219,6 +223,7 @@ int dsaxbf_set_weights(dsaxbf_plan *p, const float *antpos, const float *cal,
   e = hipStreamSynchronize(p->stream);
   if (e != hipSuccess && rc == DSAXBF_OK) rc = dsaxbf_fail(DSAXBF_EHIP, "weights kernel: %s", hipGetErrorString(e));
   if (rc == DSAXBF_OK) p->have_weights = 1;
+  pthread_mutex_unlock(&p->pointing);
   return rc;
 }
 

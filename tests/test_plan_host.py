@@ -5,6 +5,7 @@ log.  Checks what the plans share between calls, streams and threads."""
 import ctypes as C
 import os
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -135,4 +136,19 @@ def test_captured_launches_use_none_of_it(lib, bf, kind):
         ops = [" ".join(x.split()[::2]) for x in lib.stub_log().decode().splitlines()]
         assert (ops == ["launch plain", "power"]) == alone
         _set(lib, stub_capturing=None)
+    lib.dsaxbf_destroy(p)
+
+
+def test_pointings_set_from_two_threads_do_not_mix(lib, bf):
+    """dsaxbf_set_weights packs its arguments into memory that the plan keeps: calls
+    from two threads each compute their weights from their own arguments."""
+    p, cfg = _plan(lib, bf)
+    _set(lib, stub_slow_copies=1, stub_torn=0)
+    threads = [threading.Thread(target=lambda v=v: [_weights(lib, p, cfg, v) for _ in range(8)]) for v in (1.0, 2.0)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    _set(lib, stub_slow_copies=0)
+    assert C.c_int.in_dll(lib, "stub_torn").value == 0
     lib.dsaxbf_destroy(p)
