@@ -379,7 +379,7 @@ static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, void *packed, 
     rc = bfk_beamform(d, d_in, p->d_wfrag, p->d_wscale, d_scale, d_out, d_power, bpart,
                       d->stuff == DSAXBF_STUFF_NONE ? d_beam_power : NULL, psum, &summed, packed, s);
     if (mine) {
-      if (!rc) end_turn(p, packed != NULL, psum != NULL, s);
+      end_turn(p, packed != NULL, psum != NULL, s);   /* (of a launch that failed, what was queued) */
       pthread_mutex_unlock(&p->turn);
     }
     if (rc) return dsaxbf_fail(rc, "%s", bfk_last_error());

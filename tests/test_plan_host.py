@@ -152,3 +152,16 @@ def test_pointings_set_from_two_threads_do_not_mix(lib, bf):
     _set(lib, stub_slow_copies=0)
     assert C.c_int.in_dll(lib, "stub_torn").value == 0
     lib.dsaxbf_destroy(p)
+
+
+def test_a_launch_that_failed_half_way_keeps_its_turn(lib, bf):
+    """Repacking may be queued when the launch behind it fails: the next execute, on
+    another stream, still waits for it."""
+    p, cfg = _plan(lib, bf, packed=4096)
+    _weights(lib, p, cfg)
+    lib.stub_reset()
+    _set(lib, stub_fail_launch=1)
+    assert _execute(lib, p, STREAMS[0]) != 0
+    assert _execute(lib, p, STREAMS[1]) == 0
+    assert _ordered(lib.stub_log())
+    lib.dsaxbf_destroy(p)
