@@ -140,6 +140,7 @@ int dsaxbf_batch_create(dsaxbf_batch **out, dsaxbf_plan *const *plans, int n,
     dsaxbf_batch_destroy(b);
     return rc;
   }
+  for (int i = 0; i < n; i++) dsaxbf_join_batch(plans[i]);
   *out = b;
   return DSAXBF_OK;
 }

@@ -24,5 +24,7 @@ int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_sca
 /* dsaxbf_set_variant for the batch layer's own choice: the plan's executes may
  * still run the spread tiles. */
 int dsaxbf_pick_variant(dsaxbf_plan *p, int v);
+/* The plan is a batch's from now on: it gives back its repacked block. */
+void dsaxbf_join_batch(dsaxbf_plan *p);
 
 #endif

@@ -33,6 +33,7 @@ struct dsaxbf_plan {
   pthread_mutex_t pointing; /* held by the call whose arguments they are */
   void *d_packed;       /* the repacked block (or NULL), and its last use */
   hipEvent_t packed_done;
+  int batched;          /* the plan has joined a batch, whose launches do not repack */
   void *d_psum;         /* of launches that sum the beam powers themselves (behind d_wargs), or NULL */
   hipEvent_t psum_ready, psum_done;   /* the last such launch on the plan's stream, and on another */
   int psum_elsewhere;   /* psum_done is of a launch that the plan's stream does not follow yet */
@@ -117,6 +118,27 @@ void dsaxbf_destroy(dsaxbf_plan *p) {
   free(p);
 }
 
+/* The repacked block where the plan's executes use it, and none where they do not.
+ * (Without the memory for it the block runs the variant.)  Not in
+ * dsaxbf_set_variant, which a caller may call under capture. */
+static void fit_packed(dsaxbf_plan *p) {
+  const bfk_dims *d = &p->dims;
+  const int want = !p->batched && bfk_use_packed(d);
+  pthread_mutex_lock(&p->turn);
+  if (p->d_packed && !want) {
+    hipEventSynchronize(p->packed_done);
+    hipFree(p->d_packed);
+    p->d_packed = NULL;
+  } else if (!p->d_packed && want) {
+    if ((!p->packed_done && hipEventCreateWithFlags(&p->packed_done, hipEventDisableTiming) != hipSuccess) ||
+        hipMalloc(&p->d_packed, bfk_packed_bytes(d)) != hipSuccess) {
+      p->d_packed = NULL;
+      (void)hipGetLastError();
+    }
+  }
+  pthread_mutex_unlock(&p->turn);
+}
+
 int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
   dsaxbf_clear_error();
   if (!out) return dsaxbf_fail(DSAXBF_EINVAL, "plan pointer is NULL");
@@ -159,14 +181,7 @@ int dsaxbf_create(dsaxbf_plan **out, const dsaxbf_config *cfg) {
     dsaxbf_destroy(p);
     return dsaxbf_fail(DSAXBF_ENOMEM, "device allocation failed: %s", hipGetErrorString(e));
   }
-  /* (without the memory for it the block runs the variant) */
-  if (bfk_use_packed(d)) {
-    if (hipEventCreateWithFlags(&p->packed_done, hipEventDisableTiming) != hipSuccess ||
-        hipMalloc(&p->d_packed, bfk_packed_bytes(d)) != hipSuccess) {
-      p->d_packed = NULL;
-      (void)hipGetLastError();
-    }
-  }
+  fit_packed(p);
   p->h_wargs = calloc(1, wfirst_bytes(d));
   if (!p->h_wargs) {
     dsaxbf_destroy(p);
@@ -223,6 +238,7 @@ int dsaxbf_set_weights(dsaxbf_plan *p, const float *antpos, const float *cal,
   e = hipStreamSynchronize(p->stream);
   if (e != hipSuccess && rc == DSAXBF_OK) rc = dsaxbf_fail(DSAXBF_EHIP, "weights kernel: %s", hipGetErrorString(e));
   if (rc == DSAXBF_OK) p->have_weights = 1;
+  fit_packed(p);
   pthread_mutex_unlock(&p->pointing);
   return rc;
 }
@@ -349,7 +365,7 @@ static void end_turn(dsaxbf_plan *p, int packed, int psum, hipStream_t s) {
 
 /* One block on device buffers with the per-unit beam-power partial sums in
  * bpart (kernel launches only). */
-static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, void *packed, const uint8_t *d_in, const float *d_scale,
+static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, int packed, const uint8_t *d_in, const float *d_scale,
                         uint8_t *d_out, float *d_power, float *d_beam_power, void *stream) {
   if (!p || !d_in || !d_scale || !d_out) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
   const bfk_dims *d = &p->dims;
@@ -365,21 +381,26 @@ static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, void *packed, 
        graph's replays would not wait for each other, so under capture the block
        runs without either. */
     if (!d_beam_power || d->stuff != DSAXBF_STUFF_NONE || d->pinned) psum = NULL;
-    if (packed && !bfk_use_packed(d)) packed = NULL;
-    if ((packed || psum) && (capturing(s) || (psum && s != p->stream && capturing(p->stream)))) packed = psum = NULL;
+    packed = packed && p->packed_done && bfk_use_packed(d);
+    if ((packed || psum) && (capturing(s) || (psum && s != p->stream && capturing(p->stream)))) {
+      packed = 0;
+      psum = NULL;
+    }
     const int mine = packed || psum;
     if (mine) {
       pthread_mutex_lock(&p->turn);
-      if (wait_turn(p, packed != NULL, psum != NULL, s) != hipSuccess) {
+      packed = packed && p->d_packed;
+      if (wait_turn(p, packed, psum != NULL, s) != hipSuccess) {
         pthread_mutex_unlock(&p->turn);
         return dsaxbf_fail(DSAXBF_EHIP, "waiting for the plan's buffers");
       }
     }
     /* (-q replaces beam 0's partial sums afterwards) */
     rc = bfk_beamform(d, d_in, p->d_wfrag, p->d_wscale, d_scale, d_out, d_power, bpart,
-                      d->stuff == DSAXBF_STUFF_NONE ? d_beam_power : NULL, psum, &summed, packed, s);
+                      d->stuff == DSAXBF_STUFF_NONE ? d_beam_power : NULL, psum, &summed,
+                      packed ? p->d_packed : NULL, s);
     if (mine) {
-      end_turn(p, packed != NULL, psum != NULL, s);   /* (of a launch that failed, what was queued) */
+      end_turn(p, packed, psum != NULL, s);   /* (of a launch that failed, what was queued) */
       pthread_mutex_unlock(&p->turn);
     }
     if (rc) return dsaxbf_fail(rc, "%s", bfk_last_error());
@@ -398,7 +419,7 @@ static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, void *packed, 
 int dsaxbf_execute(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
                    float *d_power, float *d_beam_power, void *stream) {
   if (!p) return dsaxbf_fail(DSAXBF_EINVAL, "NULL plan");
-  return execute_with(p, p->d_bpart, p->d_psum, p->d_packed, d_in, d_scale, d_out, d_power, d_beam_power, stream);
+  return execute_with(p, p->d_bpart, p->d_psum, 1, d_in, d_scale, d_out, d_power, d_beam_power, stream);
 }
 
 int dsaxbf_execute_noalloc(dsaxbf_plan *p, const uint8_t *d_in, const float *d_scale, uint8_t *d_out,
@@ -412,7 +433,7 @@ int dsaxbf_execute_noalloc(dsaxbf_plan *p, const uint8_t *d_in, const float *d_s
                        need, have);
   /* every partial sum is overwritten by this launch before it is read: the
      array needs no clearing between calls */
-  return execute_with(p, (float *)p->d_scratch, NULL, NULL, d_in, d_scale, d_out, d_power, d_beam_power, stream);
+  return execute_with(p, (float *)p->d_scratch, NULL, 0, d_in, d_scale, d_out, d_power, d_beam_power, stream);
 }
 
 int dsaxbf_beam_power(dsaxbf_plan *p, float *d_beam_power, void *stream) {
@@ -485,6 +506,11 @@ int dsaxbf_pick_variant(dsaxbf_plan *p, int v) {
   int rc = dsaxbf_set_variant(p, v);
   p->dims.pinned = pinned;
   return rc;
+}
+
+void dsaxbf_join_batch(dsaxbf_plan *p) {
+  p->batched = 1;
+  fit_packed(p);
 }
 
 int dsaxbf_get_variant(const dsaxbf_plan *p) { return p ? p->dims.variant : -1; }
@@ -568,11 +594,16 @@ int dsaxbf_autotune(dsaxbf_plan *p, int reps, float *ms) {
   /* any voltages do: the work does not depend on the values */
   HIPCHK(hipMemsetAsync(p->d_in, 0x5a, dsaxbf_input_bytes(&p->cfg), p->stream), "hipMemsetAsync");
   HIPCHK(hipMemsetAsync(p->d_scale, 0, sizeof(float) * p->cfg.nbeam, p->stream), "hipMemsetAsync");
+  const int pinned = p->dims.pinned;
+  p->batched = p->dims.pinned = 0;
+  fit_packed(p);         /* to be timed with the others */
+  p->dims.pinned = pinned;
   int best, spread;
   int rc = dsaxbf_time_variants(p, p->d_in, p->d_scale, p->d_out, reps, ms, &best, &spread);
   if (rc == DSAXBF_OK) {
     p->dims.variant = best;
     p->dims.pinned = !spread;
   }
+  fit_packed(p);
   return rc;
 }

@@ -248,6 +248,9 @@ int dsaxbf_beam_power(dsaxbf_plan *plan, float *d_beam_power, void *stream);
  * also sums the beam powers, in counters of the plan.  Above 64 antennas such a
  * plan may first repack the block into a buffer of its own (one byte a
  * sample, antennas padded to 128 or 256; without the memory the variant runs).
+ * The buffer is given back by the first dsaxbf_set_weights after a variant was
+ * set, and by dsaxbf_batch_create, whose launches do not repack: from then on
+ * the plan's own executes run the variant, until dsaxbf_autotune.
  * Executes of one plan that overlap take the counters and the buffer in turn;
  * executes that are captured use neither.
  * No counterpart in the reference (its five kernels per int have one fixed

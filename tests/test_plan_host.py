@@ -165,3 +165,40 @@ def test_a_launch_that_failed_half_way_keeps_its_turn(lib, bf):
     assert _execute(lib, p, STREAMS[1]) == 0
     assert _ordered(lib.stub_log())
     lib.dsaxbf_destroy(p)
+
+
+def test_the_repacked_block_is_held_only_where_executes_use_it(lib, bf):
+    """A plan gives back its repacked block once a variant is set (at the next
+    pointing, the call that may free memory) and when it joins a batch, whose
+    launches do not repack; the autotuner takes it again."""
+    live, log = C.c_long.in_dll(lib, "stub_live"), lambda: lib.stub_log().split()[-1:]
+    start = live.value
+
+    def ran(power=False):
+        lib.stub_reset()
+        assert _execute(lib, p, None, power) == 0
+        return [x.split()[-1] for x in lib.stub_log().splitlines() if x.startswith(b"launch")]
+
+    size = 1 << 20
+    p, cfg = _plan(lib, bf)
+    _weights(lib, p, cfg)
+    least = live.value - start
+    lib.dsaxbf_destroy(p)
+    assert live.value == start
+    p, cfg = _plan(lib, bf, packed=size)
+    _weights(lib, p, cfg)
+    assert ran() == [b"packed"] and live.value - start == least + size
+    assert lib.dsaxbf_set_variant(p, lib.dsaxbf_get_variant(p)) == 0
+    assert ran() == [b"plain"]
+    _weights(lib, p, cfg)
+    assert ran() == [b"plain"] and live.value - start == least
+    assert lib.dsaxbf_autotune(p, 1, None) == 0            # (the stub's times are equal)
+    assert ran() == [b"packed"] and live.value - start == least + size
+    batch, one = C.c_void_p(), (C.c_void_p * 1)
+    assert lib.dsaxbf_batch_create(C.byref(batch), one(p), 1, one(64), one(64), one(64), None) == 0
+    assert ran() == [b"plain"] and live.value - start == least
+    _weights(lib, p, cfg)
+    assert ran() == [b"plain"] and live.value - start == least
+    lib.dsaxbf_batch_destroy(batch)
+    lib.dsaxbf_destroy(p)
+    assert live.value == start
