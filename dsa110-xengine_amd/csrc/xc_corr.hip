@@ -508,8 +508,6 @@ extern "C" size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice) {
   return nslice > 1 ? (size_t)nslice * bfk_xcorr_vis_bytes(nant, nchan) : 0;
 }
 
-// d_turn: the input's size; d_part: bfk_xcorr_part_bytes of nslice, or of nfused where
-// that (bfk_xcorr_fused_slices) is given and the fused kernel runs.
 // Time slices of the fused kernel, 0 where it does not run: above 64 antennas, with
 // sums that FP32 may not hold, and where the turned copy is faster.  us alone and
 // among others, turned and fused: up to 32 antennas always (32 x 384 x 4096 52/54
@@ -538,6 +536,9 @@ extern "C" int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order) 
   return s < 1 ? 1 : s;
 }
 
+// nfused: 0, or bfk_xcorr_fused_slices, with which the fused kernel runs.  d_part:
+// bfk_xcorr_part_bytes of its slices, or of nslice; d_turn: the input's size, not used
+// by the fused kernel.
 extern "C" int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t *d_in, uint8_t *d_turn,
                          float *d_part, int nslice, int nfused, float *d_vis, void *stream) {
   if (nant < 1 || nant > 96 || nchan < 8 || nchan % 8 || npkt < XUP || npkt % XUP || order < 0 || order > 1) {
@@ -552,7 +553,7 @@ extern "C" int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t
     bfk_set_error("bfk_xcorr: %d slices of the fused kernel (partials %p)", nfused, (void *)d_part);
     return -1;
   }
-  if (nslice < 1 || nslice > npkt / XUP || (nslice > 1 && !d_part) || !d_turn) {
+  if (nslice < 1 || nslice > npkt / XUP || (!nfused && ((nslice > 1 && !d_part) || !d_turn))) {
     bfk_set_error("bfk_xcorr: %d slices of %d units (partials %p)", nslice, npkt / XUP, (void *)d_part);
     return -1;
   }

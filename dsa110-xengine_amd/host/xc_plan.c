@@ -27,7 +27,7 @@ struct dsaxbf_xengine {
   int nant, nchan, npkt, order, device, nslice;
   int nfused;           /* slices of the kernel that reads the block itself; 0: it does not run */
   hipStream_t stream;
-  uint8_t *d_in, *d_turn;
+  uint8_t *d_in, *d_turn;   /* d_turn: NULL where that kernel runs */
   float *d_vis, *d_part;
 };
 
@@ -77,7 +77,7 @@ int dsaxbf_xengine_create(dsaxbf_xengine **out, int nant, int nchan, int npkt, i
   const size_t nin = (size_t)npkt * nant * nchan * 4, npart = part_bytes(x, x->nslice, x->nfused);
   hipError_t e = hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void **)&x->d_in, nin);
-  if (e == hipSuccess) e = hipMalloc((void **)&x->d_turn, nin);
+  if (e == hipSuccess && !x->nfused) e = hipMalloc((void **)&x->d_turn, nin);
   if (e == hipSuccess) e = hipMalloc((void **)&x->d_vis, bfk_xcorr_vis_bytes(nant, nchan));
   if (e == hipSuccess && npart) e = hipMalloc((void **)&x->d_part, npart);
   if (e != hipSuccess) {
@@ -112,6 +112,17 @@ int dsaxbf_xengine_set_slices(dsaxbf_xengine *x, int nslice) {
   const size_t npart = part_bytes(x, nslice, nfused);
   if (npart && hipMalloc((void **)&part, npart) != hipSuccess)
     return dsaxbf_fail(DSAXBF_ENOMEM, "partial visibilities (%zu bytes)", npart);
+  if (!nfused && !x->d_turn) {
+    const size_t nin = (size_t)x->npkt * x->nant * x->nchan * 4;
+    if (hipMalloc((void **)&x->d_turn, nin) != hipSuccess) {
+      x->d_turn = NULL;
+      hipFree(part);
+      return dsaxbf_fail(DSAXBF_ENOMEM, "turned block (%zu bytes)", nin);
+    }
+  } else if (nfused) {
+    hipFree(x->d_turn);
+    x->d_turn = NULL;
+  }
   hipFree(x->d_part);
   x->d_part = part;
   x->nslice = nslice;

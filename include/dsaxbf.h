@@ -407,13 +407,13 @@ void *dsaxbf_xengine_stream(dsaxbf_xengine *x);   /* the plan's hipStream_t */
  * input's size), the correlation over time slices, and the sum of the
  * slices' partial visibilities (plan-owned) when there is more than one
  * slice.  Up to 64 antennas, unless slices are set, the correlation may read
- * the block itself instead, in slices of its own. */
+ * the block itself instead, in slices of its own and without the planes. */
 int dsaxbf_xengine_execute(dsaxbf_xengine *x, const uint8_t *d_in, float *d_vis,
                            void *stream);
 /* Time slices the correlation runs in (1 .. npkt/32; 0 = the library's
  * choice for the shape, the default).  Tuning only: results are identical
- * (exact integer sums).  Reallocates the partial sums; not while a launch
- * on the plan is in flight. */
+ * (exact integer sums).  Reallocates the partial sums and the planes; not
+ * while a launch on the plan is in flight. */
 int dsaxbf_xengine_set_slices(dsaxbf_xengine *x, int nslice);
 int dsaxbf_xengine_get_slices(const dsaxbf_xengine *x);
 /* Host block in, host visibilities out (copies, run, wait): the

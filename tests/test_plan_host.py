@@ -202,3 +202,26 @@ def test_the_repacked_block_is_held_only_where_executes_use_it(lib, bf):
     lib.dsaxbf_batch_destroy(batch)
     lib.dsaxbf_destroy(p)
     assert live.value == start
+
+
+def test_the_correlators_turned_copy_is_held_only_where_it_is_used(lib):
+    """A correlator plan whose kernel reads the block itself has no turned copy (the
+    input's size) until slices are set, and again none when they are the library's."""
+    live = C.c_long.in_dll(lib, "stub_live")
+    nin = 64 * 64 * 48 * 4
+    for fused in (0, 2):
+        start = live.value
+        _set(lib, stub_fused_slices=fused)
+        x = C.c_void_p()
+        assert lib.dsaxbf_xengine_create(C.byref(x), 64, 48, 64, 0, 0) == 0
+        for slices in (None, 1, 2, 0):
+            if slices is not None:
+                assert lib.dsaxbf_xengine_set_slices(x, slices) == 0
+            turned = not fused or slices in (1, 2)
+            part = 64 * (2 if slices == 2 else fused if not turned else 0)
+            assert live.value - start == nin + 64 + part + (nin if turned else 0)
+            lib.stub_reset()
+            assert lib.dsaxbf_xengine_execute(x, ANY, ANY, None) == 0
+            assert lib.stub_log() == (b"xcorr turned\n" if turned else b"xcorr fused\n")
+        lib.dsaxbf_xengine_destroy(x)
+        assert live.value == start
