@@ -10,8 +10,8 @@
 // upper triangle into [baseline][channel][pol][re, im] (:366-457).
 //
 // Here:
-//   - Up to 64 antennas, where that is faster, one kernel reads the block itself
-//     (xc_fused_kernel below); else:
+//   - Up to 64 antennas, where that pays (bfk_xcorr_use_fused), one kernel reads the
+//     block itself (xc_fused_kernel below); else:
 //   - xc_turn_kernel turns the packed block, still one byte (4-bit re, 4-bit
 //     im) per sample, into (channel, pol) planes [channel*2 + pol][antenna]
 //     [sample]: each lane reads one channel's 4-byte words of 64 packets
@@ -508,35 +508,91 @@ extern "C" size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice) {
   return nslice > 1 ? (size_t)nslice * bfk_xcorr_vis_bytes(nant, nchan) : 0;
 }
 
-// Time slices of the fused kernel, 0 where it does not run: above 64 antennas, with
-// sums that FP32 may not hold, and where the turned copy is faster.  us alone and
-// among others, turned and fused: up to 32 antennas always (32 x 384 x 4096 52/54
-// and 34/34; 10 x 64 x 1024 11.0/9.6 and 11.4/6.8; 20 x 16 x 128 7.8/6.5 and
-// 7.6/3.7).  Up to 64 with antennas outermost a thread's 16 bytes cost a 128-byte
-// line through the L1, so only blocks of some size gain (64 x 384 x 4096 124/129 and
-// 87/91, 45 x 96 x 4096 (35 MB) 33/21 and 28/21, 64 x 128 x 1024 (17 MB) 24/16 and
-// 29/13), with groups outermost smaller ones too (64 x 384 x 4096 125/127 and 57/51,
-// 63 x 48 x 2048 (12 MB) 21/12 and 24/8.6, 64 x 24 x 2048 18/9.5 and 21/8.0), wide
-// short ones in their one slice (antennas outermost 40 x 384 x 256 15.5/8.0 and 14.3/6.8,
-// 64 x 384 x 384 26/16 and 25/11, 64 x 200 x 256 14.9/9.0 and 18.5/7.9; groups outermost
-// 61 x 264 x 256 18.7/10.3 and 15.5/6.3, 64 x 160 x 256 14.3/8.2 and 15.2/5.7, 64 x 96 x
-// 256 12.3/6.6 and 14.8/5.4), and the shortest, which its one launch bounds (60 x 16 x
-// 128 9.9/6.6 and 12/4.3).  Slices
-// fill the CUs while each has 128 (256 above 32 antennas) packets: 64 x 384 x 512
-// in one 30/13, in two 30/19; 16 x 384 x 1024 in one, two and four 21/9, 16/7, 13/7.
-extern "C" int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order) {
+// The turned path or the fused kernel, and the latter's time slices, by modelled
+// times in us: of a block alone on one stream, and among others (three plans in turn,
+// where the launches themselves take 3.75, 6.6 and 9.4 for one, two and three).  Fitted
+// to 325 shapes of 8 to 64 antennas, 8 to 384 channels and 64 to 4096 samples in one to
+// 24 slices each, near the faster ones to 3 % (6 % above 32 antennas with antennas
+// outermost).
+//   fused: a workgroup per 8 channels (4 above 32 antennas) and slice; a base and some
+//     per 8 antennas, then a time per 32 packets.  Up to 32 antennas two share a CU.
+//     With antennas outermost a 128-byte line serves eight workgroups of one XCD, if
+//     the XCD has whole eights.  Several slices: the sum of their partials.
+//   turned: bytes, the units of a wave's slice, visibilities, and again the sum.
+struct XcCost {
+  float alone, among;
+};
+static float vis_mb(int nant, int nchan) { return 8e-6f * (float)nant * (float)(nant + 1) * (float)nchan; }
+static XcCost xc_fused_cost(int nant, int nchan, int npkt, int order, int slices) {
+  //                               base  /8 ant  /unit  + /antenna  MB    sum  /slice  /MB
+  static const float c[2][2][8] = {{{3.31f, .864f, .75f, .012f, .521f, 1.36f, .235f, 0.f},
+                                    {2.78f, 1.05f, .849f, .003f, .258f, 1.45f, .24f, .147f}},
+                                   {{5.13f, .437f, .512f, .019f, .258f, 1.92f, .22f, .177f},
+                                    {4.86f, .559f, .952f, .004f, .181f, 1.28f, .255f, .22f}}};
+  const float(&p)[8] = c[nant > 32][order];
+  const int sets = nchan / (nant <= 32 ? 8 : 4), wgs = sets * slices, room = nant <= 32 ? 512 : 256;
+  const int units = (npkt / XUP + slices - 1) / slices;
+  const float mb = 4e-6f * (float)npkt * (float)nant * (float)nchan, vis = vis_mb(nant, nchan) * (float)slices;
+  float unit = p[2] + p[3] * (float)nant;
+  if (nant <= 32 && wgs > 256) unit *= 1.8f;
+  if (nant > 32 && order == 0 && nchan > 32 && wgs % 64 && wgs % (8 * sets)) unit *= 1.16f;
+  const float once = p[0] + p[1] * (float)((nant + 7) / 8), chain = unit * (float)units;
+  const float sum = slices > 1 ? p[5] + p[6] * (float)slices + p[7] * vis : 0.f;
+  const float alone = fmaxf(once + (float)((wgs + room - 1) / room) * chain, mb / 4.3f) + p[4] * vis + sum;
+  const float share = (once + chain) * (float)wgs / (float)room + (slices > 1 ? p[7] * vis : 0.f);
+  return {alone, fmaxf(fmaxf(slices > 1 ? 6.6f : 3.75f, alone / 2.75f), fmaxf(share, mb / 4.3f))};
+}
+static XcCost xc_turned_cost(int nant, int nchan, int npkt, int order) {
+  //                               base   MB     /unit  /8 ant  vis MB  sum
+  static const float c[2][2][6] = {{{6.27f, .354f, .235f, .298f, .619f, 2.26f}, {6.32f, .266f, .25f, .275f, .815f, 2.61f}},
+                                   {{7.91f, .432f, .324f, .102f, .45f, 1.9f}, {7.19f, .406f, .337f, .211f, .346f, 2.52f}}};
+  const float(&p)[6] = c[nant > 32][order];
+  const int slices = bfk_xcorr_default_slices(nchan, npkt), units = (npkt / XUP + slices - 1) / slices;
+  const float mb = 4e-6f * (float)npkt * (float)nant * (float)nchan, vis = vis_mb(nant, nchan);
+  const float alone = p[0] + p[1] * mb + p[2] * (float)units + p[3] * (float)((nant + 7) / 8) + p[4] * vis * (float)slices +
+                      (slices > 1 ? p[5] : 0.f);
+  return {alone, fmaxf(slices > 1 ? 9.4f : 6.5f, fmaxf(alone / 2.3f, .66f * mb + .25f * vis))};
+}
+// The fused kernel's slices that make the product of its times least, none of them
+// above `most`; 0 where there are none, or the kernel cannot run: above 64 antennas, or
+// with sums that FP32 may not hold.
+static int xc_slices(int nant, int nchan, int npkt, int order, XcCost most) {
   if (nant > 64 || npkt > 65536) return 0;
-  const long bytes = (long)npkt * nant * nchan * 4;
-  if (nant > 32 && npkt > 64 && !(npkt <= 256 && nchan >= (order == 0 ? 300 : 160)) &&
-      bytes < (order == 0 ? 32000000 : 10000000))
-    return 0;
-  const int wgs = nchan / (nant <= 32 ? 8 : 4), most = npkt / (nant <= 32 ? 128 : 256);
-  int s = wgs >= 192 ? 1 : 256 / wgs;
-  if (s > most) s = most;
-  return s < 1 ? 1 : s;
+  const int room = (nant <= 32 ? 512 : 256) / (nchan / (nant <= 32 ? 8 : 4));
+  int best = 0;
+  float least = 0.f;
+  for (int s = 1; s <= 32 && s <= npkt / XUP && (s == 1 || s <= room); s++) {
+    const XcCost f = xc_fused_cost(nant, nchan, npkt, order, s);
+    if (f.alone > most.alone || f.among > most.among || (best && f.alone * f.among >= least)) continue;
+    least = f.alone * f.among;
+    best = s;
+  }
+  return best;
+}
+extern "C" int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order) {
+  return xc_slices(nant, nchan, npkt, order, {1e9f, 1e9f});
+}
+// The slices in which the fused kernel takes the turned path's place, or 0: where its
+// time among others is no longer, that of a block alone, with the 11 us of a launch and
+// its wait beside the kernels, at most 3 to 4 % longer (3 % shorter above 32 antennas
+// with antennas outermost, where the model errs by more), and their product 5 % less.
+// Of 70 shapes that it picks a block alone takes 0.58 to 1.07 times the turned path's
+// time (mean 0.96), one among others 0.50 to 0.93 (0.66).  us alone and among others,
+// turned and fused: 64 antennas x 384 channels x 4096 samples, antennas outermost 127/143
+// and 87/92, groups outermost 130/145 and 57/52; 63 x 48 x 2048, groups outermost 21.4/12.4
+// and 23.0/8.3 (with the launch and wait 32.6 and 34.3); 8 x 328 x 128 7.2/6.8 and 6.0/3.8.
+// Left turned: 60 x 16 x 128 10.0/6.6 and 12.1/4.2, 32 x 32 x 1088 12.8/9.6 and 15.0/6.6, 64
+// x 128 x 1024 with antennas outermost 23.4/15.8 and 27.6/14.1.
+extern "C" int bfk_xcorr_use_fused(int nant, int nchan, int npkt, int order) {
+  static const float longer[2][2] = {{1.03f, 1.03f}, {.97f, 1.04f}};
+  const XcCost t = xc_turned_cost(nant, nchan, npkt, order);
+  const int s = xc_slices(nant, nchan, npkt, order, {longer[nant > 32][order] * (t.alone + 11.f) - 11.f, t.among});
+  if (!s) return 0;
+  const XcCost f = xc_fused_cost(nant, nchan, npkt, order, s);
+  return f.alone * f.among < .95f * t.alone * t.among ? s : 0;
 }
 
-// nfused: 0, or bfk_xcorr_fused_slices, with which the fused kernel runs.  d_part:
+// nfused: 0, or the slices in which the fused kernel runs.  d_part:
 // bfk_xcorr_part_bytes of its slices, or of nslice; d_turn: the input's size, not used
 // by the fused kernel.
 extern "C" int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t *d_in, uint8_t *d_turn,
@@ -549,7 +605,7 @@ extern "C" int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t
     bfk_set_error("bfk_xcorr: block above 2 GiB");
     return -1;
   }
-  if (nfused && (nfused != bfk_xcorr_fused_slices(nant, nchan, npkt, order) || (nfused > 1 && !d_part))) {
+  if (nfused && (nant > 64 || npkt > 65536 || nfused < 0 || nfused > npkt / XUP || (nfused > 1 && !d_part))) {
     bfk_set_error("bfk_xcorr: %d slices of the fused kernel (partials %p)", nfused, (void *)d_part);
     return -1;
   }

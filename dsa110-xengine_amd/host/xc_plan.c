@@ -19,7 +19,7 @@
 size_t bfk_xcorr_vis_bytes(int nant, int nchan);
 size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice);
 int bfk_xcorr_default_slices(int nchan, int npkt);
-int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order);
+int bfk_xcorr_use_fused(int nant, int nchan, int npkt, int order);
 int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t *d_in, uint8_t *d_turn, float *d_part,
               int nslice, int nfused, float *d_vis, void *stream);
 
@@ -73,7 +73,7 @@ int dsaxbf_xengine_create(dsaxbf_xengine **out, int nant, int nchan, int npkt, i
   x->order = input_order;
   x->device = device;
   x->nslice = bfk_xcorr_default_slices(nchan, npkt);
-  x->nfused = bfk_xcorr_fused_slices(nant, nchan, npkt, input_order);
+  x->nfused = bfk_xcorr_use_fused(nant, nchan, npkt, input_order);
   const size_t nin = (size_t)npkt * nant * nchan * 4, npart = part_bytes(x, x->nslice, x->nfused);
   hipError_t e = hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void **)&x->d_in, nin);
@@ -101,7 +101,7 @@ int dsaxbf_xengine_set_slices(dsaxbf_xengine *x, int nslice) {
   dsaxbf_clear_error();
   if (!x) return dsaxbf_fail(DSAXBF_EINVAL, "NULL argument");
   /* (a number of slices asks for the turned copy and those slices) */
-  const int nfused = nslice ? 0 : bfk_xcorr_fused_slices(x->nant, x->nchan, x->npkt, x->order);
+  const int nfused = nslice ? 0 : bfk_xcorr_use_fused(x->nant, x->nchan, x->npkt, x->order);
   if (nslice == 0) nslice = bfk_xcorr_default_slices(x->nchan, x->npkt);
   if (nslice < 1 || nslice > x->npkt / 32)
     return dsaxbf_fail(DSAXBF_EINVAL, "nslice=%d outside 1..%d", nslice, x->npkt / 32);

@@ -170,7 +170,7 @@ void bfk_batch_free(void *h) { free(h); }
 size_t bfk_xcorr_vis_bytes(int nant, int nchan) { return 64; }
 size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice) { return nslice > 1 ? 64 * (size_t)nslice : 0; }
 int bfk_xcorr_default_slices(int nchan, int npkt) { return 1; }
-int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order) { return stub_fused_slices; }
+int bfk_xcorr_use_fused(int nant, int nchan, int npkt, int order) { return stub_fused_slices; }
 int bfk_xcorr(int nant, int nchan, int npkt, int order, const uint8_t *in, uint8_t *turn, float *part, int nslice,
               int nfused, float *vis, void *s) {
   pthread_mutex_lock(&lock);

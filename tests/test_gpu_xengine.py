@@ -138,3 +138,27 @@ def test_xengine_reads_the_block_itself(bf, orc, nant, nchan, npkt, order):
     assert np.array_equal(vis[0][:, :8], orc.xcorr(nant, 8, npkt, group.ravel(), 0))
     for x in plans:
         x.close()
+
+
+@pytest.mark.parametrize("nant,nchan,npkt,order", [
+    (1, 8, 32, 1), (17, 24, 1056, 1), (32, 40, 640, 0), (33, 24, 64, 0), (64, 8, 32, 1), (64, 48, 864, 1), (63, 48, 1024, 1),
+    (45, 40, 416, 0), (34, 304, 96, 0), (61, 160, 256, 1)])
+def test_xengine_block_reading_kernel_in_any_slices(bf, nant, nchan, npkt, order):
+    """The kernel that reads the block itself, by its launcher, whether or not plans of
+    this shape run it: one slice, uneven ones and as many as there are units of 32
+    packets (to 32) give the turned path's visibilities bit for bit."""
+    import ctypes as C
+    cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=8, input_order=order)
+    block = np.random.default_rng(nant).integers(0, 256, bf.input_bytes(cfg), dtype=np.uint8)
+    x = bf.XEngine(nant, nchan, npkt, order)
+    x.slices = x.slices
+    most = min(32, npkt // 32)
+    d_in, d_vis, d_part = bf.DeviceBuffer(block.nbytes), bf.DeviceBuffer(x.vis_bytes), bf.DeviceBuffer(most * x.vis_bytes)
+    d_in.upload(block)
+    x.execute(d_in, d_vis)
+    want = d_vis.download(np.empty((x.nbase, nchan, 2, 2), np.float32), x.stream)
+    for n in sorted({1, 2, 3, 7, most} & set(range(1, most + 1))):
+        d_vis.upload(np.full(want.shape, -1, np.float32))
+        assert bf.lib.bfk_xcorr(nant, nchan, npkt, order, d_in.ptr, None, d_part.ptr, 1, n, d_vis.ptr, C.c_void_p(x.stream)) == 0
+        assert np.array_equal(d_vis.download(np.empty_like(want), x.stream), want), n
+    x.close()
