@@ -11,7 +11,8 @@
 // every block below about 500 tiles takes that long.  Here the 16 steps of a
 // tile run in 16 waves and the 32-beam tiles in different workgroups: the same
 // block is 32 workgroups of one step per wave and takes 7 us, bound by latencies
-// (staging, weights, one chain, the sums).  56 channels x 512 samples x 200
+// (staging, weights, one chain, the sums), or 11 with the beam powers, whose own
+// launch takes 4.  56 channels x 512 samples x 200
 // antennas -> 128 beams, FP8: 106 -> 32 us.  A full chip prefers the other
 // schedules, whose waves read a staged or unpacked operand for more beams; the
 // rule is in bf_dispatch.hip.
@@ -232,7 +233,10 @@ __global__ __launch_bounds__(ST) void bf_spread_kernel(BfArgs a, int nbw, int po
   float part[2][1][NP];                          // in the adding waves
   // (a copy of the lane number that the compiler cannot see through: addresses
   // made from it stay in the adding branch instead of in registers across the
-  // chains, where they spill)
+  // chains.  Up to 64 antennas nothing then spills, up to 128 one to three
+  // registers in five of the kernels.  Above, where 64 registers of weights are
+  // prefetched beside 32 accumulators and 16 waves leave 128 in all, 8 to 44
+  // do, 36 to 164 bytes a lane, most with 8-sample bins)
   auto hide = [](int v) {
     asm volatile("" : "+v"(v));
     return v;
@@ -283,7 +287,7 @@ __global__ __launch_bounds__(ST) void bf_spread_kernel(BfArgs a, int nbw, int po
       const bool pf = NKC > 1 || u == 1;
       const int ni = !last || (NKC > 1 && u == 0 && S::NU == 2) ? i : min(i + 1, nbt - 1);
       spread_unit<PREC>(cr, ci, W, d0, d1, src, pf, wrec(ni, last ? 0 : kc + 1));
-      __builtin_amdgcn_sched_barrier(0);       // (the next chunk's operands would spill)
+      __builtin_amdgcn_sched_barrier(0);       // (the next chunk's operands would spill, more than does)
     }
 #pragma unroll
     for (int j = 0; j < NP; j++) {

@@ -10,11 +10,11 @@
 //   fl_stats_kernel   one pass for every statistic, optionally scaling the
 //                     block in place first (scaley fused, as a per-channel
 //                     table of the 256 byte values built in LDS with the
-//                     reference's FP64 formula): a workgroup owns a
-//                     beam's 256-channel slab, each lane 4 channels read as
-//                     one dword per row (a wave reads 256 contiguous bytes),
-//                     the 16 waves the 32 time segments of the reference's
-//                     threads.  Sums are integers (exact in any order); the
+//                     reference's FP64 formula): a workgroup owns a slab of
+//                     256 to 32 of a beam's channels, each lane 4 of them read
+//                     as one dword per row (a wave reads 256 contiguous bytes,
+//                     or 32 and up of several rows), the 16 waves the 32 time
+//                     segments of the reference's threads.  Sums are integers (exact in any order); the
 //                     variance comes from exact integer sums (the reference's
 //                     float sums differ from it by their rounding, < 1e-5
 //                     relative); ppspec keeps the reference's 32-segment
@@ -843,7 +843,10 @@ __global__ __launch_bounds__(256) void fl_flagts_list_kernel(uint8_t *data, cons
   }
 }
 
-// flag (gpu_flagger.cu:458-474): column midx[i] = bm * nchan + ch, every time.
+// flag (gpu_flagger.cu:458-474): column midx[i] = bm * nchan + ch, every time.  3 %
+// of the columns of 12 x 8192 x 400 take 10 us, but 16 after scaley in 32-channel
+// slabs, also some ms after it (10 after it in 256-channel slabs, which take 71 us
+// longer): what state of the caches the narrow slabs leave was not looked into.
 __global__ __launch_bounds__(256) void fl_flag_cols_kernel(uint8_t *data, const int *midx, int n,
                                                            const float *bpwr, int nb, int nt, int nc) {
   const int i = blockIdx.y;

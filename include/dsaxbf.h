@@ -227,7 +227,8 @@ int dsaxbf_execute_noalloc(dsaxbf_plan *plan, const uint8_t *d_in, const float *
 int dsaxbf_beam_power(dsaxbf_plan *plan, float *d_beam_power, void *stream);
 
 /* Variants of the fused kernel: three schedules and three tile shapes.  All
- * give bit-identical results; which is fastest depends on the shape (few beams
+ * give bit-identical results (with group weights up to FP32 rounding: shared tiles
+ * may add the powers in another order); which is fastest depends on the shape (few beams
  * favour small tiles) and the GPU.
  *   CLASSIC_256    one tile (256 beams x 64 samples x 8 channels) per
  *                  workgroup, two workgroups per CU (nant <= 64);
