@@ -131,6 +131,37 @@ static TileCost variant_cost(const bfk_dims *d) {
                                  : fmaxf(t.t2, steady);
   return {alone, fmaxf(alone / 3, steady)};
 }
+// Whether spread tiles of nbw beam tiles a workgroup, of modelled times s, hold up
+// against the variant's v: with both corrected by what 1250 blocks that the model gave
+// spread tiles took, neither may be longer (among others 3 % less).  By real over
+// modelled times, to 9-15 %: the antennas of the last chunk, the share of the CUs in
+// the first round and, for the variant, antennas outermost in it, for spread tiles
+// 8-sample bins.  Without it the variant was over 5 % faster for 15 of them alone and
+// for 64 among others (193 antennas x 40 channels x 512 samples -> 325 beams FP8, fine
+// weights, 98/35 us against 95/52); with it for none and 14 of 1098, and of 450 other
+// blocks for none and 10, which take about half the time alone.  (Below 9 us blocks
+// among others are bound by their launches.)
+static bool spread_holds(const bfk_dims *d, int nbw, const TileCost &s, const TileCost &v) {
+  static const float variant[3][2][4] = {{{.95f, .04f, -.05f, .06f}, {1.18f, .19f, -.42f, .06f}},
+                                         {{.78f, .08f, .08f, .12f}, {.88f, .13f, -.01f, .13f}},
+                                         {{.66f, .07f, .16f, .2f}, {.81f, .39f, .06f, .29f}}};
+  static const float spread[3][2][4] = {{{1.2f, .05f, -.05f, .13f}, {1.08f, .23f, -.11f, .1f}},
+                                        {{1.06f, .18f, -.05f, .11f}, {.84f, .22f, .14f, .08f}},
+                                        {{.75f, .22f, .25f, .2f}, {.86f, .29f, .11f, .18f}}};
+  const int k = d->nkc == 1 ? 0 : d->nkc == 2 ? 1 : 2;
+  const int beams = d->variant == BFK_VAR_SHARED_256 ? 256 : bfk_classic_beams(d->variant, d->nkc);
+  const float tiles = (float)(d->nsamp / TCU) * (float)d->ngroup, na = (float)d->nant / (float)d->nant_pad - .75f;
+  const float fv = fminf(tiles * (float)((d->nbeam + beams - 1) / beams) / 256, 1.f);
+  const float fs = fminf(tiles * (float)(((d->nbeam + 31) / 32 + nbw - 1) / nbw) / 256, 1.f);
+  auto real = [&](const float(&c)[4], float model, float fill, float last) {
+    return model * (c[0] + c[1] * na + c[2] * fill + c[3] * last);
+  };
+  const float ov = d->order == 0 ? fv : 0.f, bins = d->tavg == 8 ? 1.f : 0.f;
+  if (real(spread[k][0], s.alone, fs, bins) > real(variant[k][0], v.alone, fv, ov)) return false;
+  const float among = s.among > 9 ? real(spread[k][1], s.among, fs, bins) : s.among;
+  const float most = v.among > 9 ? real(variant[k][1], v.among, fv, ov) : v.among;
+  return fmaxf(among, 6.6f) * 1.03f <= fmaxf(most, 6.6f * 1.03f);
+}
 static int spread_tiles(const bfk_dims *d, TileCost *cost) {
   static const float t0[3][2] = {{4.5f, 4.6f}, {5.5f, 5.f}, {17.5f, 16.f}}, t1[3][2] = {{3.9f, 3.6f}, {7.6f, 7.4f}, {15.f, 14.f}};
   const int k = d->nkc == 1 ? 0 : d->nkc == 2 ? 1 : 2;
@@ -140,6 +171,7 @@ static int spread_tiles(const bfk_dims *d, TileCost *cost) {
   const TileCost v = variant_cost(d);
   float best = 0.f;
   int tiles = 0;
+  TileCost pick = {0.f, 0.f};
   for (int nset = (live + 15) / 16; nset <= live; nset++) {
     const int nbw = (live + nset - 1) / nset;
     const long wgs = ntile * nset, rounds = (wgs + 255) / 256;
@@ -152,9 +184,11 @@ static int spread_tiles(const bfk_dims *d, TileCost *cost) {
     if (!tiles || alone * among < best) {
       best = alone * among;
       tiles = nbw;
-      *cost = {alone, among};
+      pick = {alone, among};
     }
   }
+  if (!tiles || !spread_holds(d, tiles, pick, v)) return 0;
+  *cost = pick;
   return tiles;
 }
 extern "C" int bfk_spread_tiles(const bfk_dims *d) {

@@ -23,38 +23,37 @@ def psum_bytes(bf, cfg):
 
 
 # Blocks that run spread tiles: antennas, channels, packets, beams, precision, fine weights, the
-# 32-beam tiles that a workgroup takes, and whether the launch sums the beam powers itself.  Every
-# precision and weight mode with one, two, three and more tiles, with and without the sums (which
-# occur up to three), up to 64 antennas; with two and more at 65 to 128 and 129 to 256.
+# 32-beam tiles that a workgroup takes, and whether the launch sums the beam powers itself; in all
+# bins and both input orders.  Each precision and weight mode with one, two, three and more tiles,
+# with and without the sums (which occur up to three), up to 64 antennas; with two and more at 65
+# to 128 and 129 to 256 (as far as there are such blocks of up to 20 MB).
 SPREAD = [
-    (35, 184, 384, 11, 0, 0, 1, 0), (55, 144, 96, 11, 0, 0, 1, 1), (43, 32, 288, 365, 0, 0, 2, 0),
-    (20, 64, 224, 111, 0, 0, 2, 1), (62, 88, 224, 267, 0, 0, 3, 0), (35, 80, 256, 70, 0, 0, 3, 1),
-    (46, 184, 352, 158, 0, 0, 5, 0), (38, 184, 384, 1, 0, 1, 1, 0), (24, 72, 64, 233, 0, 1, 1, 1),
-    (53, 96, 96, 354, 0, 1, 2, 0), (50, 120, 256, 60, 0, 1, 2, 1), (49, 112, 192, 134, 0, 1, 3, 0),
-    (54, 128, 160, 71, 0, 1, 3, 1), (34, 168, 352, 299, 0, 1, 10, 0), (26, 184, 384, 20, 1, 0, 1, 0),
-    (54, 32, 320, 158, 1, 0, 1, 1), (26, 160, 96, 177, 1, 0, 2, 0), (60, 184, 128, 56, 1, 0, 2, 1),
-    (53, 64, 384, 90, 1, 0, 3, 0), (25, 160, 128, 89, 1, 0, 3, 1), (62, 40, 320, 194, 1, 0, 4, 0),
-    (23, 184, 384, 16, 1, 1, 1, 0), (59, 32, 256, 31, 1, 1, 1, 1), (21, 72, 256, 133, 1, 1, 2, 0),
-    (24, 184, 160, 46, 1, 1, 2, 1), (64, 72, 288, 188, 1, 1, 3, 0), (31, 120, 160, 90, 1, 1, 3, 1),
-    (24, 80, 288, 299, 1, 1, 5, 0), (25, 192, 384, 7, 2, 0, 1, 0), (47, 56, 128, 15, 2, 0, 1, 1),
-    (43, 40, 288, 190, 2, 0, 2, 0), (31, 88, 288, 47, 2, 0, 2, 1), (32, 72, 128, 287, 2, 0, 3, 0),
-    (36, 136, 96, 150, 2, 0, 3, 1), (23, 48, 224, 231, 2, 0, 4, 0), (28, 192, 384, 19, 2, 1, 1, 0),
-    (34, 16, 288, 69, 2, 1, 1, 1), (24, 160, 96, 170, 2, 1, 2, 0), (20, 120, 256, 43, 2, 1, 2, 1),
-    (53, 176, 64, 284, 2, 1, 3, 0), (61, 48, 384, 81, 2, 1, 3, 1), (61, 104, 128, 281, 2, 1, 5, 0),
-    (37, 184, 384, 25, 3, 0, 1, 0), (25, 72, 64, 74, 3, 0, 1, 1), (51, 144, 256, 33, 3, 0, 2, 0),
-    (33, 88, 352, 34, 3, 0, 2, 1), (21, 24, 384, 283, 3, 0, 3, 0), (28, 56, 320, 70, 3, 0, 3, 1),
-    (64, 120, 96, 200, 3, 0, 4, 0), (25, 192, 384, 29, 3, 1, 1, 0), (36, 80, 32, 75, 3, 1, 1, 1),
-    (58, 64, 192, 164, 3, 1, 2, 0), (51, 56, 288, 102, 3, 1, 2, 1), (57, 120, 352, 75, 3, 1, 3, 0),
-    (21, 96, 224, 70, 3, 1, 3, 1), (45, 192, 128, 103, 3, 1, 4, 0), (70, 32, 288, 232, 0, 0, 2, 0),
-    (80, 184, 96, 219, 0, 0, 4, 0), (67, 96, 160, 145, 0, 1, 2, 0), (82, 120, 128, 383, 0, 1, 4, 0),
-    (90, 144, 64, 356, 1, 0, 2, 0), (127, 176, 128, 319, 1, 0, 5, 0), (75, 176, 64, 199, 1, 1, 2, 0),
-    (91, 80, 160, 220, 1, 1, 4, 0), (66, 144, 256, 52, 2, 0, 2, 0), (65, 120, 320, 346, 2, 0, 11, 0),
-    (84, 192, 96, 127, 2, 1, 2, 0), (97, 48, 192, 315, 2, 1, 5, 0), (68, 56, 128, 348, 3, 0, 2, 0),
-    (81, 168, 160, 271, 3, 0, 5, 0), (76, 152, 64, 205, 3, 1, 2, 0), (114, 136, 128, 165, 3, 1, 6, 0),
-    (176, 64, 256, 214, 0, 0, 2, 0), (158, 144, 128, 308, 0, 0, 5, 0), (179, 88, 128, 248, 0, 1, 2, 0),
-    (167, 112, 160, 319, 0, 1, 5, 0), (155, 24, 352, 242, 1, 0, 2, 0), (167, 72, 224, 211, 1, 0, 4, 0),
-    (147, 32, 192, 366, 1, 1, 2, 0), (176, 56, 192, 313, 1, 1, 5, 0), (162, 24, 256, 324, 2, 0, 2, 0),
-    (158, 88, 160, 199, 2, 0, 4, 0), (145, 16, 384, 360, 2, 1, 2, 0), (178, 64, 160, 366, 2, 1, 6, 0),
+    (23, 264, 384, 27, 0, 0, 1, 0), (61, 56, 480, 19, 0, 0, 1, 1), (35, 88, 64, 399, 0, 0, 2, 0),
+    (34, 112, 288, 58, 0, 0, 2, 1), (26, 56, 384, 149, 0, 0, 3, 0), (58, 56, 352, 77, 0, 0, 3, 1),
+    (46, 72, 352, 158, 0, 0, 5, 0), (45, 288, 320, 13, 0, 1, 1, 0), (21, 56, 224, 134, 0, 1, 1, 1),
+    (40, 16, 448, 290, 0, 1, 2, 0), (25, 240, 64, 105, 0, 1, 2, 1), (44, 168, 64, 325, 0, 1, 3, 0),
+    (61, 112, 224, 148, 0, 1, 5, 0), (40, 192, 576, 20, 1, 0, 1, 0), (55, 24, 32, 65, 1, 0, 1, 1),
+    (32, 40, 224, 226, 1, 0, 2, 0), (25, 96, 160, 119, 1, 0, 2, 1), (47, 56, 160, 324, 1, 0, 3, 0),
+    (22, 96, 224, 93, 1, 0, 3, 1), (30, 304, 32, 351, 1, 0, 4, 0), (31, 144, 608, 7, 1, 1, 1, 0),
+    (21, 8, 128, 270, 1, 1, 1, 1), (30, 72, 96, 325, 1, 1, 2, 0), (42, 160, 96, 111, 1, 1, 2, 1),
+    (34, 128, 96, 259, 1, 1, 3, 0), (45, 224, 64, 255, 1, 1, 4, 0), (60, 304, 224, 21, 2, 0, 1, 0),
+    (33, 16, 288, 109, 2, 0, 1, 1), (28, 32, 288, 243, 2, 0, 2, 0), (43, 64, 96, 305, 2, 0, 2, 1),
+    (22, 64, 128, 282, 2, 0, 3, 0), (58, 24, 544, 151, 2, 0, 3, 1), (29, 168, 640, 16, 2, 1, 1, 0),
+    (47, 64, 96, 208, 2, 1, 1, 1), (48, 232, 32, 308, 2, 1, 2, 0), (25, 32, 448, 115, 2, 1, 2, 1),
+    (26, 96, 96, 349, 2, 1, 3, 0), (45, 152, 96, 199, 2, 1, 4, 0), (38, 256, 384, 10, 3, 0, 1, 0),
+    (25, 136, 96, 74, 3, 0, 1, 1), (36, 304, 32, 198, 3, 0, 2, 0), (43, 40, 640, 35, 3, 0, 2, 1),
+    (46, 304, 32, 285, 3, 0, 3, 0), (34, 160, 640, 30, 3, 1, 1, 0), (52, 112, 64, 45, 3, 1, 1, 1),
+    (51, 24, 352, 368, 3, 1, 2, 0), (64, 168, 96, 113, 3, 1, 2, 1), (60, 160, 160, 70, 3, 1, 3, 0),
+    (21, 96, 224, 90, 3, 1, 3, 1), (26, 48, 512, 136, 3, 1, 5, 0), (86, 24, 288, 322, 0, 0, 2, 0),
+    (106, 200, 192, 136, 0, 0, 5, 0), (96, 128, 96, 175, 0, 1, 2, 0), (105, 72, 544, 317, 0, 1, 10, 0),
+    (113, 56, 128, 303, 1, 0, 2, 0), (78, 312, 160, 159, 1, 0, 5, 0), (72, 128, 96, 189, 1, 1, 2, 0),
+    (76, 160, 384, 264, 1, 1, 9, 0), (72, 96, 448, 38, 2, 0, 2, 0), (102, 96, 416, 99, 2, 0, 4, 0),
+    (123, 88, 96, 253, 2, 1, 2, 0), (68, 40, 224, 315, 3, 0, 2, 0), (95, 288, 128, 141, 3, 0, 5, 0),
+    (122, 64, 192, 167, 3, 1, 2, 0), (94, 88, 192, 152, 3, 1, 5, 0), (218, 192, 96, 113, 0, 0, 2, 0),
+    (130, 136, 256, 399, 0, 0, 13, 0), (143, 24, 256, 338, 0, 1, 2, 0), (248, 48, 384, 302, 0, 1, 5, 0),
+    (212, 296, 32, 219, 1, 0, 2, 0), (147, 176, 192, 307, 1, 0, 10, 0), (198, 208, 32, 315, 1, 1, 2, 0),
+    (135, 96, 384, 271, 1, 1, 9, 0), (150, 40, 416, 97, 2, 0, 2, 0), (143, 208, 160, 271, 2, 0, 9, 0),
+    (242, 88, 128, 177, 2, 1, 2, 0),
 ]
 
 
@@ -62,10 +61,13 @@ SPREAD = [
 def test_spread_tiles_a_workgroup(bf, nant, nchan, npkt, nbeam, prec, fine, tiles, sums):
     """The table's blocks run spread tiles of as many beam tiles a workgroup as it says;
     a plan whose variant is set runs that."""
-    cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=32, precision=prec, weight_mode=fine)
-    assert bf.lib.bfk_spread_tiles(dims(cfg)) == tiles
-    assert bool(psum_bytes(bf, cfg)) == bool(sums)
-    assert bf.lib.bfk_unset_differs(dims(cfg))
+    for tavg in (8, 16, 32, 64):
+        for order in (0, 1):
+            cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, precision=prec, weight_mode=fine,
+                            input_order=order)
+            assert bf.lib.bfk_spread_tiles(dims(cfg)) == tiles
+            assert bool(psum_bytes(bf, cfg)) == bool(sums)
+            assert bf.lib.bfk_unset_differs(dims(cfg))
 
 
 @pytest.mark.parametrize("nbeam", [65, 96, 128])
@@ -104,3 +106,12 @@ def test_correlator_route_by_both_times(bf, nant, nchan, npkt, order, fused):
     """Shapes timed well on one side of the rule: a block alone and one among others,
     the turned path and the kernel that reads the block."""
     assert bool(bf.lib.bfk_xcorr_use_fused(nant, nchan, npkt, order)) == bool(fused)
+
+
+@pytest.mark.parametrize("nant,nchan,npkt,nbeam,prec,fine,tavg,order", [
+    (217, 168, 128, 245, 0, 0, 8, 1), (193, 40, 256, 325, 1, 1, 32, 1), (28, 120, 896, 64, 1, 1, 32, 0), (26, 224, 224, 57, 1, 1, 64, 0),
+    (131, 344, 32, 789, 0, 1, 64, 1), (197, 240, 96, 631, 0, 1, 8, 1), (60, 384, 1856, 60, 3, 0, 16, 0), (56, 328, 384, 47, 1, 0, 16, 0)])
+def test_blocks_whose_variant_is_faster_run_no_spread_tiles(bf, nant, nchan, npkt, nbeam, prec, fine, tavg, order):
+    """Blocks that took 10 to 50 % longer in spread tiles, alone or among others."""
+    cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, precision=prec, weight_mode=fine, input_order=order)
+    assert bf.lib.bfk_spread_tiles(dims(cfg)) == 0
