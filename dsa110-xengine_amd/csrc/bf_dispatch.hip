@@ -211,14 +211,15 @@ static TileCost packed_cost(const bfk_dims *d) {
       {{{112, 92, 74, 110}, {64, 53, 47, 70}, {56, 32, 29, 43}}, {{110, 88, 70, 100}, {62, 48, 41, 60}, {55, 30, 27, 39}}},
       {{{222, 182, 152, 0}, {135, 117, 104, 0}, {110, 70, 66, 0}}, {{214, 175, 138, 0}, {130, 104, 90, 0}, {115, 68, 62, 0}}}};
   const float(&p)[3][4] = per[d->nkc == 4][d->wmode == 0];
-  const long tiles = (long)((d->nsamp + 2 * TCU - 1) / (2 * TCU)) * d->ngroup;
+  // (an XCD with the most tiles of each set, on its 32 CUs)
+  const long tiles = ((long)((d->nsamp + 2 * TCU - 1) / (2 * TCU)) * d->ngroup + 7) / 8;
   const int live = (d->nbeam + 31) / 32, nset = bfk_packed_sets(live);
   // the sets one after another, each workgroup on the CU that is free first: up to
   // 8 times at which CUs become free (more are taken as the last)
   struct {
     float at;
     long n;
-  } cu[9] = {{0.f, 256}};
+  } cu[9] = {{0.f, 32}};
   int ncu = 1;
   float sum = 0.f, end = 0.f;
   for (int i = 0; i < nset; i++) {
@@ -227,10 +228,10 @@ static TileCost packed_cost(const bfk_dims *d) {
                     (split == 1 && live < 8 * i + 8 ? 0.28f + 0.09f * (float)(live - 8 * i) : 1.f);
     sum += t;
     for (long n = tiles; n > 0;) {
-      if (ncu == 1 && n >= 256) {
-        cu[0].at += t * (float)(n / 256);
+      if (ncu == 1 && n >= 32) {
+        cu[0].at += t * (float)(n / 32);
         end = fmaxf(end, cu[0].at);
-        n %= 256;
+        n %= 32;
         continue;
       }
       const long k = n < cu[0].n ? n : cu[0].n;
@@ -254,12 +255,12 @@ static TileCost packed_cost(const bfk_dims *d) {
       }
     }
   }
-  const float pack = 2.f * d->nsamp * d->nchan * (d->nant + d->nant_pad) / 5.1e6f, share = sum * (float)tiles / 256;
+  const float pack = 2.f * d->nsamp * d->nchan * (d->nant + d->nant_pad) / 5.1e6f, share = sum * (float)tiles / 32;
   const float alone = pack + 5 + end;
   return {alone, fmaxf(alone / 3, share + pack)};
 }
-extern "C" int bfk_use_packed(const bfk_dims *d) {
-  if (d->pinned || !bfk_packed_bytes(d) || !bfk_variant_supported(d, d->variant)) return 0;
+static bool packed_holds(const bfk_dims *d, float less) {
+  if (d->pinned || !bfk_packed_bytes(d) || !bfk_variant_supported(d, d->variant)) return false;
   // (256-beam tiles: fine weights contend for the L2 among others; zeros take the
   // place of missing beam tiles, and five of eight this part of the time)
   static const float contend[4] = {1.05f, 1.1f, 1.25f, 1.27f};
@@ -272,9 +273,24 @@ extern "C" int bfk_use_packed(const bfk_dims *d) {
     v.alone *= part;
     v.among *= part * (group ? 1.f : contend[d->prec]);
   }
+  v.alone *= less;
+  v.among *= less;
   spread_tiles(d, &v);
   const TileCost k = packed_cost(d);
   return k.alone < 1.05f * v.alone && k.among < 1.05f * v.among && k.alone * k.among < 0.95f * v.alone * v.among;
+}
+extern "C" int bfk_use_packed(const bfk_dims *d) {
+  return !d->pinned && bfk_packed_bytes(d) && bfk_variant_supported(d, d->variant);
+}
+// With groups outermost eight antennas' chunks are together and the variant wastes less
+// of its lines: 256-beam tiles take 0.9 of their times above, classic ones 0.78.  Of 380
+// blocks that the times above chose, with the chip's 256 CUs for an XCD's 32, 13 were 5
+// to 56 % slower repacked, alone or among others, all of this order (67 antennas x 120
+// channels x 1536 samples -> 100 beams in FP8 56/37 and 72/42 us, 195 x 304 x 1600 -> 58
+// 206/188 and 249/220; 119 x 112 x 704 -> 706 in FP6, 33 workgroups on an XCD's CUs,
+// 92/80 and 143/76).  None of the 354 left is, and the others were 1.02 and 0.88.
+extern "C" int bfk_pack_block(const bfk_dims *d) {
+  return packed_holds(d, d->order == 0 ? 1.f : d->variant == BFK_VAR_SHARED_256 ? 0.9f : 0.78f);
 }
 
 extern "C" int bfk_variant_supported(const bfk_dims *d, int v) {

@@ -81,8 +81,10 @@ int bfk_beamform(const bfk_dims *d, const uint8_t *d_in, const void *d_wfrag,
                  const float *d_wscale, const float *d_scale, uint8_t *d_out,
                  float *d_power, float *d_bpart, float *d_beam_power, void *d_psum,
                  int *summed, void *d_packed, void *stream);
-/* Blocks that bfk_use_packed names run faster through a repacked copy: d_packed,
- * bfk_packed_bytes, for one launch at a time (NULL: they run the variant). */
+/* Blocks that bfk_pack_block names run faster through a repacked copy: d_packed,
+ * bfk_packed_bytes, for one launch at a time (NULL: they run the variant).
+ * bfk_use_packed: 1 where the repacked path can run the block. */
+int bfk_pack_block(const bfk_dims *d);
 int bfk_use_packed(const bfk_dims *d);
 size_t bfk_packed_bytes(const bfk_dims *d);
 

@@ -123,7 +123,7 @@ void dsaxbf_destroy(dsaxbf_plan *p) {
  * dsaxbf_set_variant, which a caller may call under capture. */
 static void fit_packed(dsaxbf_plan *p) {
   const bfk_dims *d = &p->dims;
-  const int want = !p->batched && bfk_use_packed(d);
+  const int want = !p->batched && bfk_pack_block(d);
   pthread_mutex_lock(&p->turn);
   if (p->d_packed && !want) {
     hipEventSynchronize(p->packed_done);
@@ -381,7 +381,7 @@ static int execute_with(dsaxbf_plan *p, float *bpart, void *psum, int packed, co
        graph's replays would not wait for each other, so under capture the block
        runs without either. */
     if (!d_beam_power || d->stuff != DSAXBF_STUFF_NONE || d->pinned) psum = NULL;
-    packed = packed && p->packed_done && bfk_use_packed(d);
+    packed = packed && p->packed_done && bfk_pack_block(d);
     if ((packed || psum) && (capturing(s) || (psum && s != p->stream && capturing(p->stream)))) {
       packed = 0;
       psum = NULL;
@@ -552,7 +552,7 @@ int dsaxbf_time_variants(dsaxbf_plan *p, const uint8_t *d_in, const float *d_sca
     }
     p->dims.variant = unpinned ? best : v;
     p->dims.pinned = !unpinned;
-    if (unpinned && (!spread_wins || !(bfk_unset_differs(&p->dims) || (p->d_packed && bfk_use_packed(&p->dims))))) break;
+    if (unpinned && (!spread_wins || !(bfk_unset_differs(&p->dims) || (p->d_packed && bfk_pack_block(&p->dims))))) break;
     float t = 0.f;
     he = hipSuccess;
     for (int r = -1; r < reps && rc == DSAXBF_OK && he == hipSuccess; r++) {

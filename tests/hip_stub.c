@@ -125,7 +125,7 @@ size_t bfk_wscale_bytes(const bfk_dims *d) { return 64; }
 size_t bfk_bpart_bytes(const bfk_dims *d) { return 64; }
 size_t bfk_psum_bytes(const bfk_dims *d) { return stub_psum_bytes; }
 size_t bfk_packed_bytes(const bfk_dims *d) { return stub_packed_bytes; }
-int bfk_use_packed(const bfk_dims *d) { return stub_packed_bytes && !d->pinned; }
+int bfk_pack_block(const bfk_dims *d) { return stub_packed_bytes && !d->pinned; }
 int bfk_variant_supported(const bfk_dims *d, int v) { return v != 1; }
 int bfk_spread_tiles(const bfk_dims *d) { return stub_psum_bytes != 0; }
 int bfk_unset_differs(const bfk_dims *d) { return stub_psum_bytes != 0; }

@@ -115,3 +115,53 @@ def test_blocks_whose_variant_is_faster_run_no_spread_tiles(bf, nant, nchan, npk
     """Blocks that took 10 to 50 % longer in spread tiles, alone or among others."""
     cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, precision=prec, weight_mode=fine, input_order=order)
     assert bf.lib.bfk_spread_tiles(dims(cfg)) == 0
+
+
+# Blocks that are repacked, in all bins: antennas, channels, packets, beams, precision, fine weights,
+# input order.  Each precision and order at 65 to 128 and 129 to 256 antennas with one, two, three or
+# four, five to seven, and eight 32-beam tiles in the last set.
+PACKS = [
+    (73, 144, 736, 538, 0, 1, 0), (109, 128, 544, 314, 0, 1, 0), (70, 104, 736, 343, 0, 1, 0),
+    (75, 176, 320, 418, 0, 1, 0), (69, 144, 832, 487, 0, 1, 0), (69, 192, 512, 524, 0, 1, 1),
+    (112, 56, 1184, 307, 0, 1, 1), (102, 152, 288, 590, 0, 1, 1), (66, 112, 608, 159, 0, 1, 1),
+    (106, 88, 608, 529, 1, 0, 0), (84, 88, 768, 294, 1, 1, 0), (78, 168, 416, 382, 1, 1, 0),
+    (86, 104, 768, 204, 1, 0, 0), (105, 160, 288, 511, 1, 1, 0), (74, 120, 768, 525, 1, 0, 1),
+    (95, 88, 992, 317, 1, 0, 1), (76, 112, 800, 582, 1, 1, 1), (96, 152, 512, 398, 1, 1, 1),
+    (65, 120, 896, 484, 1, 0, 1), (115, 56, 416, 520, 2, 1, 0), (67, 48, 832, 292, 2, 0, 0),
+    (75, 64, 544, 592, 2, 0, 0), (73, 176, 512, 216, 2, 1, 0), (69, 96, 608, 486, 2, 0, 0),
+    (76, 152, 672, 528, 2, 0, 1), (106, 176, 320, 575, 2, 1, 1), (66, 104, 672, 356, 2, 0, 1),
+    (70, 112, 992, 464, 2, 1, 1), (97, 152, 256, 507, 2, 1, 1), (65, 144, 736, 261, 3, 1, 0),
+    (100, 96, 736, 573, 3, 0, 0), (95, 144, 256, 583, 3, 1, 0), (90, 64, 1120, 174, 3, 1, 0),
+    (96, 192, 224, 510, 3, 0, 0), (107, 72, 832, 543, 3, 0, 1), (128, 192, 128, 552, 3, 1, 1),
+    (78, 40, 896, 356, 3, 1, 1), (99, 160, 448, 148, 3, 1, 1), (80, 144, 736, 231, 3, 1, 1),
+    (180, 64, 704, 525, 0, 0, 0), (155, 40, 960, 568, 0, 1, 0), (140, 48, 960, 581, 0, 1, 0),
+    (199, 80, 512, 467, 0, 1, 0), (133, 32, 1088, 488, 0, 0, 0), (143, 96, 416, 524, 0, 1, 1),
+    (148, 152, 224, 552, 0, 1, 1), (151, 168, 288, 595, 0, 1, 1), (136, 136, 256, 451, 0, 1, 1),
+    (140, 80, 480, 504, 0, 0, 1), (194, 184, 224, 536, 1, 1, 0), (194, 40, 896, 567, 1, 0, 0),
+    (205, 112, 320, 110, 1, 1, 0), (136, 80, 448, 452, 1, 0, 0), (148, 152, 256, 489, 1, 1, 0),
+    (211, 32, 1216, 540, 1, 1, 1), (166, 56, 896, 545, 1, 1, 1), (133, 56, 1088, 363, 1, 1, 1),
+    (153, 48, 768, 418, 1, 1, 1), (144, 32, 1056, 484, 1, 0, 1), (160, 80, 352, 533, 2, 1, 0),
+    (239, 56, 608, 547, 2, 0, 0), (146, 96, 288, 593, 2, 1, 0), (148, 64, 768, 415, 2, 0, 0),
+    (177, 96, 384, 482, 2, 1, 0), (183, 64, 704, 537, 2, 1, 1), (142, 168, 224, 308, 2, 1, 1),
+    (190, 64, 384, 594, 2, 0, 1), (162, 32, 1120, 391, 2, 0, 1), (130, 40, 864, 490, 2, 1, 1),
+]
+
+
+@pytest.mark.parametrize("nant,nchan,npkt,nbeam,prec,fine,order", PACKS)
+def test_repacked_blocks(bf, nant, nchan, npkt, nbeam, prec, fine, order):
+    """The table's blocks are repacked; a plan whose variant is set runs that."""
+    for tavg in (8, 16, 32, 64):
+        cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=tavg, precision=prec, weight_mode=fine, input_order=order)
+        assert bf.lib.bfk_pack_block(dims(cfg)) and not bf.lib.bfk_pack_block(dims(cfg, 1))
+
+
+@pytest.mark.parametrize("nant,nchan,npkt,nbeam,prec,fine,packs", [
+    (67, 120, 768, 100, 1, 0, 0), (130, 64, 512, 100, 1, 1, 0), (195, 304, 800, 58, 1, 1, 0), (162, 336, 224, 40, 1, 1, 0), (119, 112, 352, 706, 2, 0, 0),
+    (67, 104, 640, 1, 3, 1, 1), (129, 72, 480, 400, 1, 0, 1), (256, 384, 2048, 1024, 1, 1, 1)])
+def test_blocks_with_groups_outermost_are_repacked_where_that_is_faster(bf, nant, nchan, npkt, nbeam, prec, fine, packs):
+    """Blocks timed both ways in the order of dsaX_split -r, whose lines the variants
+    waste less of: those that took up to 56 % longer alone, or 48 % among others,
+    repacked stay as they are."""
+    cfg = bf.config(nant=nant, nchan=nchan, npkt=npkt, nbeam=nbeam, tavg=32, precision=prec, weight_mode=fine, input_order=1)
+    assert bool(bf.lib.bfk_pack_block(dims(cfg))) == bool(packs)
+    assert bf.lib.bfk_use_packed(dims(cfg))
