@@ -511,8 +511,8 @@ extern "C" size_t bfk_xcorr_part_bytes(int nant, int nchan, int nslice) {
 // The turned path or the fused kernel, and the latter's time slices, by modelled
 // times in us: of a block alone on one stream, and among others (three plans in turn,
 // where the launches themselves take 3.75, 6.6 and 9.4 for one, two and three).  Fitted
-// to 325 shapes of 8 to 64 antennas, 8 to 384 channels and 64 to 4096 samples in one to
-// 24 slices each, near the faster ones to 3 % (6 % above 32 antennas with antennas
+// to 469 shapes of 8 to 64 antennas, 8 to 384 channels and 64 to 4096 samples in one to
+// 24 slices each, near the faster ones to 3 % (5 % above 32 antennas with antennas
 // outermost).
 //   fused: a workgroup per 8 channels (4 above 32 antennas) and slice; a base and some
 //     per 8 antennas, then a time per 32 packets.  Up to 32 antennas two share a CU.
@@ -527,15 +527,15 @@ static XcCost xc_fused_cost(int nant, int nchan, int npkt, int order, int slices
   //                               base  /8 ant  /unit  + /antenna  MB    sum  /slice  /MB
   static const float c[2][2][8] = {{{3.31f, .864f, .75f, .012f, .521f, 1.36f, .235f, 0.f},
                                     {2.78f, 1.05f, .849f, .003f, .258f, 1.45f, .24f, .147f}},
-                                   {{5.13f, .437f, .512f, .019f, .258f, 1.92f, .22f, .177f},
-                                    {4.86f, .559f, .952f, .004f, .181f, 1.28f, .255f, .22f}}};
+                                   {{5.83f, .285f, .474f, .02f, .314f, 1.78f, .218f, .174f},
+                                    {4.76f, .57f, .982f, .003f, .181f, 1.44f, .241f, .213f}}};
   const float(&p)[8] = c[nant > 32][order];
   const int sets = nchan / (nant <= 32 ? 8 : 4), wgs = sets * slices, room = nant <= 32 ? 512 : 256;
   const int units = (npkt / XUP + slices - 1) / slices;
   const float mb = 4e-6f * (float)npkt * (float)nant * (float)nchan, vis = vis_mb(nant, nchan) * (float)slices;
   float unit = p[2] + p[3] * (float)nant;
   if (nant <= 32 && wgs > 256) unit *= 1.8f;
-  if (nant > 32 && order == 0 && nchan > 32 && wgs % 64 && wgs % (8 * sets)) unit *= 1.16f;
+  if (nant > 32 && order == 0 && nchan > 32 && wgs % 64 && wgs % (8 * sets)) unit *= 1.12f;
   const float once = p[0] + p[1] * (float)((nant + 7) / 8), chain = unit * (float)units;
   const float sum = slices > 1 ? p[5] + p[6] * (float)slices + p[7] * vis : 0.f;
   const float alone = fmaxf(once + (float)((wgs + room - 1) / room) * chain, mb / 4.3f) + p[4] * vis + sum;
@@ -545,7 +545,7 @@ static XcCost xc_fused_cost(int nant, int nchan, int npkt, int order, int slices
 static XcCost xc_turned_cost(int nant, int nchan, int npkt, int order) {
   //                               base   MB     /unit  /8 ant  vis MB  sum
   static const float c[2][2][6] = {{{6.27f, .354f, .235f, .298f, .619f, 2.26f}, {6.32f, .266f, .25f, .275f, .815f, 2.61f}},
-                                   {{7.91f, .432f, .324f, .102f, .45f, 1.9f}, {7.19f, .406f, .337f, .211f, .346f, 2.52f}}};
+                                   {{7.87f, .453f, .311f, .091f, .41f, 1.98f}, {7.46f, .407f, .333f, .17f, .323f, 2.58f}}};
   const float(&p)[6] = c[nant > 32][order];
   const int slices = bfk_xcorr_default_slices(nchan, npkt), units = (npkt / XUP + slices - 1) / slices;
   const float mb = 4e-6f * (float)npkt * (float)nant * (float)nchan, vis = vis_mb(nant, nchan);
@@ -574,17 +574,17 @@ extern "C" int bfk_xcorr_fused_slices(int nant, int nchan, int npkt, int order) 
 }
 // The slices in which the fused kernel takes the turned path's place, or 0: where its
 // time among others is no longer, that of a block alone, with the 11 us of a launch and
-// its wait beside the kernels, at most 3 to 4 % longer (3 % shorter above 32 antennas
+// its wait beside the kernels, at most 3 to 4 % longer (5 % shorter above 32 antennas
 // with antennas outermost, where the model errs by more), and their product 5 % less.
-// Of 70 shapes that it picks a block alone takes 0.58 to 1.07 times the turned path's
-// time (mean 0.96), one among others 0.50 to 0.93 (0.66).  us alone and among others,
+// In the 207 of the shapes that it picks a block alone takes 0.48 to 1.12 times the
+// turned path's time (mean 0.95, over 1.05 in 7), one among others 0.64.  us alone and among others,
 // turned and fused: 64 antennas x 384 channels x 4096 samples, antennas outermost 127/143
 // and 87/92, groups outermost 130/145 and 57/52; 63 x 48 x 2048, groups outermost 21.4/12.4
 // and 23.0/8.3 (with the launch and wait 32.6 and 34.3); 8 x 328 x 128 7.2/6.8 and 6.0/3.8.
 // Left turned: 60 x 16 x 128 10.0/6.6 and 12.1/4.2, 32 x 32 x 1088 12.8/9.6 and 15.0/6.6, 64
 // x 128 x 1024 with antennas outermost 23.4/15.8 and 27.6/14.1.
 extern "C" int bfk_xcorr_use_fused(int nant, int nchan, int npkt, int order) {
-  static const float longer[2][2] = {{1.03f, 1.03f}, {.97f, 1.04f}};
+  static const float longer[2][2] = {{1.03f, 1.03f}, {.95f, 1.04f}};
   const XcCost t = xc_turned_cost(nant, nchan, npkt, order);
   const int s = xc_slices(nant, nchan, npkt, order, {longer[nant > 32][order] * (t.alone + 11.f) - 11.f, t.among});
   if (!s) return 0;
